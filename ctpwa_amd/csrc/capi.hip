@@ -296,6 +296,7 @@ struct ctpwa_handle {
     int* wg_cls = nullptr;
     long long* wg_rng = nullptr;
     int nacc = 0;
+    int noalloc_nwg = 0;            // workgroups that the no-alloc entry point's limit counts
     PrepArgs prep{};
     FinArgs fin{};
     AuxArgs aux{};
@@ -400,7 +401,7 @@ static void apply_codegen_env(Model_& M) {
     if (const char* e = std::getenv("CTPWA_EVAL_WGS")) {
         int w = std::atoi(e);
         if (w != 64 && w != 128 && w != 256) throw std::runtime_error("CTPWA_EVAL_WGS must be 64, 128 or 256");
-        M.wgs = w;
+        if (M.groups == 1) M.wgs = w;
     }
 }
 
@@ -484,13 +485,45 @@ static void check_q0_masses(const Model_& M) {
     }
 }
 
-// workgroups of the fused kernel: about 1024 (four 128-thread workgroups per CU), at least
-// 256 events each, shared out among the classes by event count, each a whole number of
-// 256-event steps of one class.  scan_phsp == false (phase-space term from the stored
-// Gram): the phase space gets none.
+// Workgroup ranges of the fused kernel: `target` workgroups shared out among the classes by
+// event count times cost, each a whole number of `step`-event iterations of one class.
+// scan_phsp == false (phase-space term from the stored Gram): the phase space gets none.
+// at_most: no more than `target` workgroups in all.
+struct Partition {
+    std::vector<int> cls;
+    std::vector<long long> rng;
+    int g0[3] = {0, 0, 0}, g1[3] = {0, 0, 0};
+};
+static Partition partition(const ctpwa_handle* h, bool scan_phsp, long long target, long long step, double wcost, bool at_most) {
+    Partition R;
+    const double weff = (scan_phsp ? (double)h->n[0] : 0.0) + wcost * (double)(h->n[1] + h->n[2]);
+    for (int c = 0; c < 3; ++c) {
+        R.g0[c] = (int)R.cls.size();
+        const long long n = (c == 0 && !scan_phsp) ? 0 : h->n[c];
+        if (n > 0) {
+            const double share = (double)target * ((c == 0 ? 1.0 : wcost) * (double)n) / weff;
+            const long long want = std::max<long long>(1, at_most ? (long long)share : (long long)std::llround(share));
+            long long chunk = (n + want - 1) / want;
+            chunk = ((chunk + step - 1) / step) * step;
+            const long long nw = (n + chunk - 1) / chunk;
+            for (long long g = 0; g < nw; ++g) {
+                R.cls.push_back(c);
+                R.rng.push_back(h->off[c] + g * chunk);
+                R.rng.push_back(h->off[c] + std::min(n, (g + 1) * chunk));
+            }
+        }
+        R.g1[c] = (int)R.cls.size();
+    }
+    return R;
+}
+
+// The fused kernel's workgroups.  One wave per event (groups == 1): about 1024 (four
+// 128-thread workgroups per CU), at least 256 events each.  Wave groups: one workgroup per
+// CU (its eight waves hold all the registers of a CU's two waves per SIMD) with at least
+// 128 events; 1024 of them, four rounds of workgroups, took 512 us instead of 496 at 1.5M
+// events and 149 amplitudes, and left four times the partial sums to add up.
 static void setup_partition(ctpwa_handle* h, bool scan_phsp) {
     const long long nev = (scan_phsp ? h->n[0] : 0) + h->n[1] + h->n[2];
-    long long target = std::min<long long>(1024, std::max<long long>(1, (nev + 255) / 256));
     // relative cost of a data or background event: the workgroups of each class get events
     // in inverse proportion, so that the classes finish together.  A phase-space event costs
     // about 20 FP64 instructions per amplitude (sums and gradient accumulators), 10 per
@@ -505,30 +538,28 @@ static void setup_partition(ctpwa_handle* h, bool scan_phsp) {
     double wcost = 1.0 + (any_pw ? 140.0 : 40.0) / base;
     if (const char* e = std::getenv("CTPWA_DATA_COST")) wcost = std::atof(e);
     if (!(wcost >= 0.25 && wcost <= 4.0)) throw std::runtime_error("CTPWA_DATA_COST must lie in [0.25, 4]");
-    const double weff = (scan_phsp ? (double)h->n[0] : 0.0) + wcost * (double)(h->n[1] + h->n[2]);
-    std::vector<int> cls;
-    std::vector<long long> rng;
-    for (int c = 0; c < 3; ++c) {
-        h->g0[c] = (int)cls.size();
-        long long n = (c == 0 && !scan_phsp) ? 0 : h->n[c];
-        if (n > 0) {
-            const double wn = (c == 0 ? 1.0 : wcost) * (double)n;
-            long long want = std::max<long long>(1, (long long)std::llround((double)target * wn / weff));
-            long long chunk = (n + want - 1) / want;
-            const long long gw = h->M.wgs;          // whole iterations for every thread
-            chunk = ((chunk + gw - 1) / gw) * gw;
-            long long nw = (n + chunk - 1) / chunk;
-            for (long long g = 0; g < nw; ++g) {
-                cls.push_back(c);
-                rng.push_back(h->off[c] + g * chunk);
-                rng.push_back(h->off[c] + std::min(n, (g + 1) * chunk));
-            }
+    const long long t1 = std::min<long long>(1024, std::max<long long>(1, (nev + 255) / 256));
+    Partition R;
+    if (M.groups > 1) {
+        int ncu = 0;
+        HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
+        const long long t = std::min<long long>(std::max(4, std::min(ncu, 1024)), std::max<long long>(1, (nev + 127) / 128));
+        // (a class too small for a workgroup of its own still gets one)
+        for (long long k = t;; --k) {
+            R = partition(h, scan_phsp, k, M.ev_step(), wcost, true);
+            if ((long long)R.cls.size() <= t || k <= 1) break;
         }
-        h->g1[c] = (int)cls.size();
+        // what ctpwa_nll_grad_noalloc accepts is a matter of the model and the event counts
+        // (include/ctpwa_amd.h), not of this kernel's split
+        h->noalloc_nwg = (int)partition(h, scan_phsp, t1, 128, wcost, false).cls.size();
+    } else {
+        R = partition(h, scan_phsp, t1, M.ev_step(), wcost, false);
+        h->noalloc_nwg = (int)R.cls.size();
     }
-    h->nwg = (int)cls.size();
-    h->wg_cls = h->upload(cls);
-    h->wg_rng = h->upload(rng);
+    for (int c = 0; c < 3; ++c) { h->g0[c] = R.g0[c]; h->g1[c] = R.g1[c]; }
+    h->nwg = (int)R.cls.size();
+    h->wg_cls = h->upload(R.cls);
+    h->wg_rng = h->upload(R.rng);
 }
 
 static bool constant_weights(const double* w, long long n, double* c) {
@@ -1030,7 +1061,8 @@ extern "C" int ctpwa_nll_grad(ctpwa_handle* h, const double* params_dev, double*
 
 extern "C" int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev, double* out_dev, void* stream) {
     if (!h || !params_dev || !out_dev) return fail("ctpwa_nll_grad_noalloc: NULL argument");
-    const size_t need = (size_t)h->nacc * (size_t)std::max(1, h->nwg) + 3 * (size_t)h->nacc;
+    const size_t nacc = 1 + 2 * (size_t)h->M.P.namp + (size_t)h->M.nth_all + h->M.cterms.size();
+    const size_t need = nacc * (size_t)std::max({1, h->nwg, h->noalloc_nwg}) + 3 * nacc;
     if (need > NOALLOC_DOUBLES)
         return fail("ctpwa_nll_grad_noalloc: the evaluation needs " + std::to_string(need) +
                     " doubles of scratch, more than the " + std::to_string(NOALLOC_DOUBLES) + " it holds");

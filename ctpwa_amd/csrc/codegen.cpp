@@ -563,20 +563,13 @@ std::string generate_custom2_kernel(const Model_& M) {
 // L, barrier radius and fixed daughter masses (the rho states of the pi+- pi0 chains of a
 // three-pion model).  The fused kernel loads each distinct one once: fewer scalar
 // registers, which otherwise run out and spill to vector-register lanes that every event
-// iteration reads back.  alias[d][c] = (d' << 8) | c' of the first equal coefficient, or -1.
-static std::vector<std::vector<int>> shared_coefficients(const Model_& M) {
+// iteration reads back.  For the denominators `dens`: alias[d][c] = (d' << 8) | c' of the
+// first equal coefficient among them, or -1.
+static std::vector<std::vector<int>> shared_coefficients(const Model_& M, const std::vector<int>& dens) {
     const Plan& P = M.P;
     std::vector<std::vector<int>> alias(M.dens.size());
     std::map<std::string, int> first;
-    auto src = [](const PRes& R, int k) {
-        std::ostringstream q;
-        q.precision(17);
-        if ((int)R.params.size() <= k) q << "none";
-        else if ((int)R.slots.size() > k && R.slots[k] >= 0) q << "slot" << R.slots[k];
-        else q << "val" << R.params[k];
-        return q.str();
-    };
-    for (size_t d = 0; d < M.dens.size(); ++d) {
+    for (int d : dens) {
         const DenSpec& D = M.dens[d];
         alias[d].assign(D.ncoef, -1);
         if (D.stat || D.ncoef > 255) continue;
@@ -587,35 +580,84 @@ static std::vector<std::vector<int>> shared_coefficients(const Model_& M) {
             std::ostringstream key;
             key.precision(17);
             if (c == 0) {
-                key << "m2|" << (R.params.empty() ? std::string("one") : src(R, 0));
+                key << "m2|" << (R.params.empty() ? std::string("one") : param_src(R, 0));
             } else if (R.model == M_BW) {
-                key << "bw1|" << src(R, 0) << "|" << src(R, 1);
+                key << "bw1|" << param_src(R, 0) << "|" << param_src(R, 1);
             } else if (R.model == M_BWR) {
                 // q0 from fixed daughter masses only (a cascade's daughter mass parameter
                 // makes q0 depend on the block)
                 if (!(n.md1 > 0 || n.d1ref >= 0) || !(n.md2 > 0 || n.d2ref >= 0)) continue;
-                key << "bwr1|" << src(R, 0) << "|" << src(R, 1) << "|" << n.lmin << "|" << (n.has_bf ? n.bf_d : 0.0) << "|"
+                key << "bwr1|" << param_src(R, 0) << "|" << param_src(R, 1) << "|" << n.lmin << "|" << (n.has_bf ? n.bf_d : 0.0) << "|"
                     << (n.md1 > 0 ? n.md1 : 0.0) << "|" << (n.md2 > 0 ? n.md2 : 0.0);
             } else {
                 continue;
             }
             auto it = first.find(key.str());
-            if (it == first.end()) first[key.str()] = ((int)d << 8) | c;
+            if (it == first.end()) first[key.str()] = (d << 8) | c;
             else alias[d][c] = it->second;
         }
     }
     return alias;
 }
 
+// what one wave group evaluates: its blocks and amplitudes, the distinct propagators, SL
+// tensors and invariants they use, the gradient accumulators it holds (columns of the
+// partial sums: amplitudes, propagator terms and Custom terms are each contiguous)
+struct Group {
+    std::vector<int> blocks, amps, dens, us, invs, customs, ths, cts;
+};
+
+static Group make_group(const Model_& M, int g) {
+    const Plan& P = M.P;
+    Group G;
+    std::vector<char> den(M.dens.size(), 0), u(M.us.size(), 0), inv(M.inv.size(), 0);
+    for (size_t b = 0; b < P.blocks.size(); ++b) {
+        if (P.blocks[b].nsl == 0 || M.bgroup[b] != g) continue;
+        G.blocks.push_back((int)b);
+        for (int d : M.block_dens[b]) den[M.den_canon[d]] = 1;
+        for (int c : M.block_customs[b]) G.customs.push_back(c);
+        for (int k = 0; k < P.blocks[b].nsl; ++k) {
+            G.amps.push_back(P.blocks[b].site + k);
+            u[M.amps[P.blocks[b].site + k].u] = 1;
+        }
+    }
+    for (size_t d = 0; d < M.dens.size(); ++d) {
+        if (!den[d]) continue;
+        G.dens.push_back((int)d);
+        for (const Term& t : M.dens[d].re) if (t.inv >= 0) inv[t.inv] = 1;
+        for (const Term& t : M.dens[d].im) if (t.inv >= 0) inv[t.inv] = 1;
+    }
+    for (size_t k = 0; k < u.size(); ++k) if (u[k]) G.us.push_back((int)k);
+    for (size_t k = 0; k < inv.size(); ++k) if (inv[k]) G.invs.push_back((int)k);
+    for (size_t t = 0; t < M.thterms.size(); ++t) if (M.bgroup[M.dens[M.thterms[t].den].block] == g) G.ths.push_back((int)t);
+    for (size_t t = 0; t < M.cterms.size(); ++t) if (M.bgroup[M.customs[M.cterms[t].custom].block] == g) G.cts.push_back((int)t);
+    auto contiguous = [](const std::vector<int>& v) {
+        for (size_t k = 1; k < v.size(); ++k) if (v[k] != v[k - 1] + 1) return false;
+        return true;
+    };
+    if (!contiguous(G.amps) || !contiguous(G.ths) || !contiguous(G.cts))
+        throw std::runtime_error("fused kernel generator: a wave group's accumulators are not contiguous");
+    return G;
+}
+
 std::string generate_eval_kernel(const Model_& M) {
     const Plan& P = M.P;
-    int NU = (int)M.us.size(), NP = P.npol, NA = P.namp;
-    int NTH = (int)M.thterms.size();
-    int NACC = M.nacc();
-    std::vector<int> used(M.inv.size(), 0);
-    for (const DenSpec& Dn : M.dens) {
-        for (const Term& t : Dn.re) if (t.inv >= 0) used[t.inv] = 1;
-        for (const Term& t : Dn.im) if (t.inv >= 0) used[t.inv] = 1;
+    const int NP = P.npol, NACC = M.nacc(), NG = M.groups;
+    std::vector<Group> groups;
+    for (int g = 0; g < NG; ++g) groups.push_back(make_group(M, g));
+    // everything, for the whole-event kernels
+    Group all;
+    for (const Group& g : groups) {
+        all.blocks.insert(all.blocks.end(), g.blocks.begin(), g.blocks.end());
+        all.amps.insert(all.amps.end(), g.amps.begin(), g.amps.end());
+        all.dens.insert(all.dens.end(), g.dens.begin(), g.dens.end());
+        all.us.insert(all.us.end(), g.us.begin(), g.us.end());
+        all.invs.insert(all.invs.end(), g.invs.begin(), g.invs.end());
+        all.customs.insert(all.customs.end(), g.customs.begin(), g.customs.end());
+    }
+    for (std::vector<int>* v : {&all.us, &all.invs}) {
+        std::sort(v->begin(), v->end());
+        v->erase(std::unique(v->begin(), v->end()), v->end());
     }
     std::ostringstream o;
     long long tile_bytes = 16;       // LDS tile buffer of the pipelined form (per buffer)
@@ -639,26 +681,16 @@ std::string generate_eval_kernel(const Model_& M) {
          "  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b);\n"
          "  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));\n"
          "  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);\n}\n";
-    // one workgroup's share of the events: the body is shared by the single-likelihood
-    // kernel and the grouped kernel that evaluates many likelihoods of this model in one
-    // launch, so a likelihood's sums do not depend on how it was launched (UL: how the
-    // coefficients are read, which does not change their values)
-    o << "template <bool UL>\n__device__ __forceinline__ void eval_body(\n"
-         "    const double* __restrict__ tab, const void* __restrict__ slv, const double* __restrict__ inv,\n"
-         "    const float* __restrict__ invf, const double* __restrict__ wts, double* __restrict__ part,\n"
-         "    const int* __restrict__ wg_cls, const long long* __restrict__ wg_rng, long long ld, int nwg,\n"
-         "    double w1, double w2, int pw1, int pw2, const int wg, double (*__restrict__ red)[" << NACC << "],\n"
-         "    unsigned char* __restrict__ lbuf, const double* __restrict__ cfb)\n{\n";
     // storage types: FP64, or FP32 SL tensors / FP32 invariants except s (mixed)
     const char* SLT = M.mixed ? "float2" : "double2";
-    o << "  const " << SLT << "* __restrict__ sl = (const " << SLT << "*)slv;\n";
     std::vector<int> imap = M.imap();
-    auto inv_load = [&](size_t i, const std::string& ev) {
+    auto inv_raw = [&](int i, const std::string& ev) {
         std::ostringstream q;
         if (imap[i] >= 0) q << "inv[" << imap[i] << "LL * ld + " << ev << "]";
-        else q << "(double)invf[" << (-imap[i] - 1) << "LL * ld + " << ev << "]";
+        else q << "invf[" << (-imap[i] - 1) << "LL * ld + " << ev << "]";
         return q.str();
     };
+    auto inv_load = [&](int i, const std::string& ev) { return (imap[i] >= 0 ? "" : "(double)") + inv_raw(i, ev); };
     auto sl_conv = [&](const std::string& x) {
         return M.mixed ? "make_double2((double)" + x + ".x, (double)" + x + ".y)" : x;
     };
@@ -673,24 +705,23 @@ std::string generate_eval_kernel(const Model_& M) {
           << DH_(-g) << " * s" << u << "_" << m << ".y);\n";
         return q.str();
     };
-    o << "  const int cls = wg_cls[wg];\n"
-         "  const long long e0 = wg_rng[2 * wg], e1 = wg_rng[2 * wg + 1];\n"
-         "  const double wc = (cls == 1) ? w1 : w2;\n  const int pw = (cls == 1) ? pw1 : ((cls == 2) ? pw2 : 0);\n"
-         "  const double LOG_FLOOR = log(1e-10);\n";
-    // theta-only coefficients (wave-uniform)
-    o << "  const double* tb = tab;\n";
-    const std::vector<std::vector<int>> coef_alias = shared_coefficients(M);
-    // ul: inside eval_body, whose UL instantiation (the grouped kernels, where the table
-    // pointer comes from a job descriptor in memory rather than a kernel argument) reads
-    // the coefficients through uld() so that they stay in scalar registers
-    auto emit_coefs = [&](const char* ind, bool ul) {
+    // theta-only coefficients (wave-uniform) of a group.  COEF_UL: inside eval_body, whose UL
+    // instantiation (the grouped kernels, where the table pointer comes from a job
+    // descriptor in memory rather than a kernel argument) reads the coefficients through
+    // uld() so that they stay in scalar registers.  COEF_LOOP: read again in every loop
+    // iteration, through a constant-address-space pointer (scalar loads for any uniform
+    // pointer): a wave group's 50 coefficients are more scalar registers than there are
+    enum { COEF_TAB, COEF_UL, COEF_LOOP, COEF_AGAIN };
+    auto emit_coefs = [&](const Group& G, const char* ind, int how) {
+        const std::vector<std::vector<int>> coef_alias = shared_coefficients(M, G.dens);
         auto ld = [&](const std::string& x) {
-            return ul ? "(UL ? uld(tb + (" + x + ")) : tb[" + x + "])" : "tb[" + x + "]";
+            return how >= COEF_LOOP ? "tc[" + x + "]" : how == COEF_UL ? "(UL ? uld(tb + (" + x + ")) : tb[" + x + "])" : "tb[" + x + "]";
         };
-        for (int a = 0; a < NA; ++a)
+        for (int a : G.amps)
             o << ind << "const double c" << a << "r = " << ld("OFFC + " + std::to_string(2 * a)) << ", c" << a
               << "i = " << ld("OFFC + " + std::to_string(2 * a + 1)) << ";\n";
-        for (size_t d = 0; d < M.dens.size(); ++d)
+        if (how == COEF_AGAIN) return;
+        for (int d : G.dens)
             for (int c = 0; c < M.dens[d].ncoef; ++c) {
                 const int src = coef_alias[d][c];
                 if (src >= 0) {
@@ -701,158 +732,9 @@ std::string generate_eval_kernel(const Model_& M) {
                   << ld("OFFR + " + std::to_string((long long)(M.dens[d].coef_base + c)) + "LL * REC") << ";\n";
             }
     };
-    emit_coefs("  ", true);
-    o << "  double av = 0.0;\n";
-    // constant-weight data and background classes: sum_e w ln I_e = w ln prod_e I_e, the
-    // product kept as a mantissa in [0.5, 1) and a binary exponent (two frexp per event
-    // instead of a logarithm; one logarithm per thread after the loop)
-    o << "  double lm = 1.0;\n  int le = 0;\n";
-    for (int a = 0; a < NA; ++a) o << "  double ax" << a << "r = 0.0, ax" << a << "i = 0.0;\n";
-    for (int t = 0; t < NTH; ++t) o << "  double at" << t << " = 0.0;\n";
-    const int NCT = (int)M.cterms.size();
-    for (int t = 0; t < NCT; ++t) o << "  double ct" << t << " = 0.0;\n";
-    const int WGS = M.wgs, NW = M.wgs / 64;
-    if (M.lds_pipe) {
-        // Tiles of WGS events: every per-event input row of the next tile is copied
-        // HBM -> LDS by the DMA path (global_load_lds_dwordx4, no registers held) while
-        // the current tile is computed from LDS.  Row r of a tile occupies
-        // [roff_r, roff_r + WGS * es_r) of the tile buffer; the event layout (class
-        // offsets and leading dimension multiples of 64 events) keeps every 16-byte chunk
-        // aligned and inside its row.
-        struct Row { std::string src; int es; long long off; std::string rd; };
-        std::vector<Row> rows;
-        long long tb = 0;
-        const int esl = M.mixed ? 8 : 16;
-        for (int u = 0; u < NU; ++u)
-            for (int p = 0; p < NP; ++p) {
-                std::string nm = std::to_string(u) + "_" + std::to_string(p);
-                if (p >= NPS) {
-                    rows.push_back(Row{std::string(), 0, tb, mirror(u, p, "    ")});
-                    continue;
-                }
-                std::ostringstream src;
-                src << "(const unsigned char*)sl + " << (long long)u * NPS + p << "LL * ld * " << esl;
-                std::ostringstream rd;
-                rd << "    const " << SLT << " g" << nm << " = ((const " << SLT << "*)(B + " << tb << "))[threadIdx.x];\n"
-                   << "    const double2 s" << nm << " = " << sl_conv("g" + nm) << ";\n";
-                rows.push_back(Row{src.str(), esl, tb, rd.str()});
-                tb += (long long)WGS * esl;
-            }
-        for (size_t i = 0; i < M.inv.size(); ++i) {
-            if (!used[i]) continue;
-            std::ostringstream src, rd;
-            if (imap[i] >= 0) {
-                src << "(const unsigned char*)inv + " << imap[i] << "LL * ld * 8";
-                rd << "    const double x" << i << " = ((const double*)(B + " << tb << "))[threadIdx.x];\n";
-                rows.push_back(Row{src.str(), 8, tb, rd.str()});
-                tb += (long long)WGS * 8;
-            } else {
-                src << "(const unsigned char*)invf + " << (-imap[i] - 1) << "LL * ld * 4";
-                rd << "    const double x" << i << " = (double)((const float*)(B + " << tb << "))[threadIdx.x];\n";
-                rows.push_back(Row{src.str(), 4, tb, rd.str()});
-                tb += (long long)WGS * 4;
-            }
-        }
-        o << "  typedef __attribute__((address_space(3))) void* lds_ptr;\n";
-        o << "  const int ntile = (int)((e1 - e0 + " << WGS - 1 << ") / " << WGS << ");\n";
-        // issue the copies of the tile starting at event ts into buffer dst
-        o << "  auto issue = [&](unsigned char* dst, const long long ts) {\n"
-             "    const int t = threadIdx.x;\n";
-        for (const Row& r : rows) {
-            if (r.es == 0) continue;             // a mirrored polarisation: no copy
-            int nl = WGS * r.es / 16;
-            o << "    if (t < " << nl << " && ts + (long long)(t * " << 16 / r.es << ") < e1)\n"
-              << "      __builtin_amdgcn_global_load_lds((const void*)(" << r.src << " + ts * " << r.es << " + t * 16),\n"
-              << "                                     (lds_ptr)(dst + " << r.off << " + (t & ~63) * 16), 16, 0, 0);\n";
-        }
-        o << "  };\n";
-        o << "  issue(lbuf, e0);\n";
-        o << "  for (int it = 0; it < ntile; ++it) {\n"
-             "    const long long ts = e0 + (long long)it * " << WGS << ";\n"
-             "    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this thread's copies landed\n"
-             "    __syncthreads();                      // every thread's copies landed; previous tile consumed\n"
-             "    if (it + 1 < ntile) issue(lbuf + ((it + 1) & 1) * " << tb << ", ts + " << WGS << ");\n"
-             "    const unsigned char* B = lbuf + (it & 1) * " << tb << ";\n"
-             "    const long long e = ts + threadIdx.x;\n"
-             "    if (e < e1) {\n";
-        for (const Row& r : rows) o << r.rd;
-        tile_bytes = tb;
-    } else {
-        if (M.prefetch_sl) {
-            // the SL values and invariants of the thread's next event (depth 1) or next two
-            // events (depth 2: register sets n and m, rotated each iteration) are loaded
-            // ahead in registers, in their stored types, so their latency overlaps the
-            // current event's arithmetic
-            const int depth = M.prefetch_sl;
-            auto inv_raw = [&](size_t i, const std::string& ev) {
-                std::ostringstream q;
-                if (imap[i] >= 0) q << "inv[" << imap[i] << "LL * ld + " << ev << "]";
-                else q << "invf[" << (-imap[i] - 1) << "LL * ld + " << ev << "]";
-                return q.str();
-            };
-            auto decl_set = [&](const char* pre, const char* ev) {
-                for (int u = 0; u < NU; ++u)
-                    for (int p = 0; p < NPS; ++p)
-                        o << "  " << SLT << " " << pre << u << "_" << p << " = sl[" << (long long)u * NPS + p << "LL * ld + " << ev
-                          << "];\n";
-                for (size_t i = 0; i < M.inv.size(); ++i)
-                    if (used[i]) o << "  " << (imap[i] >= 0 ? "double" : "float") << " " << pre << "x" << i << " = " << inv_raw(i, ev) << ";\n";
-            };
-            // the event weight of a class with per-event weights is loaded ahead too: a load
-            // issued after the next-event loads would make its wait cover them as well
-            o << "  long long e = e0 + threadIdx.x;\n  const long long ep = (e < e1) ? e : e0;\n";
-            decl_set("n", "ep");
-            o << "  double nwt = pw ? wts[ep] : wc;\n";
-            if (depth > 1) {
-                o << "  const long long ep2 = (e + " << WGS << " < e1) ? e + " << WGS << " : e0;\n";
-                decl_set("m", "ep2");
-                o << "  double mwt = pw ? wts[ep2] : wc;\n";
-            }
-            o << "  for (; e < e1; e += " << WGS << ") {\n";
-            for (int u = 0; u < NU; ++u)
-                for (int p = 0; p < NP; ++p) {
-                    std::string nm = std::to_string(u) + "_" + std::to_string(p);
-                    if (p >= NPS) o << mirror(u, p, "    ");
-                    else o << "    const double2 s" << nm << " = " << sl_conv("n" + nm) << ";\n";
-                }
-            for (size_t i = 0; i < M.inv.size(); ++i)
-                if (used[i]) o << "    const double x" << i << " = (double)nx" << i << ";\n";
-            o << "    const double wev = nwt;\n";
-            const long long ahead = (long long)depth * WGS;
-            o << "    { const long long en = (e + " << ahead << " < e1) ? e + " << ahead << " : e;\n";
-            const char* tgt = depth > 1 ? "m" : "n";
-            for (int u = 0; u < NU; ++u)
-                for (int p = 0; p < NPS; ++p) {
-                    if (depth > 1) o << "      n" << u << "_" << p << " = m" << u << "_" << p << ";\n";
-                    o << "      " << tgt << u << "_" << p << " = sl[" << (long long)u * NPS + p << "LL * ld + en];\n";
-                }
-            for (size_t i = 0; i < M.inv.size(); ++i)
-                if (used[i]) {
-                    if (depth > 1) o << "      nx" << i << " = mx" << i << ";\n";
-                    o << "      " << tgt << "x" << i << " = " << inv_raw(i, "en") << ";\n";
-                }
-            if (depth > 1) o << "      nwt = mwt;\n";
-            o << "      if (pw) " << tgt << "wt = wts[en];\n";
-            o << "    }\n";
-        } else {
-            o << "  for (long long e = e0 + threadIdx.x; e < e1; e += " << WGS << ") {\n";
-            for (int u = 0; u < NU; ++u)
-                for (int p = 0; p < NP; ++p) {
-                    std::string nm = std::to_string(u) + "_" + std::to_string(p);
-                    if (p >= NPS) {
-                        o << mirror(u, p, "    ");
-                        continue;
-                    }
-                    o << "    const " << SLT << " g" << nm << " = sl[" << (long long)u * NPS + p << "LL * ld + e];\n";
-                    o << "    const double2 s" << nm << " = " << sl_conv("g" + nm) << ";\n";
-                }
-            for (size_t i = 0; i < M.inv.size(); ++i)
-                if (used[i]) o << "    const double x" << i << " = " << inv_load(i, "e") << ";\n";
-        }
-    }
     // per-event core: denominators, Custom factors, block products (shared by the fused
     // kernel and the amplitude/intensity kernel of models with Custom lineshapes)
-    auto emit_core = [&](std::ostringstream& o) {
+    auto emit_core = [&](const Group& G) {
         auto term_expr = [&](int d, const Term& t) {
             std::string coef = (t.coef < 0) ? D(t.cval) : ("k" + std::to_string(d) + "_" + std::to_string(t.coef));
             if (t.inv < 0) return coef;
@@ -870,12 +752,12 @@ std::string generate_eval_kernel(const Model_& M) {
         // steps per group instead of per propagator; each q_d is within a few ulp of 1/m_d, and
         // a group of 8 squared moduli stays far inside the FP64 range.
         std::vector<int> recip;
-        for (size_t d = 0; d < M.dens.size(); ++d) {
+        for (int d : G.dens) {
             const DenSpec& Dn = M.dens[d];
-            term_sum("dr", (int)d, Dn.re);
-            term_sum("di", (int)d, Dn.im);
+            term_sum("dr", d, Dn.re);
+            term_sum("di", d, Dn.im);
             if (Dn.stat) continue;   // table lineshape: the factor itself
-            recip.push_back((int)d);
+            recip.push_back(d);
             o << "    const double m" << d << " = dr" << d << " * dr" << d << " + di" << d << " * di" << d << ";\n";
         }
         for (size_t g0 = 0; g0 < recip.size(); g0 += 8) {
@@ -930,7 +812,7 @@ std::string generate_eval_kernel(const Model_& M) {
             }
             o << "    const double q" << recip[g0] << " = r" << recip[g0] << ";\n";
         }
-        for (size_t d = 0; d < M.dens.size(); ++d) {
+        for (int d : G.dens) {
             if (M.dens[d].stat) {
                 o << "    const double pr" << d << " = dr" << d << ", pi" << d << " = di" << d << ";\n";
                 continue;
@@ -939,18 +821,17 @@ std::string generate_eval_kernel(const Model_& M) {
         }
         // Custom lineshape factors as written for this parameter point by ctpwa_custom (their
         // derivatives are loaded where the gradient accumulators use them)
-        for (size_t c = 0; c < M.customs.size(); ++c) {
+        for (int c : G.customs) {
             const long long r0 = (long long)c * M.ncf();
             o << "    const double F" << c << "r = cfb[" << r0 << "LL * ld + e], F" << c << "i = cfb[" << r0 + 1
               << "LL * ld + e];\n";
         }
-        for (size_t b = 0; b < P.blocks.size(); ++b) {
+        for (int b : G.blocks) {
             const std::vector<int>& ds = M.block_dens[b];
-            if (P.blocks[b].nsl == 0) continue;
             if (ds.empty()) o << "    double br" << b << " = 1.0, bi" << b << " = 0.0;\n";
-            else o << "    double br" << b << " = pr" << ds[0] << ", bi" << b << " = pi" << ds[0] << ";\n";
+            else o << "    double br" << b << " = pr" << M.den_canon[ds[0]] << ", bi" << b << " = pi" << M.den_canon[ds[0]] << ";\n";
             for (size_t k = 1; k < ds.size(); ++k) {
-                int d = ds[k];
+                const int d = M.den_canon[ds[k]];
                 o << "    { const double tr = br" << b << " * pr" << d << " - bi" << b << " * pi" << d
                   << "; bi" << b << " = br" << b << " * pi" << d << " + bi" << b << " * pr" << d << "; br" << b << " = tr; }\n";
             }
@@ -963,125 +844,117 @@ std::string generate_eval_kernel(const Model_& M) {
             }
         }
     };
-    emit_core(o);
-    for (int u = 0; u < NU; ++u) o << "    double y" << u << "r = 0.0, y" << u << "i = 0.0;\n";
-    for (int a = 0; a < NA; ++a) {
-        int b = M.amps[a].block, u = M.amps[a].u;
-        o << "    y" << u << "r += c" << a << "r * br" << b << "; y" << u << "r -= c" << a << "i * bi" << b << "; y" << u
-          << "i += c" << a << "r * bi" << b << "; y" << u << "i += c" << a << "i * br" << b << ";\n";
-    }
-    // mirror-image polarisations (one stored, sl_u,1 = g_u conj(sl_u,0)): with U_G = sum over
+    // coupling sums y_u = sum_a c_a Psi_b of a group's SL tensors, and its share of S_p.
+    // Mirror-image polarisations (one stored, sl_u,1 = g_u conj(sl_u,0)): with U_G = sum over
     // the SL tensors of sign g_u = G of Re(y_u) sl_u,0 and V_G the same with Im(y_u),
     // S_0 = U + i V and S_1 = conj(U') + i conj(V') (U = U_+ + U_-, U' = U_+ - U_-): 4
     // products per SL tensor for both polarisations instead of 8
     const bool mirror_pair = (NP == 2 && NPS == 1);
-    bool gpos = false, gneg = false;
-    for (int u = 0; u < NU && mirror_pair; ++u) (M.psign[u] > 0 ? gpos : gneg) = true;
-    if (mirror_pair) {
-        for (int G = 0; G < 2; ++G) {
-            if (!(G == 0 ? gpos : gneg)) continue;
-            const char* g = G == 0 ? "P" : "N";
-            o << "    double U" << g << "r = 0.0, U" << g << "i = 0.0, V" << g << "r = 0.0, V" << g << "i = 0.0;\n";
-            for (int u = 0; u < NU; ++u) {
-                if ((M.psign[u] > 0) != (G == 0)) continue;
-                o << "    U" << g << "r += y" << u << "r * s" << u << "_0.x; U" << g << "i += y" << u << "r * s" << u << "_0.y; V" << g
-                  << "r += y" << u << "i * s" << u << "_0.x; V" << g << "i += y" << u << "i * s" << u << "_0.y;\n";
+    auto emit_sums = [&](const Group& G) {
+        for (int u : G.us) o << "    double y" << u << "r = 0.0, y" << u << "i = 0.0;\n";
+        for (int a : G.amps) {
+            int b = M.amps[a].block, u = M.amps[a].u;
+            o << "    y" << u << "r += c" << a << "r * br" << b << "; y" << u << "r -= c" << a << "i * bi" << b << "; y" << u
+              << "i += c" << a << "r * bi" << b << "; y" << u << "i += c" << a << "i * br" << b << ";\n";
+        }
+        if (mirror_pair) {
+            bool gpos = false, gneg = false;
+            for (int u : G.us) (M.psign[u] > 0 ? gpos : gneg) = true;
+            for (int s = 0; s < 2; ++s) {
+                if (!(s == 0 ? gpos : gneg)) continue;
+                const char* g = s == 0 ? "P" : "N";
+                o << "    double U" << g << "r = 0.0, U" << g << "i = 0.0, V" << g << "r = 0.0, V" << g << "i = 0.0;\n";
+                for (int u : G.us) {
+                    if ((M.psign[u] > 0) != (s == 0)) continue;
+                    o << "    U" << g << "r += y" << u << "r * s" << u << "_0.x; U" << g << "i += y" << u << "r * s" << u << "_0.y; V" << g
+                      << "r += y" << u << "i * s" << u << "_0.x; V" << g << "i += y" << u << "i * s" << u << "_0.y;\n";
+                }
             }
-        }
-        if (gpos && gneg)
-            o << "    const double Ur = UPr + UNr, Ui = UPi + UNi, Vr = VPr + VNr, Vi = VPi + VNi;\n"
-                 "    const double Ur_ = UPr - UNr, Ui_ = UPi - UNi, Vr_ = VPr - VNr, Vi_ = VPi - VNi;\n";
-        else if (gpos)
-            o << "    const double Ur = UPr, Ui = UPi, Vr = VPr, Vi = VPi;\n"
-                 "    const double Ur_ = UPr, Ui_ = UPi, Vr_ = VPr, Vi_ = VPi;\n";
-        else
-            o << "    const double Ur = UNr, Ui = UNi, Vr = VNr, Vi = VNi;\n"
-                 "    const double Ur_ = -UNr, Ui_ = -UNi, Vr_ = -VNr, Vi_ = -VNi;\n";
-        o << "    const double S0r = Ur - Vi, S0i = Ui + Vr;\n"
-             "    const double S1r = Ur_ + Vi_, S1i = Vr_ - Ui_;\n";
-    } else {
-        for (int p = 0; p < NP; ++p) {
-            o << "    double S" << p << "r = 0.0, S" << p << "i = 0.0;\n";
-            for (int u = 0; u < NU; ++u)
-                o << "    S" << p << "r += y" << u << "r * s" << u << "_" << p << ".x; S" << p << "r -= y" << u << "i * s" << u << "_" << p
-                  << ".y; S" << p << "i += y" << u << "r * s" << u << "_" << p << ".y; S" << p << "i += y" << u << "i * s" << u << "_" << p << ".x;\n";
-        }
-    }
-    o << "    double I = 0.0;\n";
-    for (int p = 0; p < NP; ++p) o << "    I += S" << p << "r * S" << p << "r; I += S" << p << "i * S" << p << "i;\n";
-    for (int p = 0; p < NP; ++p) o << "    double w" << p << "r, w" << p << "i;\n";
-    o << "    if (cls == 0) {\n      av += I;\n";
-    for (int p = 0; p < NP; ++p) o << "      w" << p << "r = S" << p << "r; w" << p << "i = S" << p << "i;\n";
-    o << "    } else {\n      const double we = " << (M.prefetch_sl && !M.lds_pipe ? "wev" : "pw ? wts[e] : wc") << ";\n"
-         "      if (pw) {\n        av += (I == 0.0 ? LOG_FLOOR : log(I)) * we;\n      } else {\n"
-         "        const double Il = (I == 0.0) ? 1e-10 : I;   // ln(1e-10): the I = 0 rule\n"
-         "        lm *= __builtin_amdgcn_frexp_mant(Il); le += __builtin_amdgcn_frexp_exp(Il);\n"
-         "        const int ex = __builtin_amdgcn_frexp_exp(lm); lm = __builtin_amdgcn_frexp_mant(lm); le += ex;\n"
-         "      }\n"
-         "      if (I == 0.0) {\n";
-    for (int p = 0; p < NP; ++p) o << "        w" << p << "r = 0.0; w" << p << "i = 0.0;\n";
-    o << "      } else {\n        const double f = we * frcp(I);\n";
-    for (int p = 0; p < NP; ++p)
-        o << "        w" << p << "r = fmin(fmax(S" << p << "r * f, -1e10), 1e10); w" << p << "i = fmin(fmax(S" << p
-          << "i * f, -1e10), 1e10);\n";
-    o << "      }\n    }\n";
-    if (mirror_pair) {
-        // T_u = conj(sl_u,0) w_0 + g_u sl_u,0 w_1 from the sums and differences of w_0, w_1:
-        // g = +1: (a sr + b di) + i (a si - b dr); g = -1: (a dr + b si) + i (a di - b sr)
-        o << "    const double wsr = w0r + w1r, wsi = w0i + w1i, wdr = w0r - w1r, wdi = w0i - w1i;\n";
-        for (int u = 0; u < NU; ++u) {
-            const bool pos = M.psign[u] > 0;
-            o << "    const double t" << u << "r = s" << u << "_0.x * " << (pos ? "wsr" : "wdr") << " + s" << u << "_0.y * "
-              << (pos ? "wdi" : "wsi") << ", t" << u << "i = s" << u << "_0.x * " << (pos ? "wsi" : "wdi") << " - s" << u
-              << "_0.y * " << (pos ? "wdr" : "wsr") << ";\n";
-        }
-    } else {
-        for (int u = 0; u < NU; ++u) {
-            o << "    double t" << u << "r = 0.0, t" << u << "i = 0.0;\n";
-            for (int p = 0; p < NP; ++p)
-                o << "    t" << u << "r += s" << u << "_" << p << ".x * w" << p << "r; t" << u << "r += s" << u << "_" << p << ".y * w" << p
-                  << "i; t" << u << "i += s" << u << "_" << p << ".x * w" << p << "i; t" << u << "i -= s" << u << "_" << p << ".y * w" << p << "r;\n";
-        }
-    }
-    // per block: the coupling sums P_a = conj(Psi_b) T_u (X_a += P_a), then the theta
-    // terms R_d = Z_b Psi_b Psi_d with Z_b Psi_b = sum_{a in b} c_a conj(P_a)
-    std::vector<std::vector<int>> den_terms(M.dens.size());
-    for (int t = 0; t < NTH; ++t) den_terms[M.thterms[t].den].push_back(t);
-    std::vector<std::vector<int>> custom_terms(M.customs.size());
-    for (int t = 0; t < NCT; ++t) custom_terms[M.cterms[t].custom].push_back(t);
-    for (size_t b = 0; b < P.blocks.size(); ++b) {
-        const PBlock& B = P.blocks[b];
-        for (int c = 0; c < B.nsl; ++c) {
-            int a = B.site + c, u = M.amps[a].u;
-            o << "    const double P" << a << "r = br" << b << " * t" << u << "r + bi" << b << " * t" << u << "i, P" << a
-              << "i = br" << b << " * t" << u << "i - bi" << b << " * t" << u << "r;\n";
-            o << "    ax" << a << "r += P" << a << "r; ax" << a << "i += P" << a << "i;\n";
-        }
-        bool any = false;
-        for (int d : M.block_dens[b]) if (!den_terms[d].empty()) any = true;
-        for (int c : M.block_customs[b]) if (!custom_terms[c].empty()) any = true;
-        if (B.nsl == 0 || !any) continue;
-        o << "    {\n";
-        const bool with_custom = !M.block_customs[b].empty();
-        if (with_custom) {
-            // the derivatives through Custom factors need Z_b itself
-            o << "      double zr = 0.0, zi = 0.0;\n";
-            for (int c = 0; c < B.nsl; ++c) {
-                int a = B.site + c, u = M.amps[a].u;
-                o << "      zr += c" << a << "r * t" << u << "r; zr += c" << a << "i * t" << u << "i; zi += c" << a << "i * t" << u
-                  << "r; zi -= c" << a << "r * t" << u << "i;\n";
-            }
-            o << "      const double zbr = zr * br" << b << " - zi * bi" << b << ", zbi = zr * bi" << b << " + zi * br" << b << ";\n";
+            if (gpos && gneg)
+                o << "    const double Ur = UPr + UNr, Ui = UPi + UNi, Vr = VPr + VNr, Vi = VPi + VNi;\n"
+                     "    const double Ur_ = UPr - UNr, Ui_ = UPi - UNi, Vr_ = VPr - VNr, Vi_ = VPi - VNi;\n";
+            else if (gpos)
+                o << "    const double Ur = UPr, Ui = UPi, Vr = VPr, Vi = VPi;\n"
+                     "    const double Ur_ = UPr, Ui_ = UPi, Vr_ = VPr, Vi_ = VPi;\n";
+            else
+                o << "    const double Ur = UNr, Ui = UNi, Vr = VNr, Vi = VNi;\n"
+                     "    const double Ur_ = -UNr, Ui_ = -UNi, Vr_ = -VNr, Vi_ = -VNi;\n";
+            o << "    double S0r = Ur - Vi, S0i = Ui + Vr;\n"
+                 "    double S1r = Ur_ + Vi_, S1i = Vr_ - Ui_;\n";
         } else {
-            o << "      double zbr = 0.0, zbi = 0.0;\n";
-            for (int c = 0; c < B.nsl; ++c) {
-                int a = B.site + c;
-                o << "      zbr += c" << a << "r * P" << a << "r; zbr += c" << a << "i * P" << a << "i; zbi += c" << a
-                  << "i * P" << a << "r; zbi -= c" << a << "r * P" << a << "i;\n";
+            for (int p = 0; p < NP; ++p) {
+                o << "    double S" << p << "r = 0.0, S" << p << "i = 0.0;\n";
+                for (int u : G.us)
+                    o << "    S" << p << "r += y" << u << "r * s" << u << "_" << p << ".x; S" << p << "r -= y" << u << "i * s" << u << "_" << p
+                      << ".y; S" << p << "i += y" << u << "r * s" << u << "_" << p << ".y; S" << p << "i += y" << u << "i * s" << u << "_" << p << ".x;\n";
             }
         }
-        for (int d : M.block_dens[b]) {
-            if (den_terms[d].empty()) continue;
+    };
+    // intensity, the class branch and the adjoint weights w_p; `value`: this wave also
+    // accumulates the likelihood's value; `live`: lanes past the range's end (wave groups
+    // run whole iterations) contribute nothing
+    auto emit_weights = [&](const std::string& weight, bool value, bool live) {
+        o << "    double I = 0.0;\n";
+        for (int p = 0; p < NP; ++p) o << "    I += S" << p << "r * S" << p << "r; I += S" << p << "i * S" << p << "i;\n";
+        if (live && value) o << "    if (!live) I = (cls == 0) ? 0.0 : 1.0;\n";
+        for (int p = 0; p < NP; ++p) o << "    double w" << p << "r, w" << p << "i;\n";
+        o << "    if (cls == 0) {\n";
+        if (value) o << "      av += I;\n";
+        for (int p = 0; p < NP; ++p) o << "      w" << p << "r = S" << p << "r; w" << p << "i = S" << p << "i;\n";
+        o << "    } else {\n      const double we = " << weight << ";\n";
+        if (value)
+            o << "      if (pw) {\n        av += (I == 0.0 ? LOG_FLOOR : log(I)) * we;\n      } else {\n"
+                 "        const double Il = (I == 0.0) ? 1e-10 : I;   // ln(1e-10): the I = 0 rule\n"
+                 "        lm *= __builtin_amdgcn_frexp_mant(Il); le += __builtin_amdgcn_frexp_exp(Il);\n"
+                 "        const int ex = __builtin_amdgcn_frexp_exp(lm); lm = __builtin_amdgcn_frexp_mant(lm); le += ex;\n"
+                 "      }\n";
+        o << "      if (I == 0.0) {\n";
+        for (int p = 0; p < NP; ++p) o << "        w" << p << "r = 0.0; w" << p << "i = 0.0;\n";
+        o << "      } else {\n        const double f = we * frcp(I);\n";
+        for (int p = 0; p < NP; ++p)
+            o << "        w" << p << "r = fmin(fmax(S" << p << "r * f, -1e10), 1e10); w" << p << "i = fmin(fmax(S" << p
+              << "i * f, -1e10), 1e10);\n";
+        o << "      }\n    }\n";
+        if (live) {
+            o << "    if (!live) {";
+            for (int p = 0; p < NP; ++p) o << " w" << p << "r = 0.0; w" << p << "i = 0.0;";
+            o << " }\n";
+        }
+    };
+    // the adjoint T_u of a group's SL tensors and its gradient accumulators
+    auto emit_adjoint = [&](const Group& G) {
+        if (mirror_pair) {
+            // T_u = conj(sl_u,0) w_0 + g_u sl_u,0 w_1 from the sums and differences of w_0, w_1:
+            // g = +1: (a sr + b di) + i (a si - b dr); g = -1: (a dr + b si) + i (a di - b sr)
+            o << "    const double wsr = w0r + w1r, wsi = w0i + w1i, wdr = w0r - w1r, wdi = w0i - w1i;\n";
+            for (int u : G.us) {
+                const bool pos = M.psign[u] > 0;
+                o << "    const double t" << u << "r = s" << u << "_0.x * " << (pos ? "wsr" : "wdr") << " + s" << u << "_0.y * "
+                  << (pos ? "wdi" : "wsi") << ", t" << u << "i = s" << u << "_0.x * " << (pos ? "wsi" : "wdi") << " - s" << u
+                  << "_0.y * " << (pos ? "wdr" : "wsr") << ";\n";
+            }
+        } else {
+            for (int u : G.us) {
+                o << "    double t" << u << "r = 0.0, t" << u << "i = 0.0;\n";
+                for (int p = 0; p < NP; ++p)
+                    o << "    t" << u << "r += s" << u << "_" << p << ".x * w" << p << "r; t" << u << "r += s" << u << "_" << p << ".y * w" << p
+                      << "i; t" << u << "i += s" << u << "_" << p << ".x * w" << p << "i; t" << u << "i -= s" << u << "_" << p << ".y * w" << p << "r;\n";
+            }
+        }
+        // per block: the coupling sums P_a = conj(Psi_b) T_u (X_a += P_a), then the theta
+        // terms R_d = Z_b Psi_b Psi_d with Z_b Psi_b = sum_{a in b} c_a conj(P_a).  A
+        // propagator of several blocks takes the sum of their Z_b Psi_b once, after its
+        // last block.
+        std::vector<std::vector<int>> den_terms(M.dens.size());
+        for (int t : G.ths) den_terms[M.thterms[t].den].push_back(t);
+        std::vector<std::vector<int>> custom_terms(M.customs.size());
+        for (int t : G.cts) custom_terms[M.cterms[t].custom].push_back(t);
+        std::vector<int> uses(M.dens.size(), 0), seen(M.dens.size(), 0);
+        for (int b : G.blocks)
+            for (int d : M.block_dens[b]) uses[M.den_canon[d]]++;
+        for (int d : G.dens)
+            if (!den_terms[d].empty() && uses[d] > 1) o << "    double zs" << d << "r = 0.0, zs" << d << "i = 0.0;\n";
+        auto den_accum = [&](int d, const std::string& zr, const std::string& zi) {
             // a component with one term and no invariant is accumulated by two FMAs
             int nre = 0, nim = 0;
             bool bare_re = false, bare_im = false;
@@ -1092,14 +965,14 @@ std::string generate_eval_kernel(const Model_& M) {
             }
             const bool fre = nre == 1 && bare_re, fim = nim == 1 && bare_im;
             o << "      {\n";
-            if (nre && !fre) o << "        const double rr = zbr * pr" << d << " - zbi * pi" << d << ";\n";
-            if (nim && !fim) o << "        const double ri = zbr * pi" << d << " + zbi * pr" << d << ";\n";
+            if (nre && !fre) o << "        const double rr = " << zr << " * pr" << d << " - " << zi << " * pi" << d << ";\n";
+            if (nim && !fim) o << "        const double ri = " << zr << " * pi" << d << " + " << zi << " * pr" << d << ";\n";
             for (int t : den_terms[d]) {
                 const ThTerm& T = M.thterms[t];
                 if (!T.im && fre) {
-                    o << "        at" << t << " += zbr * pr" << d << "; at" << t << " -= zbi * pi" << d << ";\n";
+                    o << "        at" << t << " += " << zr << " * pr" << d << "; at" << t << " -= " << zi << " * pi" << d << ";\n";
                 } else if (T.im && fim) {
-                    o << "        at" << t << " += zbr * pi" << d << "; at" << t << " += zbi * pr" << d << ";\n";
+                    o << "        at" << t << " += " << zr << " * pi" << d << "; at" << t << " += " << zi << " * pr" << d << ";\n";
                 } else {
                     const char* comp = T.im ? "ri" : "rr";
                     if (T.inv < 0) o << "        at" << t << " += " << comp << ";\n";
@@ -1107,72 +980,383 @@ std::string generate_eval_kernel(const Model_& M) {
                 }
             }
             o << "      }\n";
-        }
-        // Custom factors: d Psi_b / d theta_j = (product of the block's other factors) F'_c,j
-        for (int c : M.block_customs[b]) {
-            if (custom_terms[c].empty()) continue;
-            o << "      {\n        double or_ = pdr" << b << ", oi_ = pdi" << b << ";\n";
-            for (int c2 : M.block_customs[b]) {
-                if (c2 == c) continue;
-                o << "        { const double tr = or_ * F" << c2 << "r - oi_ * F" << c2 << "i; oi_ = or_ * F" << c2
-                  << "i + oi_ * F" << c2 << "r; or_ = tr; }\n";
+        };
+        for (int b : G.blocks) {
+            const PBlock& B = P.blocks[b];
+            for (int c = 0; c < B.nsl; ++c) {
+                int a = B.site + c, u = M.amps[a].u;
+                o << "    const double P" << a << "r = br" << b << " * t" << u << "r + bi" << b << " * t" << u << "i, P" << a
+                  << "i = br" << b << " * t" << u << "i - bi" << b << " * t" << u << "r;\n";
+                o << "    ax" << a << "r += P" << a << "r; ax" << a << "i += P" << a << "i;\n";
             }
-            o << "        const double wr = zr * or_ - zi * oi_, wi = zr * oi_ + zi * or_;\n";
-            for (int t : custom_terms[c]) {
-                int li = M.cterms[t].local;
-                const long long rr = (long long)c * M.ncf() + 2 + li, ri = rr + M.ncv();
-                o << "        ct" << t << " += wr * cfb[" << rr << "LL * ld + e] - wi * cfb[" << ri << "LL * ld + e];\n";
+            bool any = false;
+            for (int d : M.block_dens[b]) if (!den_terms[M.den_canon[d]].empty()) any = true;
+            for (int c : M.block_customs[b]) if (!custom_terms[c].empty()) any = true;
+            if (!any) continue;
+            o << "    {\n";
+            const bool with_custom = !M.block_customs[b].empty();
+            if (with_custom) {
+                // the derivatives through Custom factors need Z_b itself
+                o << "      double zr = 0.0, zi = 0.0;\n";
+                for (int c = 0; c < B.nsl; ++c) {
+                    int a = B.site + c, u = M.amps[a].u;
+                    o << "      zr += c" << a << "r * t" << u << "r; zr += c" << a << "i * t" << u << "i; zi += c" << a << "i * t" << u
+                      << "r; zi -= c" << a << "r * t" << u << "i;\n";
+                }
+                o << "      const double zbr = zr * br" << b << " - zi * bi" << b << ", zbi = zr * bi" << b << " + zi * br" << b << ";\n";
+            } else {
+                o << "      double zbr = 0.0, zbi = 0.0;\n";
+                for (int c = 0; c < B.nsl; ++c) {
+                    int a = B.site + c;
+                    o << "      zbr += c" << a << "r * P" << a << "r; zbr += c" << a << "i * P" << a << "i; zbi += c" << a
+                      << "i * P" << a << "r; zbi -= c" << a << "r * P" << a << "i;\n";
+                }
             }
-            o << "      }\n";
+            for (int dd : M.block_dens[b]) {
+                const int d = M.den_canon[dd];
+                if (den_terms[d].empty()) continue;
+                if (uses[d] == 1) {
+                    den_accum(d, "zbr", "zbi");
+                    continue;
+                }
+                o << "      zs" << d << "r += zbr; zs" << d << "i += zbi;\n";
+                if (++seen[d] == uses[d]) den_accum(d, "zs" + std::to_string(d) + "r", "zs" + std::to_string(d) + "i");
+            }
+            // Custom factors: d Psi_b / d theta_j = (product of the block's other factors) F'_c,j
+            for (int c : M.block_customs[b]) {
+                if (custom_terms[c].empty()) continue;
+                o << "      {\n        double or_ = pdr" << b << ", oi_ = pdi" << b << ";\n";
+                for (int c2 : M.block_customs[b]) {
+                    if (c2 == c) continue;
+                    o << "        { const double tr = or_ * F" << c2 << "r - oi_ * F" << c2 << "i; oi_ = or_ * F" << c2
+                      << "i + oi_ * F" << c2 << "r; or_ = tr; }\n";
+                }
+                o << "        const double wr = zr * or_ - zi * oi_, wi = zr * oi_ + zi * or_;\n";
+                for (int t : custom_terms[c]) {
+                    int li = M.cterms[t].local;
+                    const long long rr = (long long)c * M.ncf() + 2 + li, ri = rr + M.ncv();
+                    o << "        ct" << t << " += wr * cfb[" << rr << "LL * ld + e] - wi * cfb[" << ri << "LL * ld + e];\n";
+                }
+                o << "      }\n";
+            }
+            o << "    }\n";
         }
-        o << "    }\n";
-    }
-    o << (M.lds_pipe ? "    }\n  }\n" : "  }\n");
+    };
+    auto emit_accs = [&](const Group& G) {
+        for (int a : G.amps) o << "  double ax" << a << "r = 0.0, ax" << a << "i = 0.0;\n";
+        for (int t : G.ths) o << "  double at" << t << " = 0.0;\n";
+        for (int t : G.cts) o << "  double ct" << t << " = 0.0;\n";
+    };
+    // the SL values and invariants of the thread's next event (register set n; depth 2: also
+    // the one after it, set m) loaded ahead in registers, in their stored types, so their
+    // latency overlaps the current event's arithmetic.  The event weight of a class with
+    // per-event weights is loaded ahead too: a load issued after the next-event loads would
+    // make its wait cover them as well.
+    // Wave groups load ahead the invariants only: the SL values are first used after the
+    // propagators and the coupling sums (some 200 FP64 instructions), and with both ahead
+    // the eight groups of the 149-amplitude model spill (282 registers; 73 without, outside
+    // the loops).
+    const bool pf_sl = NG == 1;
+    auto decl_set = [&](const Group& G, const char* pre, const char* ev) {
+        if (pf_sl) for (int u : G.us)
+            for (int p = 0; p < NPS; ++p)
+                o << "  " << SLT << " " << pre << u << "_" << p << " = sl[" << (long long)u * NPS + p << "LL * ld + " << ev << "];\n";
+        for (int i : G.invs)
+            o << "  " << (imap[i] >= 0 ? "double" : "float") << " " << pre << "x" << i << " = " << inv_raw(i, ev) << ";\n";
+    };
+    auto use_set = [&](const Group& G) {
+        for (int u : G.us)
+            for (int p = 0; p < NP; ++p) {
+                std::string nm = std::to_string(u) + "_" + std::to_string(p);
+                if (p >= NPS) o << mirror(u, p, "    ");
+                else {
+                    if (!pf_sl)
+                        o << "    const " << SLT << " n" << nm << " = sl[" << (long long)u * NPS + p << "LL * ld + e];\n";
+                    o << "    const double2 s" << nm << " = " << sl_conv("n" + nm) << ";\n";
+                }
+            }
+        for (int i : G.invs) o << "    const double x" << i << " = (double)nx" << i << ";\n";
+        o << "    const double wev = nwt;\n";
+    };
+    auto next_set = [&](const Group& G, int depth) {
+        const char* tgt = depth > 1 ? "m" : "n";
+        if (pf_sl) for (int u : G.us)
+            for (int p = 0; p < NPS; ++p) {
+                if (depth > 1) o << "      n" << u << "_" << p << " = m" << u << "_" << p << ";\n";
+                o << "      " << tgt << u << "_" << p << " = sl[" << (long long)u * NPS + p << "LL * ld + en];\n";
+            }
+        for (int i : G.invs) {
+            if (depth > 1) o << "      nx" << i << " = mx" << i << ";\n";
+            o << "      " << tgt << "x" << i << " = " << inv_raw(i, "en") << ";\n";
+        }
+        if (depth > 1) o << "      nwt = mwt;\n";
+        o << "      if (pw) " << tgt << "wt = wts[en];\n";
+    };
     // ln prod I = ln(mantissa) + exponent ln 2 (ln 2 split into a high part with trailing
     // zero bits and the remainder, so that the exponent's product stays exact)
-    o << "  if (cls != 0 && !pw)\n"
-         "    av += wc * __builtin_fma((double)le, 1.90821492927058770002e-10,\n"
-         "                              __builtin_fma((double)le, 6.93147180369123816490e-01, log(lm)));\n";
+    auto emit_log = [&]() {
+        o << "  if (cls != 0 && !pw)\n"
+             "    av += wc * __builtin_fma((double)le, 1.90821492927058770002e-10,\n"
+             "                              __builtin_fma((double)le, 6.93147180369123816490e-01, log(lm)));\n";
+    };
     // reduction over the wave: 16 accumulators at a time are written to the wave's LDS slab
     // (rows padded to 17 doubles), lane 4k + q adds column k over lanes 16q .. 16q + 15 in
     // lane order, and two exchanges join the quarters (a fixed order); per 16 accumulators
-    // that is 16 LDS writes, 16 reads and 2 exchanges instead of 6 exchanges each
-    std::vector<std::string> accs;
-    accs.push_back("av");
-    for (int a = 0; a < NA; ++a) { accs.push_back("ax" + std::to_string(a) + "r"); accs.push_back("ax" + std::to_string(a) + "i"); }
-    for (int t = 0; t < NTH; ++t) accs.push_back("at" + std::to_string(t));
-    for (int t = 0; t < NCT; ++t) accs.push_back("ct" + std::to_string(t));
-    if ((int)accs.size() != NACC) throw std::runtime_error("fused kernel generator: accumulator count mismatch");
-    if (M.lds_pipe) o << "  __syncthreads();                 // every wave is done with the tile buffers\n";
-    o << "  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;\n"
-         "  {\n    double (*tl)[17] = (double (*)[17])(lbuf + wave * " << 64 * 17 * 8 << ");\n"
-         "    const int k4 = lane >> 2, q4 = lane & 3;\n";
-    for (int c0 = 0; c0 < NACC; c0 += 16) {
-        const int m = std::min(16, NACC - c0);
-        for (int k = 0; k < m; ++k) o << "    tl[lane][" << k << "] = " << accs[c0 + k] << ";\n";
-        o << "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\"); __builtin_amdgcn_wave_barrier();\n"
-             "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n"
-             "    { double s = tl[16 * q4][k4];\n"
-             "      for (int t = 1; t < 16; ++t) s += tl[16 * q4 + t][k4];\n"
-             "      s += __shfl_xor(s, 1, 64); s += __shfl_xor(s, 2, 64);\n"
-             "      if (q4 == 0 && k4 < " << m << ") red[wave][" << c0 << " + k4] = s; }\n"
-             "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\"); __builtin_amdgcn_wave_barrier();\n"
-             "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n";
+    // that is 16 LDS writes, 16 reads and 2 exchanges instead of 6 exchanges each.  The sum
+    // of accumulator c0 + k4 goes to `dst`.
+    auto emit_reduce = [&](const std::vector<std::string>& accs, const std::function<std::string(int)>& dst) {
+        o << "  {\n    double (*tl)[17] = (double (*)[17])(lbuf + wave * " << 64 * 17 * 8 << ");\n"
+             "    const int k4 = lane >> 2, q4 = lane & 3;\n";
+        for (int c0 = 0; c0 < (int)accs.size(); c0 += 16) {
+            const int m = std::min(16, (int)accs.size() - c0);
+            for (int k = 0; k < m; ++k) o << "    tl[lane][" << k << "] = " << accs[c0 + k] << ";\n";
+            o << "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\"); __builtin_amdgcn_wave_barrier();\n"
+                 "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n"
+                 "    { double s = tl[16 * q4][k4];\n"
+                 "      for (int t = 1; t < 16; ++t) s += tl[16 * q4 + t][k4];\n"
+                 "      s += __shfl_xor(s, 1, 64); s += __shfl_xor(s, 2, 64);\n"
+                 "      if (q4 == 0 && k4 < " << m << ") " << dst(c0) << " = s; }\n"
+                 "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\"); __builtin_amdgcn_wave_barrier();\n"
+                 "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n";
+        }
+        o << "  }\n";
+    };
+    auto acc_names = [&](const Group& G) {
+        std::vector<std::string> v;
+        for (int a : G.amps) { v.push_back("ax" + std::to_string(a) + "r"); v.push_back("ax" + std::to_string(a) + "i"); }
+        for (int t : G.ths) v.push_back("at" + std::to_string(t));
+        for (int t : G.cts) v.push_back("ct" + std::to_string(t));
+        return v;
+    };
+    const std::string PARAMS =
+        "    const double* __restrict__ tab, const void* __restrict__ slv, const double* __restrict__ inv,\n"
+        "    const float* __restrict__ invf, const double* __restrict__ wts, double* __restrict__ part,\n"
+        "    const int* __restrict__ wg_cls, const long long* __restrict__ wg_rng, long long ld, int nwg,\n"
+        "    double w1, double w2, int pw1, int pw2, const int wg, double (*__restrict__ red)[" + std::to_string(NG > 1 ? 1 : NACC) + "],\n"
+        "    unsigned char* __restrict__ lbuf, const double* __restrict__ cfb)\n{\n";
+    const int WGS = M.wgs, NW = M.wgs / 64;
+    auto emit_prologue = [&]() {
+        o << "  const " << SLT << "* __restrict__ sl = (const " << SLT << "*)slv;\n";
+        o << "  const int cls = wg_cls[wg];\n"
+             "  const long long e0 = wg_rng[2 * wg], e1 = wg_rng[2 * wg + 1];\n"
+             "  const double wc = (cls == 1) ? w1 : w2;\n  const int pw = (cls == 1) ? pw1 : ((cls == 2) ? pw2 : 0);\n"
+             "  const double LOG_FLOOR = log(1e-10);\n"
+             "  const double* tb = tab;\n";
+    };
+    // constant-weight data and background classes: sum_e w ln I_e = w ln prod_e I_e, the
+    // product kept as a mantissa in [0.5, 1) and a binary exponent (two frexp per event
+    // instead of a logarithm; one logarithm per thread after the loop)
+    const char* VALUE_ACCS = "  double av = 0.0;\n  double lm = 1.0;\n  int le = 0;\n";
+    // one workgroup's share of the events: the body is shared by the single-likelihood
+    // kernel and the grouped kernel that evaluates many likelihoods of this model in one
+    // launch, so a likelihood's sums do not depend on how it was launched (UL: how the
+    // coefficients are read, which does not change their values)
+    if (NG == 1) {
+        const Group& G = groups[0];
+        o << "template <bool UL>\n__device__ __forceinline__ void eval_body(\n" << PARAMS;
+        emit_prologue();
+        emit_coefs(G, "  ", COEF_UL);
+        o << VALUE_ACCS;
+        emit_accs(G);
+        if (M.lds_pipe) {
+            // Tiles of WGS events: every per-event input row of the next tile is copied
+            // HBM -> LDS by the DMA path (global_load_lds_dwordx4, no registers held) while
+            // the current tile is computed from LDS.  Row r of a tile occupies
+            // [roff_r, roff_r + WGS * es_r) of the tile buffer; the event layout (class
+            // offsets and leading dimension multiples of 64 events) keeps every 16-byte chunk
+            // aligned and inside its row.
+            struct Row { std::string src; int es; long long off; std::string rd; };
+            std::vector<Row> rows;
+            long long tb = 0;
+            const int esl = M.mixed ? 8 : 16;
+            for (int u : G.us)
+                for (int p = 0; p < NP; ++p) {
+                    std::string nm = std::to_string(u) + "_" + std::to_string(p);
+                    if (p >= NPS) {
+                        rows.push_back(Row{std::string(), 0, tb, mirror(u, p, "    ")});
+                        continue;
+                    }
+                    std::ostringstream src;
+                    src << "(const unsigned char*)sl + " << (long long)u * NPS + p << "LL * ld * " << esl;
+                    std::ostringstream rd;
+                    rd << "    const " << SLT << " g" << nm << " = ((const " << SLT << "*)(B + " << tb << "))[threadIdx.x];\n"
+                       << "    const double2 s" << nm << " = " << sl_conv("g" + nm) << ";\n";
+                    rows.push_back(Row{src.str(), esl, tb, rd.str()});
+                    tb += (long long)WGS * esl;
+                }
+            for (int i : G.invs) {
+                std::ostringstream src, rd;
+                if (imap[i] >= 0) {
+                    src << "(const unsigned char*)inv + " << imap[i] << "LL * ld * 8";
+                    rd << "    const double x" << i << " = ((const double*)(B + " << tb << "))[threadIdx.x];\n";
+                    rows.push_back(Row{src.str(), 8, tb, rd.str()});
+                    tb += (long long)WGS * 8;
+                } else {
+                    src << "(const unsigned char*)invf + " << (-imap[i] - 1) << "LL * ld * 4";
+                    rd << "    const double x" << i << " = (double)((const float*)(B + " << tb << "))[threadIdx.x];\n";
+                    rows.push_back(Row{src.str(), 4, tb, rd.str()});
+                    tb += (long long)WGS * 4;
+                }
+            }
+            o << "  typedef __attribute__((address_space(3))) void* lds_ptr;\n";
+            o << "  const int ntile = (int)((e1 - e0 + " << WGS - 1 << ") / " << WGS << ");\n";
+            // issue the copies of the tile starting at event ts into buffer dst
+            o << "  auto issue = [&](unsigned char* dst, const long long ts) {\n"
+                 "    const int t = threadIdx.x;\n";
+            for (const Row& r : rows) {
+                if (r.es == 0) continue;             // a mirrored polarisation: no copy
+                int nl = WGS * r.es / 16;
+                o << "    if (t < " << nl << " && ts + (long long)(t * " << 16 / r.es << ") < e1)\n"
+                  << "      __builtin_amdgcn_global_load_lds((const void*)(" << r.src << " + ts * " << r.es << " + t * 16),\n"
+                  << "                                     (lds_ptr)(dst + " << r.off << " + (t & ~63) * 16), 16, 0, 0);\n";
+            }
+            o << "  };\n";
+            o << "  issue(lbuf, e0);\n";
+            o << "  for (int it = 0; it < ntile; ++it) {\n"
+                 "    const long long ts = e0 + (long long)it * " << WGS << ";\n"
+                 "    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this thread's copies landed\n"
+                 "    __syncthreads();                      // every thread's copies landed; previous tile consumed\n"
+                 "    if (it + 1 < ntile) issue(lbuf + ((it + 1) & 1) * " << tb << ", ts + " << WGS << ");\n"
+                 "    const unsigned char* B = lbuf + (it & 1) * " << tb << ";\n"
+                 "    const long long e = ts + threadIdx.x;\n"
+                 "    if (e < e1) {\n";
+            for (const Row& r : rows) o << r.rd;
+            tile_bytes = tb;
+        } else if (M.prefetch_sl) {
+            const int depth = M.prefetch_sl;
+            o << "  long long e = e0 + threadIdx.x;\n  const long long ep = (e < e1) ? e : e0;\n";
+            decl_set(G, "n", "ep");
+            o << "  double nwt = pw ? wts[ep] : wc;\n";
+            if (depth > 1) {
+                o << "  const long long ep2 = (e + " << WGS << " < e1) ? e + " << WGS << " : e0;\n";
+                decl_set(G, "m", "ep2");
+                o << "  double mwt = pw ? wts[ep2] : wc;\n";
+            }
+            o << "  for (; e < e1; e += " << WGS << ") {\n";
+            use_set(G);
+            const long long ahead = (long long)depth * WGS;
+            o << "    { const long long en = (e + " << ahead << " < e1) ? e + " << ahead << " : e;\n";
+            next_set(G, depth);
+            o << "    }\n";
+        } else {
+            o << "  for (long long e = e0 + threadIdx.x; e < e1; e += " << WGS << ") {\n";
+            for (int u : G.us)
+                for (int p = 0; p < NP; ++p) {
+                    std::string nm = std::to_string(u) + "_" + std::to_string(p);
+                    if (p >= NPS) {
+                        o << mirror(u, p, "    ");
+                        continue;
+                    }
+                    o << "    const " << SLT << " g" << nm << " = sl[" << (long long)u * NPS + p << "LL * ld + e];\n";
+                    o << "    const double2 s" << nm << " = " << sl_conv("g" + nm) << ";\n";
+                }
+            for (int i : G.invs) o << "    const double x" << i << " = " << inv_load(i, "e") << ";\n";
+        }
+        emit_core(G);
+        emit_sums(G);
+        emit_weights(M.prefetch_sl && !M.lds_pipe ? "wev" : "pw ? wts[e] : wc", true, false);
+        emit_adjoint(G);
+        o << (M.lds_pipe ? "    }\n  }\n" : "  }\n");
+        emit_log();
+        std::vector<std::string> accs = acc_names(G);
+        accs.insert(accs.begin(), "av");
+        if ((int)accs.size() != NACC) throw std::runtime_error("fused kernel generator: accumulator count mismatch");
+        if (M.lds_pipe) o << "  __syncthreads();                 // every wave is done with the tile buffers\n";
+        o << "  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;\n";
+        emit_reduce(accs, [](int c0) { return "red[wave][" + std::to_string(c0) + " + k4]"; });
+        o << "  __syncthreads();\n";
+        // fixed-order combination of the wave partials
+        std::string comb;
+        if (NW == 1) comb = "red[0][k]";
+        else if (NW == 2) comb = "red[0][k] + red[1][k]";
+        else comb = "(red[0][k] + red[1][k]) + (red[2][k] + red[3][k])";
+        o << "  for (int k = threadIdx.x; k < " << NACC << "; k += " << WGS << ")\n"
+             "    part[(long long)k * nwg + wg] = " << comb << ";\n";
+        o << "}\n";
+    } else {
+        // Wave groups: the workgroup's waves take the same 64 events.  Each evaluates its
+        // own blocks, writes its share of S_p to LDS and, after one barrier, adds all
+        // shares in group order, so every wave has the event's S, I and weights; then it
+        // accumulates its own blocks' sums.  The exchange buffer is double buffered: a wave
+        // writes a buffer again only after the following iteration's barrier, which every
+        // wave reaches after its reads of it.  All waves run the same number of
+        // iterations (the barriers), lanes past the end contribute nothing.
+        const int NX = 2 * NP;
+        for (int g = 0; g < NG; ++g) {
+            const Group& G = groups[g];
+            o << "template <bool UL>\n__device__ __forceinline__ void eval_g" << g << "(\n" << PARAMS;
+            emit_prologue();
+            if (g == 0) o << VALUE_ACCS;
+            emit_accs(G);
+            o << "  const int lane = threadIdx.x & 63, wave = " << g << ";\n"
+                 "  double* xch = (double*)lbuf;\n"
+                 "  const int niter = (int)((e1 - e0 + 63) >> 6);\n"
+                 "  const long long ep = (e0 + lane < e1) ? e0 + lane : e0;\n";
+            decl_set(G, "n", "ep");
+            o << "  double nwt = pw ? wts[ep] : wc;\n"
+                 "  const long long ld_arg = ld;\n"
+                 "  for (int it = 0; it < niter; ++it) {\n"
+                 "    const long long er = e0 + (long long)it * 64 + lane;\n"
+                 "    const bool live = er < e1;\n"
+                 "    const long long e = live ? er : e0;\n"
+                 "    (void)e;\n"
+                 // a zero the optimiser cannot see through keeps the coefficient loads in the loop
+                 "    long long z = 0;\n    asm volatile(\"\" : \"+s\"(z));\n    const long long ld = ld_arg + z;\n"
+                 "    const __attribute__((address_space(4))) double* tc = (const __attribute__((address_space(4))) double*)(tb + z);\n";
+            emit_coefs(G, "    ", COEF_LOOP);
+            use_set(G);
+            o << "    { const long long en = (er + 64 < e1) ? er + 64 : e0;\n";
+            next_set(G, 1);
+            o << "    }\n";
+            emit_core(G);
+            emit_sums(G);
+            o << "    double* xb = xch + (it & 1) * " << NG * NX * 64 << " + lane;\n";
+            for (int p = 0; p < NP; ++p)
+                o << "    xb[" << (g * NX + 2 * p) * 64 << "] = S" << p << "r; xb[" << (g * NX + 2 * p + 1) * 64 << "] = S" << p << "i;\n";
+            o << "    __syncthreads();\n";
+            for (int p = 0; p < NP; ++p)
+                for (int c = 0; c < 2; ++c) {
+                    o << "    S" << p << (c ? "i" : "r") << " = xb[" << (2 * p + c) * 64 << "]";
+                    for (int h = 1; h < NG; ++h) o << " + xb[" << (h * NX + 2 * p + c) * 64 << "]";
+                    o << ";\n";
+                }
+            emit_weights("wev", g == 0, true);
+            o << "    long long z2 = 0;\n    asm volatile(\"\" : \"+s\"(z2));\n    {\n"
+                 "    const __attribute__((address_space(4))) double* tc = (const __attribute__((address_space(4))) double*)(tb + z2);\n";
+            emit_coefs(G, "    ", COEF_AGAIN);
+            emit_adjoint(G);
+            o << "    }\n  }\n";
+            if (g == 0) emit_log();
+            o << "  __syncthreads();                 // the exchange buffers become the reduction's slabs\n";
+            std::vector<std::string> accs = acc_names(G);
+            const int na = 2 * (int)G.amps.size(), nt = (int)G.ths.size();
+            const long long A0 = 1 + 2LL * G.amps[0], T0 = 1 + 2LL * P.namp + (nt ? G.ths[0] : 0),
+                            C0 = 1 + 2LL * P.namp + (long long)M.thterms.size() + (G.cts.empty() ? 0 : G.cts[0]);
+            if (g == 0) {
+                o << "  for (int s = 32; s > 0; s >>= 1) av += __shfl_xor(av, s, 64);\n"
+                     "  if (lane == 0) part[wg] = av;\n";
+            }
+            emit_reduce(accs, [&](int c0) {
+                std::ostringstream q;
+                q << "part[(k4 < " << na - c0 << " ? " << A0 + c0 << "LL + k4 : k4 < " << na + nt - c0 << " ? " << T0 + c0 - na
+                  << "LL + k4 : " << C0 + c0 - na - nt << "LL + k4) * nwg + wg]";
+                return q.str();
+            });
+            o << "}\n";
+        }
+        o << "template <bool UL>\n__device__ __forceinline__ void eval_body(\n" << PARAMS
+          << "  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));\n  switch (wave) {\n";
+        for (int g = 0; g < NG; ++g)
+            o << "  " << (g + 1 < NG ? "case " + std::to_string(g) : std::string("default")) << ": eval_g" << g
+              << "<UL>(tab, slv, inv, invf, wts, part, wg_cls, wg_rng, ld, nwg, w1, w2, pw1, pw2, wg, red, lbuf, cfb); break;\n";
+        o << "  }\n}\n";
     }
-    o << "  }\n  __syncthreads();\n";
-    // fixed-order combination of the wave partials
-    std::string comb;
-    if (NW == 1) comb = "red[0][k]";
-    else if (NW == 2) comb = "red[0][k] + red[1][k]";
-    else comb = "(red[0][k] + red[1][k]) + (red[2][k] + red[3][k])";
-    o << "  for (int k = threadIdx.x; k < " << NACC << "; k += " << WGS << ")\n"
-         "    part[(long long)k * nwg + wg] = " << comb << ";\n";
-    o << "}\n";
     std::string lb = "__launch_bounds__(" + std::to_string(WGS) + (M.min_waves > 0 ? ", " + std::to_string(M.min_waves) : std::string()) + ")";
     std::ostringstream decl;
-    decl << "  __shared__ double red[" << NW << "][" << NACC << "];\n"
+    decl << "  __shared__ double red[" << (NG > 1 ? 1 : NW) << "][" << (NG > 1 ? 1 : NACC) << "];\n"
          << "  __shared__ __attribute__((aligned(16))) unsigned char lbuf["
-         << std::max<long long>(M.lds_pipe ? 2 * tile_bytes : 0, (long long)NW * 64 * 17 * 8) << "];\n";
+         << std::max<long long>({M.lds_pipe && NG == 1 ? 2 * tile_bytes : 0, (long long)NW * 64 * 17 * 8,
+                                 NG > 1 ? 2LL * NG * 2 * NP * 64 * 8 : 0}) << "];\n";
     o << "extern \"C\" __global__ void " << lb << " ctpwa_eval(\n"
          "    const double* __restrict__ tab, const void* __restrict__ slv, const double* __restrict__ inv,\n"
          "    const float* __restrict__ invf, const double* __restrict__ wts, double* __restrict__ part,\n"
@@ -1219,6 +1403,7 @@ std::string generate_eval_kernel(const Model_& M) {
          "    if (atomicAdd(&ctr[1], 1u) == gridDim.x - 1) { atomicExch(&ctr[0], 0u); atomicExch(&ctr[1], 0u); }\n"
          "  }\n}\n";
     if (!M.customs.empty()) {
+        const int NU = (int)M.us.size(), NA = P.namp;
         // Custom factors and their derivatives for every stored event at the current
         // parameter point, rows [c * NCF + (r, i, dr[0..NCV), di[0..NCV))] of cfb.  A kernel
         // of its own: the complex-dual expression code then never shares registers with
@@ -1251,10 +1436,10 @@ std::string generate_eval_kernel(const Model_& M) {
              "    const float* __restrict__ invf, long long ld, long long e0, long long n, double* __restrict__ out,\n"
              "    int intensity, const double* __restrict__ cfb)\n{\n";
         o << "  const " << SLT << "* __restrict__ sl = (const " << SLT << "*)slv;\n  const double* tb = tab;\n";
-        emit_coefs("  ", false);
+        emit_coefs(all, "  ", COEF_TAB);
         o << "  const long long ie = (long long)blockIdx.x * 256 + threadIdx.x;\n  if (ie >= n) return;\n"
              "  const long long e = e0 + ie;\n  {\n";
-        for (int u = 0; u < NU; ++u)
+        for (int u : all.us)
             for (int p = 0; p < NP; ++p) {
                 std::string nm = std::to_string(u) + "_" + std::to_string(p);
                 if (p >= NPS) {
@@ -1264,9 +1449,8 @@ std::string generate_eval_kernel(const Model_& M) {
                 o << "    const " << SLT << " g" << nm << " = sl[" << (long long)u * NPS + p << "LL * ld + e];\n";
                 o << "    const double2 s" << nm << " = " << sl_conv("g" + nm) << ";\n";
             }
-        for (size_t i = 0; i < M.inv.size(); ++i)
-            if (used[i]) o << "    const double x" << i << " = " << inv_load(i, "e") << ";\n";
-        emit_core(o);
+        for (int i : all.invs) o << "    const double x" << i << " = " << inv_load(i, "e") << ";\n";
+        emit_core(all);
         o << "    if (intensity) {\n";
         for (int u = 0; u < NU; ++u) o << "      double y" << u << "r = 0.0, y" << u << "i = 0.0;\n";
         for (int a = 0; a < NA; ++a) {

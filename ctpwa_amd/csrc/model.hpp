@@ -185,6 +185,7 @@ struct USpec { int topo, slc; uint32_t mask; };   // mask bit k: fold node k's b
 struct Term { int inv; int coef; double cval; };   // inv < 0: constant 1; coef < 0: constant cval
 struct DenSpec {
     int block, res, node;
+    int kin = -1;               // kinematic node of the mother
     // D = sum re - i sum im; a static factor (table lineshapes) is instead the factor
     // F = sum re + i sum im itself, without theta dependence
     std::vector<Term> re, im;
@@ -223,11 +224,23 @@ struct Model_ {
     std::vector<AmpSpec> amps;                    // [namp]
     std::vector<std::vector<int>> bvars;          // [block] -> local var -> global slot
     std::vector<ThTerm> thterms;                  // theta-gradient accumulators
+    int nth_all = 0;                              // their number without merging equal propagators
     std::vector<CustomSpec> customs;
     std::vector<std::vector<int>> block_customs;  // [block] -> custom indices
     std::vector<CTerm> cterms;                    // Custom theta-gradient accumulators
     std::vector<double> tabs;                     // table lineshapes, concatenated
     int maxloc = 0;
+    // Propagators equal by construction (same kinematic node, lineshape and parameter
+    // sources) within one wave group: den_canon[d] is the first of them.  The fused kernel
+    // evaluates and accumulates the first only.
+    std::vector<int> den_canon;
+    // Wave groups of the fused kernel: 1 (every wave evaluates all blocks for its own
+    // events), or the waves of a workgroup share 64 events and wave g evaluates the blocks
+    // with bgroup[b] == g (contiguous in plan order).
+    int groups = 1;
+    std::vector<int> bgroup;
+    // events a workgroup of the fused kernel takes per loop iteration
+    int ev_step() const { return groups > 1 ? 64 : wgs; }
     // code-generation options of the fused kernel
     int min_waves = 0;       // __launch_bounds__ minimum waves per SIMD (0: compiler choice)
     int wgs = 128;           // threads (= events per tile) of a workgroup: 64, 128 or 256
@@ -288,6 +301,108 @@ inline uint32_t ref_set(const PTopo& T, int ref, int nfinal, int depth = 0) {
     int k = -ref - 1;
     if (k <= 0 || k >= (int)T.nodes.size()) throw std::runtime_error("bad node reference");
     return ref_set(T, T.nodes[k].d1ref, nfinal, depth + 1) | ref_set(T, T.nodes[k].d2ref, nfinal, depth + 1);
+}
+
+// source of parameter k of a resonance: its theta slot or fixed value
+inline std::string param_src(const PRes& R, int k) {
+    std::ostringstream q;
+    q.precision(17);
+    if ((int)R.params.size() <= k) q << "none";
+    else if ((int)R.slots.size() > k && R.slots[k] >= 0) q << "slot" << R.slots[k];
+    else q << "val" << R.params[k];
+    return q.str();
+}
+// source of a daughter's mass in a vertex's q0 (see q0_dmass in prep.hip)
+inline std::string q0_mass_src(const PBlock& B, double cfg, int ref) {
+    std::ostringstream q;
+    q.precision(17);
+    if (cfg > 0) q << "cfg" << cfg;
+    else if (ref >= 0) q << "zero";
+    else {
+        q << "one";
+        for (const PRes& r : B.res)
+            if (r.node == -ref - 1 && !r.params.empty()) { q.str(""); q << param_src(r, 0); break; }
+    }
+    return q.str();
+}
+// everything a propagator's value and coefficients depend on besides the event
+inline std::string den_key(const Model_& M, int d) {
+    const DenSpec& D = M.dens[d];
+    const PBlock& B = M.P.blocks[D.block];
+    const PRes& R = B.res[D.res];
+    const PNode& n = M.P.topos[B.topo].nodes[D.node];
+    std::ostringstream q;
+    q.precision(17);
+    q << D.kin << "|" << R.model;
+    for (size_t k = 0; k < R.params.size(); ++k) q << "|" << param_src(R, (int)k);
+    for (double c : R.ch) q << "|c" << c;
+    q << "|" << n.lmin << "|" << (n.has_bf ? n.bf_d : 0.0) << "|" << q0_mass_src(B, n.md1, n.d1ref) << "|"
+      << q0_mass_src(B, n.md2, n.d2ref);
+    for (const Term& t : D.re) q << "|r" << t.inv << "," << t.coef << "," << t.cval;
+    for (const Term& t : D.im) q << "|i" << t.inv << "," << t.coef << "," << t.cval;
+    return q.str();
+}
+
+// Wave groups of the fused kernel and the equal propagators within each.
+//
+// One thread that carries every accumulator of an event needs about 2 x (2 namp) vector
+// registers for them; past some 24 amplitudes they no longer fit and go to scratch (149
+// amplitudes, FP64: 6.27 ms per evaluation of 1.5M events, 0.25 TB/s).  Such a model's
+// blocks are shared out among the waves of a workgroup, at most 8 of them with about 19
+// amplitudes each: what one wave then holds is what the kernel of a 20-amplitude model
+// holds (0.50 ms, 3.2 TB/s; two waves per SIMD, about 500 FP64 instructions per wave and
+// iteration).  6 groups of 25 amplitudes spill (1.14 ms), and so do 10 of 15, whose ten
+// waves leave each only 168 registers (1.37 ms).
+// Blocks stay in plan order, so that a group's SL tensors, amplitudes and accumulators are
+// contiguous; the cuts minimise the largest group's cost in FP64 instructions.
+inline void assign_groups(Model_& M) {
+    const Plan& P = M.P;
+    std::vector<int> bl;
+    for (size_t b = 0; b < P.blocks.size(); ++b) if (P.blocks[b].nsl > 0) bl.push_back((int)b);
+    std::vector<std::string> key(M.dens.size());
+    for (size_t d = 0; d < M.dens.size(); ++d) key[d] = den_key(M, (int)d);
+    const int n = (int)bl.size();
+    int G = P.namp <= 24 ? 1 : std::min(8, (P.namp + 18) / 19);
+    G = std::max(1, std::min(G, n));
+    M.bgroup.assign(P.blocks.size(), 0);
+    if (G > 1) {
+        // cost[i][j]: blocks bl[i..j) as one group
+        std::vector<std::vector<double>> cost(n, std::vector<double>(n + 1, 0.0));
+        for (int i = 0; i < n; ++i) {
+            std::vector<char> us(M.us.size(), 0);
+            std::map<std::string, int> ds;
+            double c = 0.0;
+            for (int j = i; j < n; ++j) {
+                const PBlock& B = P.blocks[bl[j]];
+                c += 6.0 + 14.0 * B.nsl + 20.0 * (double)M.block_customs[bl[j]].size();
+                for (int k = 0; k < B.nsl; ++k) {
+                    const int u = M.amps[B.site + k].u;
+                    if (!us[u]) { us[u] = 1; c += 10.0; }
+                }
+                for (int d : M.block_dens[bl[j]]) if (!ds[key[d]]++) c += 16.0;
+                cost[i][j + 1] = c;
+            }
+        }
+        std::vector<std::vector<double>> best(G + 1, std::vector<double>(n + 1, 1e300));
+        std::vector<std::vector<int>> cut(G + 1, std::vector<int>(n + 1, 0));
+        best[0][0] = 0.0;
+        for (int g = 1; g <= G; ++g)
+            for (int j = g; j <= n; ++j)
+                for (int i = g - 1; i < j; ++i) {
+                    const double v = std::max(best[g - 1][i], cost[i][j]);
+                    if (v < best[g][j]) { best[g][j] = v; cut[g][j] = i; }
+                }
+        for (int g = G, j = n; g > 0; --g) {
+            for (int k = cut[g][j]; k < j; ++k) M.bgroup[bl[k]] = g - 1;
+            j = cut[g][j];
+        }
+        M.wgs = 64 * G;
+    }
+    M.groups = G;
+    std::map<std::pair<int, std::string>, int> first;
+    M.den_canon.resize(M.dens.size());
+    for (size_t d = 0; d < M.dens.size(); ++d)
+        M.den_canon[d] = first.emplace(std::make_pair(M.bgroup[M.dens[d].block], key[d]), (int)d).first->second;
 }
 
 inline Model_ derive(const Plan& P) {
@@ -385,7 +500,8 @@ inline Model_ derive(const Plan& P) {
             int k = R.node;
             int kin = M.topo_kin[B.topo][k];
             const PNode& n = T.nodes[k];
-            DenSpec D{(int)b, (int)r, k, {}, {}, 0, rec};
+            DenSpec D;
+            D.block = (int)b; D.res = (int)r; D.node = k; D.kin = kin; D.coef_base = rec;
             auto S = add_inv({kin, INV_S, 0, 0.0, 0.0, 0.0});
             auto ONE = add_inv({kin, INV_ONE, 0, 0.0, 0.0, 0.0});
             switch (R.model) {
@@ -510,9 +626,14 @@ inline Model_ derive(const Plan& P) {
             M.amps[a] = AmpSpec{(int)b, sc, u, 0};
         }
     }
+    assign_groups(M);
     for (size_t d = 0; d < M.dens.size(); ++d) {
         const DenSpec& Dn = M.dens[d];
-        if (M.bvars[Dn.block].empty()) continue;
+        if (!M.bvars[Dn.block].empty())
+            for (const std::vector<Term>* ts : {&Dn.re, &Dn.im})
+                for (const Term& t : *ts) M.nth_all += t.coef >= 0;
+        // (a propagator without a free parameter has no coefficient derivatives)
+        if (M.den_canon[d] != (int)d || den_key(M, (int)d).find("slot") == std::string::npos) continue;
         for (const Term& t : Dn.re) if (t.coef >= 0) M.thterms.push_back(ThTerm{(int)d, t.coef, 0, t.inv});
         for (const Term& t : Dn.im) if (t.coef >= 0) M.thterms.push_back(ThTerm{(int)d, t.coef, 1, t.inv});
     }

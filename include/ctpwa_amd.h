@@ -79,8 +79,8 @@ int ctpwa_nll_grad(ctpwa_handle* h, const double* params_dev, double* out_dev, v
  * totals live in a library-owned static device array of 2 MiB per GPU (held until the
  * process ends) instead of the handle's buffers; the result is bit-identical to
  * ctpwa_nll_grad.  A model whose partials exceed the array (n_acc x n_workgroups +
- * 3 n_acc > 262144 doubles, n_acc = 1 + 2 n_amp + theta-gradient terms, at most 1024
- * workgroups) is rejected with an error.  All calls on one GPU share the
+ * 3 n_acc > 262144 doubles, n_acc = 1 + 2 n_amp + theta-gradient terms counted for every
+ * propagator, one workgroup per 256 events and at most 1024) is rejected with an error.  All calls on one GPU share the
  * array: calls that overlap on one GPU race. */
 int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev, double* out_dev, void* stream);
 
