@@ -23,7 +23,7 @@
 namespace ctpwa {
 std::string generate_eval_kernel(const Model_& M);
 std::string generate_custom2_kernel(const Model_& M);
-std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm);
+std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool amps_only);
 }
 
 extern "C" hipError_t ctpwa_launch_init(const double*, long long, int, const ctpwa::DTopo*, int, const ctpwa::DNode*,
@@ -43,14 +43,16 @@ extern "C" hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs*, long long, long lo
 
 
 extern "C" hipError_t ctpwa_launch_zero(double*, long long, hipStream_t);
-extern "C" long long ctpwa_hess_rows_waves(long long);
-extern "C" hipError_t ctpwa_launch_accum_cols(const double*, long long, long long, int, const int*, double*, hipStream_t);
-extern "C" int ctpwa_gram_tables(int, int4*, int*, int2*);
-extern "C" int ctpwa_gram_nwg(int);
-extern "C" hipError_t ctpwa_launch_gram_panels(const void*, int, int, long long, long long, const double*, long long,
-                                                const int4*, int, int, double*, int, int, hipStream_t);
-extern "C" hipError_t ctpwa_launch_accum_panels(const double*, int, int, const int2*, int, double*, hipStream_t);
-extern "C" hipError_t ctpwa_launch_amp_rows(const ctpwa::AuxArgs*, long long, long long, double*, long long, int, hipStream_t);
+extern "C" int ctpwa_gram_tables(int, int2*, ctpwa::GramPair*, int*, int*);
+extern "C" int ctpwa_gram_nwg();
+extern "C" hipError_t ctpwa_launch_gram_panels(const void*, int, int, long long, const ctpwa::HessPieces*, int, const double*,
+                                                double*, hipStream_t);
+extern "C" hipError_t ctpwa_launch_gram_wide(const void*, int, int, long long, long long, long long, const double*,
+                                              const ctpwa::GramPair*, int, const int2*, const int*, int, int, double*, double*,
+                                              int, hipStream_t);
+extern "C" hipError_t ctpwa_launch_hess_accum(const ctpwa::HessPieces*, const ctpwa::HessPieces*, const ctpwa::HessTotals*,
+                                               const double*, int, const int2*, int, const double*, int, const int2*, int,
+                                               const double*, int, int, const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_partial_int(const ctpwa::AuxArgs*, const int*, const int*, int, long long, long long,
                                                double*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_partial_amp(const ctpwa::AuxArgs*, const int*, const int*, int, long long, long long,
@@ -241,44 +243,38 @@ static Staging* staging(int device) {          // called with `device` current
 }
 
 // ---------------------------------------------------------------------------
-// matrix-core Gram of ncol columns: panel pairs, tile-pair list, row-share workgroups
-// and the partials buffer [nwg][ntp][256]
+// matrix-core Gram of ncol columns: tile-pair list, workgroups, partials buffer; more than 64
+// columns: panel pairs and each tile pair's panel pair
 struct GramTabs {
     int ncol = 0, npp = 0, ntp = 0, nwg = 0;
-    int4* pp = nullptr;
+    GramPair* pp = nullptr;
     int2* tiles = nullptr;
+    int* tpair = nullptr;
     double* part = nullptr;
 };
-static long long gram_part_doubles(int ncol) {
-    int npp = 0;
-    const int ntp = ctpwa_gram_tables(ncol, nullptr, &npp, nullptr);
-    return (long long)ctpwa_gram_nwg(npp) * ntp * 256;
-}
 
 // serial numbers of handles: a handle created after another was destroyed may reuse its
 // address, never its serial
 static std::atomic<unsigned long long> g_handle_serial{0};
-// handles alive in the process (a handle's member counts itself in and out)
-static std::atomic<int> g_live_handles{0};
-struct LiveCount {
-    LiveCount() { ++g_live_handles; }
-    ~LiveCount() { --g_live_handles; }
-    LiveCount(const LiveCount&) = delete;
-    LiveCount& operator=(const LiveCount&) = delete;
-};
-
-// one set of Hessian buffers: a chunk of Jacobian rows (FP64, or FP32 in the mixed
-// form), u rows, weights, the rows kernel's per-wave column sums, and the matrix-core
-// Gram partials of the Jacobian (2C columns) and of u (NU columns)
-struct HessWS {
-    long long chunk = 0, cs_ld = 0;
+// Workspace of a generated per-event kernel with a Gram (the Hessian; the amplitude Gram):
+// the kernel, its shape, Jacobian rows of one pass (rows form), u rows, weights, the sums'
+// per-workgroup partials, and the Gram partials of the Jacobian (2C columns) and of u
+struct GramWS {
+    bool ready = false;
+    HessShape S;
+    hipModule_t mod = nullptr;
+    hipFunction_t fn = nullptr;
+    int nz = 0;                          // summed columns
+    int* perm = nullptr;                 // put order -> [Z | u] order
+    int target = 0;                      // workgroups of the per-event kernel
+    long long chunk = 0, cap = 0;        // events of a class per pass, events per pass
+    long long ldJ = 0, ldc = 0;
     void* J = nullptr;
-    double *U = nullptr, *W = nullptr, *cs = nullptr;
+    double *U = nullptr, *W = nullptr, *z = nullptr;
     GramTabs gJ, gU;
 };
 
 struct ctpwa_handle {
-    LiveCount live;
     int device = 0;
     const unsigned long long serial = ++g_handle_serial;
     Model_ M;
@@ -310,22 +306,12 @@ struct ctpwa_handle {
     int* wave_ptr = nullptr;               // partial wave w = blocks wave_blk[wave_ptr[w] .. wave_ptr[w+1])
     int* wave_blk = nullptr;
     std::string src;
-    // Hessian workspace (allocated on the first ctpwa_hessian call): the generated rows
-    // kernel, one chunk of Jacobian rows (FP64, or FP32 in the mixed form), u rows,
-    // weights, per-wave column sums, and the matrix-core Gram tables and partials of the
-    // Jacobian (2C columns) and of u (NU columns)
-    // Buffer set 0 serves the phase space on the caller's stream; set 1 serves data and
-    // background on a stream of the handle, so the two run concurrently.
-    bool hess_ready = false;
-    int hC = 0, hNU = 0, hNZ = 0, hnG = 0, hnUu = 0;
-    hipModule_t hmod = nullptr;
-    hipFunction_t fn_hrows = nullptr;
-    HessWS hws[2];
-    hipStream_t hs2 = nullptr;                  // default priority, non-blocking
-    hipEvent_t hev[2] = {nullptr, nullptr};     // start of the classes' work; end of set 1's work
-    double *htot = nullptr, *hHext = nullptr;
+    // Hessian workspace (allocated on the first ctpwa_hessian call)
+    GramWS hess;
+    int hnG = 0, hnUu = 0, hNZ = 0;
+    double* htot = nullptr;
+    int *hzvt = nullptr, *http = nullptr, *httl = nullptr;   // second-part sums of the assembly (HessAsm)
     int *hmap_ptr = nullptr, *hmap_x = nullptr;   // fit parameter -> extended entries (CSR)
-    int* hperm = nullptr;                         // rows kernel's summed columns -> [Z | u] order
     double* hmap_r = nullptr;
     // models with Custom lineshapes: second-order factor rows for the Hessian, from a
     // module compiled on the first Hessian call
@@ -334,10 +320,8 @@ struct ctpwa_handle {
     double* cfb2 = nullptr;
     int *hbcp = nullptr, *hbcl = nullptr;   // per-block Custom factor lists (CSR)
     // amplitude-Gram workspace (allocated on the first ctpwa_amplitude_gram call)
-    bool agram_ready = false;
-    long long gchunk = 0;
-    double *gX = nullptr, *gW = nullptr, *gtot = nullptr;
-    GramTabs gg;
+    GramWS agram;
+    double* gtot = nullptr;
     // no free resonance parameter: the phase-space amplitude Gram without couplings or
     // theta coefficients, built once at creation; the evaluations then scan data and
     // background only (fin.gram points here)
@@ -372,10 +356,6 @@ struct ctpwa_handle {
         int prev = 0;
         (void)hipGetDevice(&prev);
         (void)hipSetDevice(device);
-        if (hs2) (void)hipStreamSynchronize(hs2);
-        if (hs2) (void)hipStreamDestroy(hs2);
-        for (hipEvent_t ev : hev)
-            if (ev) (void)hipEventDestroy(ev);
         // the modules belong to the process-wide compile cache (shared by handles of one
         // model), not to the handle
         for (void* p : allocs) (void)hipFree(p);
@@ -1086,20 +1066,17 @@ extern "C" int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev,
 }
 
 
-// Hessian workspace: Jacobian columns C, u-vector length NU, second-part scalars NZ per event
-struct HessDims { int C, NU, NZ; };
-static HessDims hess_dims(const Model_& M) {
-    const Plan& P = M.P;
-    HessDims d{P.namp + P.ntheta, 2 * P.namp + P.ntheta, 1};
-    for (size_t b = 0; b < P.blocks.size(); ++b) {
-        if (P.blocks[b].nsl == 0) continue;
-        int nl = (int)M.bvars[b].size();
-        d.NZ += P.blocks[b].nsl * 2 * nl + nl * (nl + 1) / 2;
+// second-part sums (and the sum of alpha I) of a model's Hessian
+static int hess_nz(const Model_& M) {
+    int nz = 1;
+    for (size_t b = 0; b < M.P.blocks.size(); ++b) {
+        if (M.P.blocks[b].nsl == 0) continue;
+        const int nl = (int)M.bvars[b].size();
+        nz += M.P.blocks[b].nsl * 2 * nl + nl * (nl + 1) / 2;
     }
-    return d;
+    return nz;
 }
-// events per chunk of Jacobian rows: the rows of one chunk take at most this many bytes
-// (environment CTPWA_HESS_JBYTES overrides it for measurements)
+// bytes of Jacobian rows per pass (environment CTPWA_HESS_JBYTES overrides it for measurements)
 static long long hess_jbytes() {
     if (const char* e = std::getenv("CTPWA_HESS_JBYTES")) {
         long long v = std::atoll(e);
@@ -1107,106 +1084,300 @@ static long long hess_jbytes() {
     }
     return 2LL << 30;
 }
-static long long hess_chunk(const Model_& M, long long maxn) {
-    const HessDims d = hess_dims(M);
-    const long long row = (long long)M.P.npol * 2 * d.C * 8;
-    long long c = std::max<long long>(256, hess_jbytes() / std::max<long long>(1, row) / 256 * 256);
-    // a multiple of 4 events: the Gram's 16-byte slab loads stay aligned
-    return (std::max<long long>(1, std::min(maxn, c)) + 3) / 4 * 4;
-}
-// The data and background classes run on a second stream of the handle, concurrently
-// with the phase space, when both sides are large enough for the overlap to outweigh the
-// two cross-stream waits, and only for a handle that is alone in the process (`others`:
-// the other live handles, counted when the buffers are set up and again at every call):
-// with several (a fit service) other handles' work fills the GPU, and a second stream
-// per handle, its events and its second buffer set cost more than they gain (measured:
-// Newton fits/hour of the service down by a quarter).  Environment CTPWA_HESS_STREAMS =
-// 1 or 2 forces one or two streams.
-static int hess_streams_env() {
-    if (const char* e = std::getenv("CTPWA_HESS_STREAMS")) {
-        const int k = std::atoi(e);
-        if (k != 1 && k != 2) throw std::runtime_error("CTPWA_HESS_STREAMS must be 1 or 2");
-        return k;
+static long long up(long long x, long long m) { return (x + m - 1) / m * m; }
+// Sizes of a GramWS for the classes' event counts: events of one class per pass (chunk, a
+// multiple of 256), events of all classes per pass (cap), workgroups (four waves' registers
+// and the LDS of a CU shared out among the CU's workgroups), and the buffers in doubles
+struct GramSizes {
+    long long chunk, cap, ldJ, ldc, J, U, W, z, part;     // ldJ, ldc: rows of J and of U, W
+    int target, nz;
+};
+// the partials of a Gram: ncol <= 64 at least one workgroup per piece; more columns: two
+// workgroups per CU shared out among the panel pairs by a wave's tile pairs
+static long long gram_plan(int ncol, int ncu, std::vector<GramPair>* pairs, int* nwg) {
+    int np = 0;
+    const int ntp = ctpwa_gram_tables(ncol, nullptr, nullptr, &np, nullptr);
+    if (ncol <= 64) {
+        *nwg = ctpwa_gram_nwg() + 4;
+        return (long long)*nwg * ntp * 256;
     }
-    return 0;
-}
-static bool hess_two_streams(const long long n3[3], int others) {
-    const int k = hess_streams_env();
-    if (k) return k == 2 && n3[0] > 0 && n3[1] + n3[2] > 0;
-    return others == 0 && n3[0] >= (1LL << 20) && n3[1] + n3[2] >= (1LL << 17);
-}
-// events per chunk of each buffer set: with two streams set 0 takes the phase space and
-// set 1 data and background; with one stream set 0 takes every class
-static void hess_chunks(const Model_& M, const long long n3[3], int others, long long ch[2]) {
-    const long long n12 = std::max(n3[1], n3[2]);
-    if (!hess_two_streams(n3, others)) {
-        ch[0] = hess_chunk(M, std::max(n3[0], n12));
-        ch[1] = 0;
-        return;
+    std::vector<GramPair> pp((size_t)np);
+    ctpwa_gram_tables(ncol, nullptr, pp.data(), &np, nullptr);
+    const int budget = std::max(2 * ncu, np);
+    int cost = 0;
+    for (const GramPair& p : pp) cost += p.nq;
+    long long off = 0;
+    int s0 = 0;
+    for (GramPair& p : pp) {
+        p.s0 = s0;
+        p.ns = std::max(1, (int)((long long)budget * p.nq / cost));
+        p.off = off;
+        s0 += p.ns;
+        off += (long long)p.ns * p.nt;
     }
-    ch[0] = hess_chunk(M, n3[0]);
-    ch[1] = hess_chunk(M, n12);
+    *nwg = s0;
+    if (pairs) *pairs = pp;
+    return off * 256;
 }
-static long long hess_workspace_bytes(const Model_& M, const long long n3[3], long long ntot, int others) {
-    HessDims d = hess_dims(M);
-    long long ch[2];
-    hess_chunks(M, n3, others, ch);
-    long long nG = (long long)(2 * d.C) * (2 * d.C + 1) / 2, nUu = (long long)d.NU * (d.NU + 1) / 2;
-    long long w = 3 * (nG + nUu + d.NZ + d.NU) + (long long)d.NU * d.NU;
-    for (int k = 0; k < 2; ++k) {
-        if (ch[k] == 0) continue;
-        w += ch[k] * (M.P.npol * 2LL * d.C + d.NU + 2) + (long long)(d.NZ + d.NU) * ctpwa_hess_rows_waves(ch[k]);
-        w += gram_part_doubles(2 * d.C) + gram_part_doubles(d.NU);
+static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long n3[3], int ncu) {
+    GramSizes z{};
+    const long long row = (long long)M.P.npol * 2 * S.C * 8;
+    z.chunk = std::max<long long>(256, hess_jbytes() / row / 256 * 256);
+    const long long all = n3[0] + n3[1] + n3[2];
+    z.cap = std::max<long long>(1, std::min(all, z.chunk));
+    const int per_cu = std::max(1, (int)std::min<long long>(8 / S.G, 160 * 1024 / std::max<long long>(1, S.lds * 8)));
+    // (a class smaller than a workgroup's share still gets one)
+    z.target = (int)std::min<long long>((long long)ncu * per_cu, std::max<long long>(1, (all + 63) / 64)) + 4;
+    z.nz = S.NU > 0 ? hess_nz(M) + S.NU : 0;
+    z.z = (long long)z.nz * z.target;
+    if (S.fused) {
+        z.chunk = std::max<long long>(1, all);
+        z.cap = all;
+        const int gt = (2 * S.C + 15) / 16, ut = (S.NU + 15) / 16;
+        z.part = (long long)z.target * (gt * (gt + 1) / 2 + ut * (ut + 1) / 2) * 256;
+        return z;
     }
-    w += (long long)M.customs.size() * M.ncf2() * ntot;   // second-order Custom factor rows
-    return w * 8 + 64 * 1024;    // + the index tables and allocation slack
+    z.ldJ = up((long long)M.P.npol * z.cap + 4 * 32, 32);
+    z.ldc = up(z.cap + 4 * 64, 64);
+    z.J = z.ldJ * 2 * S.C;
+    z.U = z.ldc * S.NU;
+    z.W = z.ldc * 2;
+    int nwg = 0;
+    z.part = gram_plan(2 * S.C, ncu, nullptr, &nwg) + (S.NU > 0 ? gram_plan(S.NU, ncu, nullptr, &nwg) : 0);
+    return z;
+}
+static int device_cus(int device) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) return 256;
+    return n;
+}
+static long long hess_workspace_bytes(const Model_& M0, const long long n3[3], long long ntot) {
+    long long most = 0;
+    for (int mixed = 0; mixed < 2; ++mixed) {       // the larger of the two storage forms
+        Model_ M = M0;
+        M.mixed = mixed;
+        const HessShape S = hess_shape(M, false);
+        const GramSizes z = gram_sizes(M, S, n3, 256);
+        const long long nG = (long long)(2 * S.C) * (2 * S.C + 1) / 2, nUu = (long long)S.NU * (S.NU + 1) / 2;
+        long long w = 3 * (nG + nUu + z.nz) + (S.f32 ? z.J / 2 : z.J) + z.U + z.W + z.z + z.part;
+        w += (long long)M.P.ntheta * M.P.ntheta * 4 + (long long)M.P.namp * M.P.ntheta;      // index tables
+        w += (long long)M.customs.size() * M.ncf2() * ntot;   // second-order Custom factor rows
+        most = std::max(most, w);
+    }
+    return most * 8 + 64 * 1024;    // + the smaller tables and allocation slack
 }
 
-static void gram_setup(ctpwa_handle* h, GramTabs& g, int ncol) {
+// the amplitude Gram's workspace for classes of up to n events
+static long long agram_workspace_bytes(const Model_& M, long long n) {
+    const long long n3[3] = {n, 0, 0};
+    const HessShape S = hess_shape(M, true);
+    const GramSizes z = gram_sizes(M, S, n3, 256);
+    return (z.J + z.U + z.W + z.z + z.part + (long long)M.P.namp * (2 * M.P.namp + 1)) * 8;
+}
+
+// nwg > 0: the fused form's workgroups, each with its tile pairs' sums
+static void gram_setup(ctpwa_handle* h, GramTabs& g, int ncol, int nwg) {
     g.ncol = ncol;
-    int npp = 0;
-    g.ntp = ctpwa_gram_tables(ncol, nullptr, &npp, nullptr);
-    std::vector<int4> pp((size_t)npp);
+    g.ntp = ctpwa_gram_tables(ncol, nullptr, nullptr, &g.npp, nullptr);
     std::vector<int2> tiles((size_t)g.ntp);
-    ctpwa_gram_tables(ncol, pp.data(), &g.npp, tiles.data());
-    g.nwg = ctpwa_gram_nwg(g.npp);
+    std::vector<int> tpair((size_t)g.ntp);
+    ctpwa_gram_tables(ncol, tiles.data(), nullptr, &g.npp, tpair.data());
+    std::vector<GramPair> pp;
+    long long part = gram_plan(ncol, device_cus(h->device), &pp, &g.nwg);
+    if (nwg > 0) {
+        g.nwg = nwg;
+        part = (long long)nwg * g.ntp * 256;
+    }
     g.pp = h->upload(pp);
     g.tiles = h->upload(tiles);
-    g.part = h->alloc<double>((size_t)g.nwg * g.ntp * 256);
+    g.tpair = h->upload(tpair);
+    g.part = h->alloc<double>((size_t)part);
+}
+
+static void gramws_setup(ctpwa_handle* h, GramWS& w, bool amps_only, const long long n3[3]) {
+    const Model_& M = h->M;
+    w.S = hess_shape(M, amps_only);
+    const GramSizes z = gram_sizes(M, w.S, n3, device_cus(h->device));
+    std::vector<int> perm;
+    w.mod = compile_eval(h->device, generate_hess_kernel(M, &perm, amps_only));
+    HIPCHECK(hipModuleGetFunction(&w.fn, w.mod, amps_only ? "ctpwa_amp_gram" : w.S.fused ? "ctpwa_hess_fused" : "ctpwa_hess_rows"));
+    if ((int)perm.size() != z.nz) throw std::runtime_error("Hessian: summed-column count mismatch");
+    w.perm = h->upload(perm);
+    w.nz = z.nz;
+    w.target = z.target;
+    w.chunk = z.chunk;
+    w.cap = z.cap;
+    w.ldJ = z.ldJ;
+    w.ldc = z.ldc;
+    w.z = h->alloc<double>((size_t)z.z);
+    if (!w.S.fused) {
+        w.J = h->alloc<unsigned char>((size_t)z.J * (w.S.f32 ? sizeof(float) : sizeof(double)));
+        w.U = h->alloc<double>((size_t)z.U);
+        // the amplitude Gram weights every row by one
+        w.W = amps_only ? h->upload(std::vector<double>((size_t)z.W, 1.0)) : h->alloc<double>((size_t)z.W);
+    }
+    gram_setup(h, w.gJ, 2 * w.S.C, w.S.fused ? z.target : 0);
+    if (w.S.NU > 0) gram_setup(h, w.gU, w.S.NU, w.S.fused ? z.target : 0);
+    w.ready = true;
+}
+
+// shares out `target` workgroups among k pieces of the given costs, at least one each, at
+// most `target` in all (target >= k)
+static std::vector<int> share_out(const std::vector<double>& cost, int target) {
+    double all = 0.0;
+    for (double c : cost) all += c;
+    std::vector<int> n(cost.size(), 1);
+    const int spare = target - (int)cost.size();
+    for (size_t k = 0; k < cost.size(); ++k) n[k] += (int)(spare * (all > 0 ? cost[k] / all : 0.0));
+    return n;
+}
+
+// Runs a GramWS over the classes with use[c]: passes of up to four pieces (a piece: up to
+// `chunk` events of one class), each the per-event kernel, in the rows form the Gram kernels
+// over its rows, and the sums, which go to T
+static void gramws_run(ctpwa_handle* h, GramWS& w, const bool use[3], HessTotals T, const double* cfr, int withK, hipStream_t s) {
+    const Model_& M = h->M;
+    const int NP = M.P.npol;
+    struct Piece { int c; long long s0, cnt; };
+    std::vector<Piece> todo;
+    for (int c = 0; c < 3; ++c)
+        for (long long s0 = 0; use[c] && s0 < h->n[c]; s0 += w.chunk) todo.push_back({c, s0, std::min(w.chunk, h->n[c] - s0)});
+    bool seen[3] = {false, false, false};
+    for (size_t at = 0; at < todo.size();) {
+        HessPieces H{}, HU{};
+        long long ev = 0, row = 0, wr = 0;
+        while (at < todo.size() && H.n < 4 && (H.n == 0 || ev + todo[at].cnt <= w.cap)) {
+            const Piece& p = todo[at];
+            const int k = H.n;
+            // (a class may have one piece per pass: its sums then have one writer)
+            if (k > 0 && H.cls[k - 1] == p.c) break;
+            H.cls[k] = p.c;
+            H.e0[k] = h->off[p.c] + p.s0;
+            H.cnt[k] = p.cnt;
+            H.row0[k] = row;
+            H.w0[k] = wr;
+            ev += p.cnt;
+            row += up(NP * p.cnt, 32);          // every piece's rows start 16-byte aligned
+            wr += up(p.cnt, 64);           // (a last wave's idle lanes write there)
+            ++H.n;
+            ++at;
+        }
+        if (!w.S.fused && (row > w.ldJ || wr > w.ldc)) throw std::runtime_error("Hessian: a pass exceeds its buffers");
+        // data and background events also have a u row (and in the fused form its Gram)
+        std::vector<double> ce, cr, cu;
+        for (int k = 0; k < H.n; ++k) {
+            ce.push_back((double)H.cnt[k] * (H.cls[k] != 0 ? 1.2 : 1.0));
+            cr.push_back((double)H.cnt[k]);
+        }
+        const std::vector<int> we = share_out(ce, w.target);
+        const std::vector<int> gs = w.S.fused ? we : share_out(cr, w.gJ.nwg);
+        int g0 = 0;
+        for (int k = 0; k < H.n; ++k) {
+            const long long steps = (H.cnt[k] + 63) / 64;
+            H.spw[k] = (int)((steps + we[k] - 1) / we[k]);
+            H.wg0[k + 1] = H.wg0[k] + (int)((steps + H.spw[k] - 1) / H.spw[k]);
+            if (w.S.fused) {
+                H.glo[k] = H.wg0[k];
+                H.ghi[k] = H.wg0[k + 1];
+            } else {
+                H.glo[k] = g0;
+                g0 += gs[k];
+                H.ghi[k] = g0;
+            }
+        }
+        for (int k = 0; k < H.n && w.S.NU > 0; ++k) {
+            if (H.cls[k] == 0) continue;
+            const int q = HU.n++;
+            HU.cls[q] = H.cls[k];
+            HU.cnt[q] = H.cnt[k];
+            HU.row0[q] = HU.w0[q] = H.w0[k];
+            HU.glo[q] = H.glo[k];
+            HU.ghi[q] = H.ghi[k];
+            cu.push_back((double)H.cnt[k]);
+        }
+        if (!w.S.fused && HU.n > 0) {
+            const std::vector<int> us = share_out(cu, w.gU.nwg);
+            for (int q = 0, u0 = 0; q < HU.n; ++q) {
+                HU.glo[q] = u0;
+                u0 += us[q];
+                HU.ghi[q] = u0;
+            }
+        }
+        int nwg = H.wg0[H.n];
+        if (nwg > w.target) throw std::runtime_error("Hessian: more workgroups than partials");
+        double* gp = w.gJ.part;
+        double* upart = w.gU.part;
+        void* args[] = {&h->table, (void*)&h->slp, &h->inv, &h->invf, &h->ntot, &h->wts, &h->wc[1], &h->wc[2], &h->pw[1], &h->pw[2],
+                        &H, &w.J, &w.ldJ, &w.U, &w.W, &w.ldc, &gp, &upart, &w.z, &nwg, (void*)&cfr, &h->ntot, &withK};
+        HIPCHECK(hipModuleLaunchKernel(w.fn, nwg, 1, 1, 64 * w.S.G, 1, 1, 0, s, args, nullptr));
+        for (int c = 0; c < 3; ++c) T.first[c] = !seen[c];
+        for (int k = 0; k < H.n; ++k) seen[H.cls[k]] = true;
+        // Grams of up to 64 columns: one launch for all pieces, summed with the columns below;
+        // wider ones: a launch and its sums per piece
+        const bool jw = !w.S.fused && w.gJ.ncol > 64, uw = !w.S.fused && w.gU.ncol > 64;
+        const size_t es = w.S.f32 ? sizeof(float) : sizeof(double);
+        if (jw) {
+            for (int k = 0; k < H.n; ++k)
+                HIPCHECK(ctpwa_launch_gram_wide((const char*)w.J + (size_t)H.row0[k] * es, w.S.f32, w.gJ.ncol, w.ldJ, NP * H.cnt[k],
+                                                H.cnt[k], w.W + H.w0[k], w.gJ.pp, w.gJ.npp, w.gJ.tiles, w.gJ.tpair, w.gJ.ntp,
+                                                w.gJ.nwg, w.gJ.part, T.G[H.cls[k]], T.first[H.cls[k]], s));
+        } else if (!w.S.fused) {
+            HIPCHECK(ctpwa_launch_gram_panels(w.J, w.S.f32, w.gJ.ncol, w.ldJ, &H, NP, w.W, w.gJ.part, s));
+        }
+        if (uw) {
+            for (int q = 0; q < HU.n; ++q)
+                HIPCHECK(ctpwa_launch_gram_wide(w.U + HU.row0[q], 0, w.gU.ncol, w.ldc, HU.cnt[q], HU.cnt[q], w.W + w.ldc + HU.w0[q],
+                                                w.gU.pp, w.gU.npp, w.gU.tiles, w.gU.tpair, w.gU.ntp, w.gU.nwg, w.gU.part,
+                                                T.Uu[HU.cls[q]], T.first[HU.cls[q]], s));
+        } else if (!w.S.fused && HU.n > 0) {
+            HIPCHECK(ctpwa_launch_gram_panels(w.U, 0, w.gU.ncol, w.ldc, &HU, 1, w.W + w.ldc, w.gU.part, s));
+        }
+        if (jw && w.nz == 0 && (uw || w.S.NU == 0)) continue;
+        HIPCHECK(ctpwa_launch_hess_accum(&H, &HU, &T, w.gJ.part, jw ? 0 : w.gJ.ntp, w.gJ.tiles, w.gJ.ncol, w.gU.part,
+                                         uw || w.S.NU == 0 ? 0 : w.gU.ntp, w.gU.tiles, w.S.NU, w.z, w.nz, nwg, w.perm, s));
+    }
 }
 
 static void hess_setup(ctpwa_handle* h) {
     const Model_& M = h->M;
     const Plan& P = M.P;
-    const HessDims hd = hess_dims(M);
-    h->hC = hd.C;
-    h->hNU = hd.NU;
-    h->hNZ = hd.NZ;
-    h->hnG = 2 * hd.C * (2 * hd.C + 1) / 2;
-    h->hnUu = hd.NU * (hd.NU + 1) / 2;
     if (P.ntheta > 64) throw std::runtime_error("Hessian: more than 64 free resonance parameters is not built");
-    long long ch[2];
-    hess_chunks(M, h->n, g_live_handles.load() - 1, ch);
-    const size_t es = M.mixed ? sizeof(float) : sizeof(double);
-    for (int k = 0; k < 2; ++k) {
-        HessWS& ws = h->hws[k];
-        ws.chunk = ch[k];
-        if (ch[k] == 0) continue;
-        ws.J = h->alloc<unsigned char>((size_t)ch[k] * P.npol * 2 * h->hC * es);
-        ws.U = h->alloc<double>((size_t)ch[k] * h->hNU);
-        ws.cs_ld = ctpwa_hess_rows_waves(ch[k]);
-        ws.cs = h->alloc<double>((size_t)(h->hNZ + h->hNU) * ws.cs_ld);
-        ws.W = h->alloc<double>((size_t)ch[k] * 2);
-        gram_setup(h, ws.gJ, 2 * h->hC);
-        gram_setup(h, ws.gU, h->hNU);
-    }
-    if (ch[1] > 0) {
-        HIPCHECK(hipStreamCreateWithFlags(&h->hs2, hipStreamNonBlocking));
-        for (hipEvent_t& ev : h->hev) HIPCHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    }
+    gramws_setup(h, h->hess, false, h->n);
+    const HessShape& S = h->hess.S;
+    h->hNZ = hess_nz(M);
+    h->hnG = 2 * S.C * (2 * S.C + 1) / 2;
+    h->hnUu = S.NU * (S.NU + 1) / 2;
+    h->hess.ready = false;              // until the tables below exist
     // totals: per class G, Uu, Z, g
-    h->htot = h->alloc<double>((size_t)3 * (h->hnG + h->hnUu + h->hNZ + h->hNU));
-    h->hHext = h->alloc<double>((size_t)h->hNU * h->hNU);
+    h->htot = h->alloc<double>((size_t)3 * (h->hnG + h->hnUu + h->hNZ + S.NU));
+    // second-part sums: per block its (amplitude, local parameter) pairs of reals, then its
+    // upper triangle of parameter pairs
+    {
+        const int n = P.namp, T = P.ntheta;
+        std::vector<int> zvt((size_t)n * T, -1), ttp(1, 0), ttl;
+        std::vector<std::vector<int>> tt((size_t)T * T);
+        int z = 0;
+        for (size_t b = 0; b < P.blocks.size(); ++b) {
+            if (P.blocks[b].nsl == 0) continue;
+            const std::vector<int>& v = M.bvars[b];
+            const int nl = (int)v.size();
+            for (int a = P.blocks[b].site; a < P.blocks[b].site + P.blocks[b].nsl; ++a)
+                for (int i = 0; i < nl; ++i, z += 2) zvt[(size_t)a * T + v[i]] = z;
+            for (int i = 0; i < nl; ++i)
+                for (int k = i; k < nl; ++k, ++z) {
+                    tt[(size_t)v[i] * T + v[k]].push_back(z);
+                    if (v[i] != v[k]) tt[(size_t)v[k] * T + v[i]].push_back(z);
+                }
+        }
+        if (z != h->hNZ - 1) throw std::runtime_error("Hessian: second-part sum count mismatch");
+        for (const std::vector<int>& l : tt) {
+            ttl.insert(ttl.end(), l.begin(), l.end());
+            ttp.push_back((int)ttl.size());
+        }
+        h->hzvt = h->upload(zvt);
+        h->http = h->upload(ttp);
+        h->httl = h->upload(ttl);
+    }
     // fit parameter -> extended entries: [Re p_f] -> Re v_a, [Im p_f] -> Im v_a with
     // v_a = r_a p_f(a); theta_j -> theta_j
     {
@@ -1231,60 +1402,30 @@ static void hess_setup(ctpwa_handle* h) {
         h->hmap_x = h->upload(xs);
         h->hmap_r = h->upload(rs);
     }
-    std::vector<int> perm;
-    h->hmod = compile_eval(h->device, generate_hess_kernel(M, &perm));
-    if ((int)perm.size() != h->hNZ + h->hNU) throw std::runtime_error("Hessian: summed-column count mismatch");
-    h->hperm = h->upload(perm);
-    HIPCHECK(hipModuleGetFunction(&h->fn_hrows, h->hmod, "ctpwa_hess_rows"));
     if (!M.customs.empty()) {
         h->mod2 = compile_eval(h->device, generate_custom2_kernel(M));
         HIPCHECK(hipModuleGetFunction(&h->fn_custom2, h->mod2, "ctpwa_custom2"));
         h->cfb2 = h->alloc<double>((size_t)M.customs.size() * M.ncf2() * h->ntot);
     }
-    h->hess_ready = true;
-}
-
-// amplitude Gram of one class: Q[l][k] = sum_e sum_p conj(A_l) A_k (amplitudes without
-// couplings), the integrals behind fit fractions and the interference matrix
-// events per chunk of amplitude rows: at most 2^18, and rows of at most 256 MiB
-static long long agram_chunk(const Plan& P, long long maxn) {
-    const long long per_event = (long long)P.npol * 2 * P.namp * 8;
-    const long long cap = std::max<long long>(4, (256LL << 20) / per_event);
-    return (std::max<long long>(1, std::min<long long>(maxn, std::min<long long>(cap, 1 << 18))) + 3) / 4 * 4;
-}
-static long long agram_workspace_bytes(const Plan& P, long long maxn) {
-    const long long n2 = 2 * P.namp, ch = agram_chunk(P, maxn);
-    return ch * P.npol * n2 * 8 + ch * 8 + n2 * (n2 + 1) / 2 * 8 + gram_part_doubles((int)n2) * 8;
-}
-static void agram_setup(ctpwa_handle* h) {
-    const Plan& P = h->M.P;
-    const int n2 = 2 * P.namp;
-    long long maxn = std::max(h->n[0], std::max(h->n[1], h->n[2]));
-    h->gchunk = agram_chunk(P, maxn);
-    h->gX = h->alloc<double>((size_t)h->gchunk * P.npol * n2);
-    h->gW = h->upload(std::vector<double>((size_t)h->gchunk, 1.0));
-    h->gtot = h->alloc<double>((size_t)n2 * (n2 + 1) / 2);
-    gram_setup(h, h->gg, n2);
-    h->agram_ready = true;
+    h->hess.ready = true;
 }
 
 // Gram of class cls's amplitude rows at the parameter point the table holds, to out
 // [namp][namp][2]: with the theta coefficients K_a (withK = 1) or without them (0)
 static void class_gram(ctpwa_handle* h, int cls, int withK, double* out, hipStream_t s) {
-    if (!h->agram_ready) agram_setup(h);
     const Plan& P = h->M.P;
-    const int n2 = 2 * P.namp;
-    const long long ldx = h->gchunk * P.npol;
-    HIPCHECK(ctpwa_launch_zero(h->gtot, (long long)n2 * (n2 + 1) / 2, s));
-    const GramTabs& G = h->gg;
-    int k = 0;
-    for (long long s0 = 0; s0 < h->n[cls]; s0 += h->gchunk, ++k) {
-        long long cnt = std::min(h->gchunk, h->n[cls] - s0);
-        HIPCHECK(ctpwa_launch_amp_rows(&h->aux, h->off[cls] + s0, cnt, h->gX, ldx, withK, s));
-        HIPCHECK(ctpwa_launch_gram_panels(h->gX, 0, n2, ldx, cnt * P.npol, h->gW, cnt, G.pp, G.npp, G.ntp, G.part,
-                                          G.nwg, k > 0, s));
+    if (!h->agram.ready) {
+        // one class per call: buffers for the largest
+        const long long n3[3] = {std::max(h->n[0], std::max(h->n[1], h->n[2])), 0, 0};
+        h->gtot = h->alloc<double>((size_t)P.namp * (2 * P.namp + 1));
+        gramws_setup(h, h->agram, true, n3);
     }
-    if (h->n[cls] > 0) HIPCHECK(ctpwa_launch_accum_panels(G.part, G.nwg, G.ntp, G.tiles, n2, h->gtot, s));
+    bool use[3] = {false, false, false};
+    use[cls] = true;
+    HessTotals T{};
+    for (int c = 0; c < 3; ++c) T.G[c] = h->gtot;
+    if (h->n[cls] > 0) gramws_run(h, h->agram, use, T, h->cfb, withK, s);
+    else HIPCHECK(ctpwa_launch_zero(h->gtot, (long long)P.namp * (2 * P.namp + 1), s));
     HIPCHECK(ctpwa_launch_gram_to_complex(h->gtot, P.namp, out, s));
 }
 
@@ -1376,78 +1517,37 @@ extern "C" int ctpwa_hessian(ctpwa_handle* h, const double* params_dev, double* 
     DeviceGuard g(h->device);
     hipStream_t s = (hipStream_t)stream;
     try {
-        if (!h->hess_ready) hess_setup(h);
+        if (!h->hess.ready) hess_setup(h);
         const Model_& M = h->M;
         const Plan& P = M.P;
+        const HessShape& S = h->hess.S;
         HIPCHECK(ctpwa_launch_prep(params_dev, h->table, &h->prep, M.maxloc, 3, s));
         if (h->fn_custom2) {
             void* args[] = {&h->table, &h->inv, &h->invf, &h->ntot, &h->cfb2};
             unsigned grid = (unsigned)std::min<long long>(16384, (h->ntot + 63) / 64);
             HIPCHECK(hipModuleLaunchKernel(h->fn_custom2, grid, 1, 1, 64, 1, 1, 0, s, args, nullptr));
         }
-        size_t per_class = (size_t)h->hnG + h->hnUu + h->hNZ + h->hNU;
-        HIPCHECK(ctpwa_launch_zero(h->htot, (long long)(3 * per_class), s));
+        const size_t per_class = (size_t)h->hnG + h->hnUu + h->hNZ + S.NU;
         HessAsm as{};
-        const int f32 = M.mixed;
-        // data and background run on the handle's second stream with buffer set 1, after
-        // the coefficient table and the zeroed totals on the caller's stream
-        const int forced = hess_streams_env();
-        const bool two = h->hs2 != nullptr && (h->n[1] > 0 || h->n[2] > 0) &&
-                         (forced == 2 || (forced == 0 && g_live_handles.load() == 1));
-        if (two) {
-            HIPCHECK(hipEventRecord(h->hev[0], s));
-            HIPCHECK(hipStreamWaitEvent(h->hs2, h->hev[0], 0));
-        }
+        HessTotals T{};
+        bool use[3];
         for (int c = 0; c < 3; ++c) {
             double* base = h->htot + c * per_class;
-            as.G[c] = base;
-            as.Uu[c] = base + h->hnG;
-            as.Zs[c] = base + h->hnG + h->hnUu;
-            as.gs[c] = base + h->hnG + h->hnUu + h->hNZ;
-            HessWS& ws = h->hws[c == 0 || !two ? 0 : 1];
-            hipStream_t sc = (c == 0 || !two) ? s : h->hs2;
-            const long long ldJ = ws.chunk * P.npol;
-            const double* wts = (c > 0 && h->pw[c]) ? h->wts : nullptr;
-            double wconst = h->wc[c];
-            int cls = c;
-            int k = 0;
-            for (long long s0 = 0; s0 < h->n[c]; s0 += ws.chunk, ++k) {
-                long long cnt = std::min(ws.chunk, h->n[c] - s0);
-                long long e0 = h->off[c] + s0;
-                // per-event rows of the chunk (generated kernel)
-                void* args[] = {&h->table, (void*)&h->slp, &h->inv, &h->invf, &h->ntot, (void*)&wts, &wconst, &cls, &e0,
-                                &cnt, &ws.J, (void*)&ldJ, &ws.chunk, &ws.U, &ws.W, &ws.cs, &ws.cs_ld, &h->cfb2,
-                                &h->ntot};
-                const unsigned grid = (unsigned)((cnt + 255) / 256);
-                HIPCHECK(hipModuleLaunchKernel(h->fn_hrows, grid, 1, 1, 256, 1, 1, 0, sc, args, nullptr));
-                // weighted Grams on the matrix cores, summed over the class's chunks
-                HIPCHECK(ctpwa_launch_gram_panels(ws.J, f32, 2 * h->hC, ldJ, cnt * P.npol, ws.W, cnt, ws.gJ.pp,
-                                                  ws.gJ.npp, ws.gJ.ntp, ws.gJ.part, ws.gJ.nwg, k > 0, sc));
-                if (c > 0)
-                    HIPCHECK(ctpwa_launch_gram_panels(ws.U, 0, h->hNU, ws.chunk, cnt, ws.W + ws.chunk, cnt, ws.gU.pp,
-                                                      ws.gU.npp, ws.gU.ntp, ws.gU.part, ws.gU.nwg, k > 0, sc));
-                // Zs[c] and gs[c] are adjacent: one pass adds both from the rows kernel's sums
-                HIPCHECK(ctpwa_launch_accum_cols(ws.cs, ws.cs_ld, cnt, h->hNZ + h->hNU, h->hperm, (double*)as.Zs[c], sc));
-            }
-            if (h->n[c] > 0) {
-                HIPCHECK(ctpwa_launch_accum_panels(ws.gJ.part, ws.gJ.nwg, ws.gJ.ntp, ws.gJ.tiles, 2 * h->hC,
-                                                   (double*)as.G[c], sc));
-                if (c > 0)
-                    HIPCHECK(ctpwa_launch_accum_panels(ws.gU.part, ws.gU.nwg, ws.gU.ntp, ws.gU.tiles, h->hNU,
-                                                       (double*)as.Uu[c], sc));
-            }
+            as.G[c] = T.G[c] = base;
+            as.Uu[c] = T.Uu[c] = base + h->hnG;
+            as.Zs[c] = T.Z[c] = base + h->hnG + h->hnUu;
+            as.gs[c] = base + h->hnG + h->hnUu + h->hNZ;        // the u sums follow Z
+            use[c] = h->n[c] > 0;
+            as.live[c] = use[c];
         }
-        if (two) {
-            HIPCHECK(hipEventRecord(h->hev[1], h->hs2));
-            HIPCHECK(hipStreamWaitEvent(s, h->hev[1], 0));
-        }
-        as.C = h->hC; as.NU = h->hNU; as.NZ = h->hNZ;
-        as.namp = P.namp; as.nfree = P.nfree; as.ntheta = P.ntheta; as.nblock = (int)P.blocks.size();
-        as.amps = h->aux.amps; as.blocks = h->aux.blocks; as.table = h->table; as.off_v = (long long)M.off_v();
+        gramws_run(h, h->hess, use, T, h->cfb2, 1, s);
+        as.C = S.C; as.NU = S.NU; as.NZ = h->hNZ;
+        as.namp = P.namp; as.nfree = P.nfree; as.ntheta = P.ntheta;
+        as.zvt = h->hzvt; as.ttp = h->http; as.ttl = h->httl;
         as.Np = (double)h->n[0]; as.Wd = h->Wd; as.Wb = h->Wb;
         as.ngauss = (int)P.g_slot.size(); as.g_slot = h->fin.g_slot; as.g_sig = h->fin.g_sig;
         as.map_ptr = h->hmap_ptr; as.map_x = h->hmap_x; as.map_r = h->hmap_r;
-        as.Hext = h->hHext; as.out = hess_dev;
+        as.out = hess_dev;
         HIPCHECK(ctpwa_launch_hess_assemble(&as, s));
         return 0;
     } catch (const std::exception& e) {
@@ -1774,8 +1874,7 @@ extern "C" long long ctpwa_footprint_bytes(const char* plan_text, long long n_ph
         b += nt * (long long)M.customs.size() * M.ncf() * 8;     // Custom factor rows
         // no free resonance parameter: the stored phase-space Gram and its build workspace
         if (M.P.ntheta == 0)
-            b += (long long)M.P.namp * M.P.namp * 16 +
-                 agram_workspace_bytes(M.P, std::max(n_phsp, std::max(n_data, n_bkg)));
+            b += (long long)M.P.namp * M.P.namp * 16 + agram_workspace_bytes(M, std::max(n_phsp, std::max(n_data, n_bkg)));
         // (the upload staging is one pool per device for the process, not per handle)
         return b;
     } catch (const std::exception& e) {
@@ -1789,8 +1888,7 @@ extern "C" long long ctpwa_hessian_workspace_bytes(const char* plan_text, long l
     try {
         Model_ M = derive(parse_plan(plan_text));
         const long long n3[3] = {n_phsp, n_data, n_bkg};
-        // the handle these buffers are for does not exist yet: every live handle is another
-        return hess_workspace_bytes(M, n3, n_phsp + n_data + n_bkg, g_live_handles.load());
+        return hess_workspace_bytes(M, n3, n_phsp + n_data + n_bkg);
     } catch (const std::exception& e) {
         g_err = std::string("ctpwa_hessian_workspace_bytes: ") + e.what();
         return -1;
@@ -1844,7 +1942,7 @@ extern "C" long long ctpwa_generate_hessian_source(const char* plan_text, int pr
         if (precision != 0 && precision != 1) throw std::runtime_error("precision must be 0 (FP64) or 1 (mixed)");
         Model_ M = derive(parse_plan(plan_text));
         M.mixed = precision;
-        std::string src = generate_hess_kernel(M, nullptr);
+        std::string src = generate_hess_kernel(M, nullptr, false);
         // models with Custom lineshapes: the second-order factor module follows
         if (!M.customs.empty()) src += "\n// ---- module: ctpwa_custom2 ----\n" + generate_custom2_kernel(M);
         if (buf && cap > 0) {
@@ -1883,7 +1981,7 @@ extern "C" long long ctpwa_compile_check(const char* plan_text, int precision) {
             return (long long)cs;
         };
         long long cs = compile(generate_eval_kernel(M));
-        cs += compile(generate_hess_kernel(M, nullptr));
+        cs += compile(generate_hess_kernel(M, nullptr, false));
         // models with Custom lineshapes: also the Hessian's second-order factor module
         if (!M.customs.empty()) cs += compile(generate_custom2_kernel(M));
         return cs;

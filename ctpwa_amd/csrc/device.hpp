@@ -187,30 +187,56 @@ struct AuxArgs {
     const int* bcl;
 };
 
+// One pass of the Hessian's (or amplitude Gram's) per-event kernel: up to four pieces, each a
+// range of one class's events.  Mirrored in the generated source (codegen_hess.cpp).
+struct HessPieces {
+    int n;
+    int cls[4];
+    int wg0[5];              // workgroups [wg0[k], wg0[k + 1]) of the per-event kernel
+    int spw[4];              // 64-event steps per workgroup
+    long long e0[4], cnt[4]; // stored events [e0, e0 + cnt)
+    long long row0[4];       // first Jacobian row (npol cnt rows, row p cnt + r)
+    long long w0[4];         // first entry in the weights and u rows
+    int glo[4], ghi[4];      // the Gram partials [glo, ghi) of the piece
+};
+// one panel pair (P <= Q, 128 columns each) of a Gram of more than 64 columns: its tile pairs
+// [tile0, tile0 + nt), the tile pairs of a wave, its workgroups [s0, s0 + ns) and the offset of
+// their partials (in tiles)
+struct GramPair { int P, Q, tile0, nt, nq, s0, ns; long long off; };
+// where a pass adds its sums: packed Gram, packed u Gram and summed columns per class; first:
+// the class's first pass, which sets instead of adding
+struct HessTotals {
+    double* G[3];
+    double* Uu[3];
+    double* Z[3];
+    int first[3];
+};
+
 // Hessian assembly from the per-class sums
 struct HessAsm {
     // per class c: G[c] (upper-triangle list over 2C), Uu[c] (upper triangle over NU),
-    // Z[c] (NZ), g[c] (NU)
+    // Z[c] (NZ), g[c] (NU); live[c] 0: the class has no events (its sums are not read)
     const double* G[3];
     const double* Uu[3];
     const double* Zs[3];
     const double* gs[3];
+    int live[3];
     int C, NU, NZ;
-    int namp, nfree, ntheta, nblock;
-    const DAmp* amps;
-    const DBlock* blocks;
-    const double* table;
-    long long off_v;
+    int namp, nfree, ntheta;
     double Np, Wd, Wb;
     int ngauss;
     const int* g_slot;
     const double* g_sig;
+    // second-part sums: zvt[a ntheta + j] the index in Z of <S, dA_a/dtheta_j> (real part,
+    // then imaginary), or -1; ttl[ttp[j ntheta + k] ..) the indices of the pair's terms
+    const int* zvt;
+    const int* ttp;
+    const int* ttl;
     // fit parameter q = (Re p_f, Im p_f, theta) -> extended entries map_x[map_ptr[q] ..
     // map_ptr[q + 1]) with factors map_r (v_a = r_a p_f(a))
     const int* map_ptr;
     const int* map_x;
     const double* map_r;
-    double* Hext;            // [NU][NU] scratch
     double* out;             // [np][np]
 };
 

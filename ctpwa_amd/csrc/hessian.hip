@@ -31,24 +31,24 @@ namespace ctpwa {
 
 
 
-// Weighted Gram of a column-major matrix X[col][row] (column stride ldx, rows
-// [0, nrows)) on the matrix cores, for any number of columns:
+// Weighted Gram of a column-major matrix X[column][row] (column stride ldx) on the matrix
+// cores:
 //   G[a][b] = sum_rows w(row) X[a][row] X[b][row],  w(row) = Wt[row mod nev]
-// (rows p * nev + r share event r's weight).  Columns are grouped in panels of 64 (four
-// 16-column tiles); workgroup (x, y) takes panel pair y = (P, Q), P <= Q, and share x of
-// the rows.  Each of its four waves owns a contiguous range of the share, stages R-row
-// slabs of the pair's columns in its own LDS region (register prefetch of the next slab,
-// column stride padded by one element against bank conflicts) and accumulates the pair's
-// 16x16 tile products (I <= J on a diagonal pair) in registers with
-// v_mfma_f64_16x16x4 (T = double) or v_mfma_f32_16x16x4 (T = float: the mixed form's
-// FP32 Jacobian, products summed in FP32 over one slab, then added into FP64
-// accumulators).  The waves combine their tiles through LDS in wave order and the
-// workgroup writes (or, for a later chunk of rows, adds) one partial per tile pair;
-// k_accum_panels sums the partials in a fixed order.
+// (rows p * nev + r share event r's weight).  The rows of a pass's pieces lie one after the
+// other; share x of the workgroups belongs to one piece, so that one launch serves every event
+// class.  (Rows in blocks of 32, each block's columns together, do not speed this kernel or
+// k_gram_wide up, and the FP32 writer's stores take 25 % longer.)  This kernel takes up to 64
+// columns (four 16-column tiles); k_gram_wide takes more.  Each of a workgroup's four waves
+// owns a contiguous range of the share, stages R-row slabs of the columns in its own LDS
+// region (register prefetch of the next slab, column stride padded by one element against
+// bank conflicts) and accumulates the 16x16 tile products I <= J in registers with
+// v_mfma_f64_16x16x4 (T = double) or v_mfma_f32_16x16x4 (T = float: the mixed form's FP32
+// Jacobian, products summed in FP32 over one slab, then added into FP64 accumulators).  The
+// waves combine their tiles through LDS in wave order and the workgroup writes one partial
+// per tile pair; k_hess_accum sums the partials in a fixed order.
 // Lane layouts (16x16x4, one block): A[i][k] in lane 16 k + i, B[k][j] in lane 16 k + j;
 // D[4 r + q][j] (f64) or D[4 q + r][j] (f32) in component r of lane 16 q + j.
 constexpr int GP_WAVES = 4;
-constexpr int GP_PAIRS = 16;                 // tile pairs of two different panels
 template <typename T> struct GP;
 template <> struct GP<double> {
     static constexpr int R = 16;
@@ -62,44 +62,39 @@ template <> struct GP<float> {
 };
 typedef double gp_acc64 __attribute__((ext_vector_type(4)));
 
-// LDS bytes of k_gram_panels<T, NT, FULL>: per wave a slab of the pair's columns, or the
-// combined tile pairs
-inline size_t gram_panels_lds(bool f32, int NT, bool full) {
+// LDS bytes of k_gram_panels<T, NT>: per wave a slab of the columns, or the combined tile pairs
+inline size_t gram_panels_lds(bool f32, int NT) {
     const int R = f32 ? 32 : 16;
     const size_t es = f32 ? 4 : 8;
-    const int cols = full ? 128 : NT * 16;
-    const int npair = full ? NT * NT : NT * (NT + 1) / 2;
-    size_t slabs = (size_t)GP_WAVES * cols * (R + 1) * es;
+    const int npair = NT * (NT + 1) / 2;
+    size_t slabs = (size_t)GP_WAVES * NT * 16 * (R + 1) * es;
     size_t comb = (size_t)npair * 256 * sizeof(double);
     return std::max(slabs, comb);
 }
 
-// NT: tiles per panel; FULL: all NT x NT tile pairs of the panel pair (a Gram of several
-// panels: a diagonal pair then also computes its tiles below the diagonal, which the
-// accumulation skips), else the NT (NT + 1) / 2 pairs I <= J (a Gram of one panel).  With
-// the pair count fixed at compile time every pair's product is unconditional.
-template <typename T, int NT, bool FULL>
+// NT: tiles of the columns; the NT (NT + 1) / 2 tile pairs I <= J.  With the pair count fixed
+// at compile time every pair's product is unconditional.
+template <typename T, int NT>
 __global__ void __launch_bounds__(64 * GP_WAVES)
-k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows, const double* __restrict__ Wt,
-              long long nev, const int4* __restrict__ pp, int ntp, double* __restrict__ part, int accumulate) {
+k_gram_panels(const T* __restrict__ X0, int ncol, long long ldx, HessPieces H, int rpe, const double* __restrict__ Wt0,
+              double* __restrict__ part) {
     constexpr int R = GP<T>::R, ST = R + 1;
-    constexpr int NPAIR = FULL ? NT * NT : NT * (NT + 1) / 2;
+    constexpr int NPAIR = NT * (NT + 1) / 2;
     typedef typename GP<T>::acc_t acc_t;
     extern __shared__ __attribute__((aligned(16))) unsigned char gp_smem[];
     __shared__ double wsh[GP_WAVES][R];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int4 pq = pp[blockIdx.y];                 // panels P, Q; first tile pair; tile pairs
-    const int P = pq.x, Q = pq.y, tp0 = pq.z;
-    const bool diag = P == Q;
-    const int wP = min(64, ncol - 64 * P), wQ = min(64, ncol - 64 * Q);
-    const int ncl = diag ? 64 : 128;
-    constexpr int NCOLS = FULL ? 128 : NT * 16;
+    constexpr int NCOLS = NT * 16;
     T* xs = (T*)gp_smem + (size_t)wave * NCOLS * ST;
     double* ws = wsh[wave];
-    const int boff0 = diag ? 0 : 64;
-    // this wave's rows: the grid's waves split [0, nrows) into ranges of whole slabs
-    const long long nw = (long long)gridDim.x * GP_WAVES;
-    const long long gw = (long long)blockIdx.x * GP_WAVES + wave;
+    int pk = 0;
+    while (pk + 1 < H.n && (int)blockIdx.x >= H.ghi[pk]) ++pk;
+    const long long nev = H.cnt[pk], nrows = nev * rpe;      // rpe rows per event
+    const T* X = X0 + H.row0[pk];
+    const double* Wt = Wt0 + H.w0[pk];
+    // this wave's rows: the piece's waves split [0, nrows) into ranges of whole slabs
+    const long long nw = (long long)(H.ghi[pk] - H.glo[pk]) * GP_WAVES;
+    const long long gw = (long long)((int)blockIdx.x - H.glo[pk]) * GP_WAVES + wave;
     const long long per = ((nrows + nw - 1) / nw + R - 1) / R * R;
     const long long r0 = gw * per < nrows ? gw * per : nrows;
     const long long r1 = r0 + per < nrows ? r0 + per : nrows;
@@ -107,9 +102,9 @@ k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows,
 #pragma unroll
     for (int q = 0; q < NPAIR; ++q) acc[q] = (gp_acc64){0.0, 0.0, 0.0, 0.0};
     // 16-byte loads: lane l carries rows VW (l mod LPC) .. + VW - 1 of column CPI it + l / LPC
-    // (the chunk's leading dimension is a multiple of 4, so every such run is aligned)
+    // (pieces start at multiples of 4 rows and ldx is one, so every such run is aligned)
     constexpr int VW = 16 / (int)sizeof(T), LPC_ = R / VW, CPI = 64 / LPC_;
-    constexpr int NLD = (FULL ? 128 : NT * 16) / CPI;
+    constexpr int NLD = NCOLS / CPI;
     typedef T vec_t __attribute__((ext_vector_type(VW)));
     const int rr0 = (lane % LPC_) * VW, ch = lane / LPC_;
     const int rw = lane % R;
@@ -117,17 +112,14 @@ k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows,
     // the base of the next slab to load advances by R with subtractions (no 64-bit division
     // per slab)
     long long eload = r0 < r1 ? r0 % nev : 0;
-    auto gcol = [&](int c) -> int {           // global column of LDS column c, or -1
-        if (c < 64) return c < wP ? 64 * P + c : -1;
-        return (c - 64) < wQ ? 64 * Q + (c - 64) : -1;
-    };
     auto load = [&](vec_t (&pre)[NLD], double& wpre, long long t0) {
         const int nt = (int)((r1 - t0) < R ? (r1 - t0) : R);
+        const T* Xb = X + t0 + rr0;
 #pragma unroll
         for (int it = 0; it < NLD; ++it) {
             const int c = CPI * it + ch;
-            const int g = c < ncl ? gcol(c) : -1;
-            const T* src = X + (long long)(g < 0 ? 0 : g) * ldx + t0 + rr0;
+            const int g = c < ncol ? c : -1;
+            const T* src = Xb + (long long)(g < 0 ? 0 : g) * ldx;
             if (g >= 0 && rr0 + VW <= nt) {
                 pre[it] = *(const vec_t*)src;
             } else {
@@ -147,10 +139,8 @@ k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows,
 #pragma unroll
         for (int it = 0; it < NLD; ++it) {
             const int c = CPI * it + ch;
-            if (c < ncl) {
 #pragma unroll
-                for (int v = 0; v < VW; ++v) xs[c * ST + rr0 + v] = pre[it][v];
-            }
+            for (int v = 0; v < VW; ++v) xs[c * ST + rr0 + v] = pre[it][v];
         }
         if (lane < R) ws[rw] = wpre;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -168,8 +158,8 @@ k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows,
                 for (int I = 0; I < NT; ++I) {
                     const double av = w * (double)xs[(I * 16 + li) * ST + kr];
 #pragma unroll
-                    for (int J = FULL ? 0 : I; J < NT; ++J, ++q)
-                        acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, (double)xs[(boff0 + J * 16 + li) * ST + kr], acc[q],
+                    for (int J = I; J < NT; ++J, ++q)
+                        acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, (double)xs[(J * 16 + li) * ST + kr], acc[q],
                                                                       0, 0, 0);
                 }
             }
@@ -186,8 +176,8 @@ k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows,
                 for (int I = 0; I < NT; ++I) {
                     const float av = w * xs[(I * 16 + li) * ST + kr];
 #pragma unroll
-                    for (int J = FULL ? 0 : I; J < NT; ++J, ++q)
-                        t[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, (float)xs[(boff0 + J * 16 + li) * ST + kr], t[q], 0, 0, 0);
+                    for (int J = I; J < NT; ++J, ++q)
+                        t[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, (float)xs[(J * 16 + li) * ST + kr], t[q], 0, 0, 0);
                 }
             }
 #pragma unroll
@@ -226,61 +216,267 @@ k_gram_panels(const T* __restrict__ X, int ncol, long long ldx, long long nrows,
         }
         __syncthreads();
     }
-    double* o = part + ((size_t)blockIdx.x * ntp + tp0) * 256;
-    for (int e = threadIdx.x; e < NPAIR * 256; e += 64 * GP_WAVES) o[e] = accumulate ? o[e] + comb[e] : comb[e];
+    double* o = part + (size_t)blockIdx.x * NPAIR * 256;
+    for (int e = threadIdx.x; e < NPAIR * 256; e += 64 * GP_WAVES) o[e] = comb[e];
 }
 
-// tot[idx(a, b)] += the sum over the nwg workgroup partials of k_gram_panels, for every
-// entry a <= b < ncol of the Gram (packed upper triangle, row-major).  tiles[q] = (I, J):
-// the 16-column tiles of tile pair q.  Each workgroup takes 64 consecutive tile elements
-// (one per lane, coalesced reads); its four waves add the partials g = w, w + 4, ...
-// with eight interleaved sums combined by a fixed tree, and wave 0 adds the waves' sums
-// in wave order: a fixed order throughout.
-__global__ void __launch_bounds__(256) k_accum_panels(const double* __restrict__ part, int nwg, int ntp,
-                                                      const int2* __restrict__ tiles, int ncol, double* __restrict__ tot) {
-    __shared__ double sh[4][64];
+// The same Gram for more than 64 columns, one piece per launch.  Panels of 128 columns (eight
+// tiles); a workgroup of eight waves takes a panel pair and a share of the rows and stages
+// slabs of R rows of the pair's 256 columns in LDS (two buffers, one barrier per slab, the next
+// slab's loads in flight during the products).  Wave i holds the tile pairs of row i: all of an
+// off-diagonal panel pair's (A read and weighted once per step), (i, i + q mod T) for
+// q <= T / 2 on the diagonal, so every wave of a workgroup has the same work and the shares
+// are dealt out by it.  Bound by the matrix cores (64 cycles per FP64 product); every column
+// is read 3.3 times for 346 columns.  No register may spill: a reload between the loads waits
+// for all of them (7.3 instead of 3.5 ms for 1.2M rows of 346 and
+// 100k rows of 322 columns).  Panels of 64 columns read every column 7.8 times
+// and computed full tile squares on the diagonal (7.5 ms).
+// LDS column strides: 16 columns x 2 rows (FP64) or x 4 rows (FP32) of a read lie in different
+// banks, and 16-byte stores stay aligned.
+constexpr int GW_WAVES = 8;
+template <typename T> struct GWS { static constexpr int ST = sizeof(T) == 8 ? 18 : 36; };
+template <typename T>
+inline size_t gram_wide_lds() { return (size_t)2 * 256 * GWS<T>::ST * sizeof(T); }
+
+template <typename T, int NQ, bool DIAG>
+__device__ __forceinline__ void gram_wide_rows(const T* __restrict__ X, int ncol, long long ldx, const GramPair& G, long long r0,
+                                               long long r1, int nev, const double* __restrict__ Wt, T* xs, double (*wsh)[GP<T>::R],
+                                               double* __restrict__ o) {
+    constexpr int R = GP<T>::R, ST = GWS<T>::ST;
+    typedef typename GP<T>::acc_t acc_t;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int li = lane & 15, lk = lane >> 4;
+    const int TQ = (min(128, ncol - 128 * G.Q) + 15) / 16, I = DIAG ? min(wave, TQ - 1) : wave;
+    gp_acc64 acc[NQ];
+    const int tl = li * ST + lk;
+    int tb[NQ];                                   // first element of the B tiles
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        acc[q] = (gp_acc64){0.0, 0.0, 0.0, 0.0};
+        tb[q] = (DIAG ? (I + q) % TQ : 8 + q) * 16 * ST;
+    }
+    // 16-byte loads, eight lanes to a column's slab: loads 0, 1 take panel P, loads 2, 3 panel Q
+    // (a diagonal pair stages its panel once).  A column past the last takes the last one: its
+    // products are not used.  Rows past the last lie in the matrix's padding and are set to 0.
+    constexpr int VW = 16 / (int)sizeof(T), CPI = 64;
+    static_assert(R / VW == 8, "eight lanes per column");
+    typedef T vec_t __attribute__((ext_vector_type(VW)));
+    const int rr0 = (threadIdx.x % 8) * VW, ch = threadIdx.x / 8;
+    // row r0 + R k + thread's event (rows that wrap to the next polarisation start again)
+    int ev = (int)((r0 + (int)threadIdx.x % R) % nev);
+    const int evstep = R % nev;
+    constexpr int NL = DIAG ? 2 : 4;
+    vec_t pre[NL];
+    double wpre = 0.0;
+    const T* Xr = X + r0;
+    auto load = [&]() {
+        // the column's address is formed anew for each load, from a column index the optimiser
+        // cannot see through: four addresses kept across the loop spill
+        int c0 = ch;
+        asm volatile("" : "+v"(c0));
+        if ((int)threadIdx.x < R) {
+            wpre = Wt[ev];
+            ev += evstep;
+            if (ev >= nev) ev -= nev;
+        }
+#pragma unroll
+        for (int it = 0; it < NL; ++it)
+            pre[it] = *(const vec_t*)(Xr + (long long)min(ncol - 1, 128 * (it < 2 ? G.P : G.Q) + CPI * (it & 1) + c0) * ldx + rr0);
+        Xr += R;
+    };
+    auto store = [&](int b, long long t0) {
+        T* xb = xs + b * 256 * ST + ch * ST + rr0;
+        if (t0 + R > r1) {
+            const int nt = (int)(r1 - t0);
+#pragma unroll
+            for (int it = 0; it < NL; ++it)
+#pragma unroll
+                for (int v = 0; v < VW; ++v) pre[it][v] = rr0 + v < nt ? pre[it][v] : (T)0;
+            wpre = (int)threadIdx.x < nt ? wpre : 0.0;
+        }
+        if ((int)threadIdx.x < R) wsh[b][threadIdx.x] = wpre;
+#pragma unroll
+        for (int it = 0; it < NL; ++it) *(vec_t*)(xb + CPI * it * ST) = pre[it];
+    };
+    if (r0 < r1) {
+        load();
+        store(0, r0);
+    }
+    __syncthreads();
+    int b = 0;
+    for (long long t0 = r0; t0 < r1; t0 += R, b ^= 1) {
+        const bool more = t0 + R < r1;
+        if (more) load();
+        const T* xb = xs + b * 256 * ST + tl;
+        const T* xa = xb + I * 16 * ST;
+        const double* ws = wsh[b] + lk;
+        if constexpr (sizeof(T) == 8) {
+#pragma unroll
+            for (int k0 = 0; k0 < R; k0 += 4) {
+                const double av = ws[k0] * xa[k0];
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, xb[tb[q] + k0], acc[q], 0, 0, 0);
+            }
+        } else {
+            // a slab's products are summed in FP32, then added into the FP64 sums
+            float av[R / 4];
+#pragma unroll
+            for (int k = 0; k < R / 4; ++k) av[k] = (float)ws[4 * k] * xa[4 * k];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                acc_t t = (acc_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < R / 4; ++k) t = __builtin_amdgcn_mfma_f32_16x16x4f32(av[k], xb[tb[q] + 4 * k], t, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[q][r] += (double)t[r];
+            }
+        }
+        if (more) store(b ^ 1, t0 + R);
+        __syncthreads();             // the slab is consumed and the next one is in place
+    }
+    // the tile pairs in the order of the tile list; a wrapped diagonal pair (J < I) is the
+    // transpose of (J, I), and (I, I + T / 2) comes twice for an even T
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int J = DIAG ? (I + q) % TQ : q;
+        const int i = DIAG ? min(I, J) : I, j = DIAG ? max(I, J) : J;
+        if (DIAG && (wave >= TQ || (2 * q == TQ && wave >= q))) continue;
+        double* oq = o + (DIAG ? i * TQ - i * (i - 1) / 2 + (j - i) : i * TQ + j) * 256;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int a = GP<T>::row(lane, r);
+            oq[DIAG && J < I ? li * 16 + a : a * 16 + li] = acc[q][r];
+        }
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64 * GW_WAVES, 4)
+k_gram_wide(const T* __restrict__ X, int ncol, long long ldx, long long nrows, int nev, const double* __restrict__ Wt,
+            const GramPair* __restrict__ pairs, int npair, double* __restrict__ part) {
+    constexpr int R = GP<T>::R;
+    extern __shared__ __attribute__((aligned(16))) unsigned char gp_smem[];
+    __shared__ double wsh[2][R];
+    int y = 0;
+    while (y + 1 < npair && (int)blockIdx.x >= pairs[y + 1].s0) ++y;
+    const GramPair G = pairs[y];
+    const int share = (int)blockIdx.x - G.s0;
+    const long long slabs = (nrows + R - 1) / R;
+    const long long per = (slabs + G.ns - 1) / G.ns;
+    const long long r0 = min(nrows, share * per * R), r1 = min(nrows, r0 + per * R);
+    // tile pair q of the panel pair at part[(off + share nt + q) 256]
+    double* o = part + (G.off + (long long)share * G.nt) * 256;
+#define GW_ROWS(NQ, D) gram_wide_rows<T, NQ, D>(X, ncol, ldx, G, r0, r1, nev, Wt, (T*)gp_smem, wsh, o); break
+    switch (G.P == G.Q ? G.nq : 8 + G.nq) {
+    case 1: GW_ROWS(1, true);
+    case 2: GW_ROWS(2, true);
+    case 3: GW_ROWS(3, true);
+    case 4: GW_ROWS(4, true);
+    case 5: GW_ROWS(5, true);
+    case 9: GW_ROWS(1, false);
+    case 10: GW_ROWS(2, false);
+    case 11: GW_ROWS(3, false);
+    case 12: GW_ROWS(4, false);
+    case 13: GW_ROWS(5, false);
+    case 14: GW_ROWS(6, false);
+    case 15: GW_ROWS(7, false);
+    case 16: GW_ROWS(8, false);
+#undef GW_ROWS
+    }
+}
+
+// tot (packed upper triangle) = or += the Gram from k_gram_wide's partials: 64 elements of one
+// tile pair per workgroup, tpair its panel pair; sixteen waves as in k_hess_accum
+constexpr int HA_WAVES = 16;
+__global__ void __launch_bounds__(64 * HA_WAVES)
+k_accum_wide(const double* __restrict__ part, const GramPair* __restrict__ pairs, const int2* __restrict__ tiles,
+             const int* __restrict__ tpair, int ncol, double* __restrict__ tot, int first) {
+    __shared__ double sh[HA_WAVES][64];
+    const int tq = blockIdx.x >> 2, e = (blockIdx.x & 3) * 64 + (threadIdx.x & 63), wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const GramPair G = pairs[tpair[tq]];
+    const double* p = part + (G.off + (tq - G.tile0)) * 256 + e;
+    double s = 0.0, s1 = 0.0;
+    int g = wave;
+    for (; g + HA_WAVES < G.ns; g += 2 * HA_WAVES) {
+        s += p[(size_t)g * G.nt * 256];
+        s1 += p[(size_t)(g + HA_WAVES) * G.nt * 256];
+    }
+    if (g < G.ns) s += p[(size_t)g * G.nt * 256];
+    sh[wave][lane] = s + s1;
+    __syncthreads();
+    if (wave == 0) {
+        double v = sh[0][lane];
+        for (int w = 1; w < HA_WAVES; ++w) v += sh[w][lane];
+        const int2 t = tiles[tq];
+        const int a = t.x * 16 + (e >> 4), b = t.y * 16 + (e & 15);
+        if (a < ncol && b < ncol && a <= b) {
+            double* o = tot + ((long long)a * ncol - (long long)a * (a - 1) / 2 + (b - a));
+            *o = first ? v : *o + v;
+        }
+    }
+}
+
+// The sums of a pass, one launch: blockIdx.y is the piece; the first nG workgroups along x
+// add the Gram partials of 64 tile elements each (tiles[q] = (I, J): the 16-column tiles of
+// tile pair q; result in the packed upper triangle, row-major), the next nU those of the u
+// Gram (pieces of HU), the rest the summed columns, one per wave (zpart[c * nwg + w], result
+// at Z[perm[c]]).  Sixteen waves per workgroup add every sixteenth partial in four
+// interleaved sums, joined in a fixed order: with four waves the 40-column Gram's 1000
+// partials were a chain of 30 dependent loads (18 us per class).
+__device__ inline void accum_tiles(const double* __restrict__ part, int lo, int hi, int ntp, const int2* __restrict__ tiles,
+                                   int ncol, double* __restrict__ tot, bool first, int blk, double (*sh)[64]) {
     const long long E = (long long)ntp * 256;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long long e = (long long)blockIdx.x * 64 + lane;
-    double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    if (e < E) {
-        int g = wave;
-        for (; g + 28 < nwg; g += 32) {
+    const long long e = (long long)blk * 64 + lane;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    int g = lo + wave;
+    for (; g + 3 * HA_WAVES < hi; g += 4 * HA_WAVES) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) s[k] += part[(size_t)(g + 4 * k) * E + e];
-        }
-        for (; g < nwg; g += 4) s[0] += part[(size_t)g * E + e];
+        for (int k = 0; k < 4; ++k) s[k] += part[(size_t)(g + k * HA_WAVES) * E + e];
     }
-    sh[wave][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    for (; g < hi; g += HA_WAVES) s[0] += part[(size_t)g * E + e];
+    sh[wave][lane] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
-    if (wave == 0 && e < E) {
-        const double v = ((sh[0][lane] + sh[1][lane]) + sh[2][lane]) + sh[3][lane];
+    if (wave == 0) {
+        double v = sh[0][lane];
+        for (int w = 1; w < HA_WAVES; ++w) v += sh[w][lane];
         const int2 t = tiles[e >> 8];
         const int a = t.x * 16 + (int)((e >> 4) & 15), b = t.y * 16 + (int)(e & 15);
-        if (a < ncol && b < ncol && a <= b) tot[(long long)a * ncol - (long long)a * (a - 1) / 2 + (b - a)] += v;
+        if (a < ncol && b < ncol && a <= b) {
+            double* o = tot + ((long long)a * ncol - (long long)a * (a - 1) / 2 + (b - a));
+            *o = first ? v : *o + v;
+        }
     }
 }
-
-// tot[c] += the sum over the nw wave sums of column c (cs[c * ld + w]) left by
-// k_hess_rows: one workgroup per column; each thread adds its strided share in two
-// interleaved sums, the waves combine by exchanges and thread 0 adds the four waves in
-// order: a fixed order
-__global__ void __launch_bounds__(256) k_accum_cols(const double* __restrict__ cs, long long ld, int nw,
-                                                    const int* __restrict__ perm, double* __restrict__ tot) {
-    __shared__ double sh[4];
-    const double* p = cs + (long long)blockIdx.x * ld;
-    double s0 = 0.0, s1 = 0.0;
-    int w = threadIdx.x;
-    for (; w + 256 < nw; w += 512) {
-        s0 += p[w];
-        s1 += p[w + 256];
+__global__ void __launch_bounds__(64 * HA_WAVES)
+k_hess_accum(HessPieces H, HessPieces HU, HessTotals T, const double* __restrict__ gpart, int ntp, const int2* __restrict__ tiles,
+             int ncol, const double* __restrict__ upart, int utp, const int2* __restrict__ utiles, int ucol,
+             const double* __restrict__ zpart, int nz, int nwg, const int* __restrict__ perm) {
+    __shared__ double sh[HA_WAVES][64];
+    const int nG = ntp * 4, nU = utp * 4, k = blockIdx.y;
+    int blk = blockIdx.x;
+    if (blk < nG) {
+        if (k >= H.n) return;
+        accum_tiles(gpart, H.glo[k], H.ghi[k], ntp, tiles, ncol, T.G[H.cls[k]], T.first[H.cls[k]], blk, sh);
+        return;
     }
-    if (w < nw) s0 += p[w];
-    double s = s0 + s1;
+    blk -= nG;
+    if (blk < nU) {
+        if (k >= HU.n) return;
+        accum_tiles(upart, HU.glo[k], HU.ghi[k], utp, utiles, ucol, T.Uu[HU.cls[k]], T.first[HU.cls[k]], blk, sh);
+        return;
+    }
+    blk -= nU;
+    const int c = blk * HA_WAVES + (threadIdx.x >> 6);
+    if (k >= H.n || c >= nz) return;
+    const double* p = zpart + (long long)c * nwg;
+    double s = 0.0;
+    for (int w = H.wg0[k] + (threadIdx.x & 63); w < H.wg0[k + 1]; w += 64) s += p[w];
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) tot[perm ? perm[blockIdx.x] : (int)blockIdx.x] += (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    if ((threadIdx.x & 63) == 0) {
+        double* o = T.Z[H.cls[k]] + perm[c];
+        *o = T.first[H.cls[k]] ? s : *o + s;
+    }
 }
 
 __device__ inline double gram_at(const double* G, int n2, int k, int l) {
@@ -327,13 +523,15 @@ __global__ void k_gram_to_complex(const double* __restrict__ G, int n, double* _
     Q[2 * q + 1] = gram_at(G, n2, l, n + k) - gram_at(G, n2, n + l, k);
 }
 
-// Hessian assembly, three kernels:
-//  k_hess_ext     Hext[x][y] over the extended parameters (Re v, Im v, theta) from the
-//                 class Grams, the u Grams and the phase-space normalisation terms,
-//                 H = -H_data + H_bkg + N_eff [A2 / (N_p pf) - g g^T / (N_p pf)^2];
-//  k_hess_second  adds the second-part terms of the (v, theta) and (theta, theta) blocks
-//                 and the Gaussian constraints (one thread, a fixed order);
-//  k_hess_map     maps to the fit parameters [Re p, Im p, theta] (v_a = r_a p_f(a)).
+// Hessian assembly in one launch: entry (r, c) of the fit-parameter Hessian
+// [Re p, Im p, theta] is the sum over the extended parameters (Re v, Im v, theta) that r and
+// c stand for (v_a = r_a p_f(a)) of
+//   H = -H_data + H_bkg + N_eff [A2 / (N_p pf) - g g^T / (N_p pf)^2] + diag(1 / sigma^2),
+// each class's part from its Gram, its u Gram and its second-part sums (zvt: the sum of
+// <S, dA_a/dtheta_j>; ttp/ttl: the sums of Re(v d2F conj(T)) of a parameter pair over the
+// blocks, in block order).  Every entry is one thread's, with no intermediate matrix.  As
+// separate kernels the second-part terms of 149 amplitudes were one workgroup's serial
+// work (137 us), and the three kernels of a 10-amplitude Hessian took 33 us.
 __device__ inline void hess_pf(const HessAsm& h, double& cp, double& cq) {
     double Np = h.Np, Neff = h.Wd - h.Wb;
     double pf = (Np > 0) ? h.Zs[0][h.NZ - 1] / Np : 0.0;
@@ -342,103 +540,46 @@ __device__ inline void hess_pf(const HessAsm& h, double& cp, double& cq) {
     cq = (Np > 0) ? -Neff / (Np * pf * Np * pf) : 0.0;
 }
 
-__global__ void __launch_bounds__(256) k_hess_ext(HessAsm h) {
-    const int NU = h.NU;
-    double cp, cq;
-    hess_pf(h, cp, cq);
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (long long)NU * NU) return;
-    const int x = (int)(q / NU), y = (int)(q - (long long)x * NU);
+__device__ inline double hess_ext(const HessAsm& h, double cp, double cq, int x, int y) {
+    const int n = h.namp, P = h.ntheta;
+    const bool tx = x >= 2 * n, ty = y >= 2 * n;
+    const double sc[3] = {cp, -1.0, 1.0};
     double H = 0.0;
     for (int c = 0; c < 3; ++c) {
+        if (!h.live[c]) continue;
         double v = d2I_sum(h, c, x, y);
-        if (c != 0) v += gram_at(h.Uu[c], NU, x, y);
-        if (c == 0) H += cp * v + cq * h.gs[0][x] * h.gs[0][y];
-        else H += (c == 1 ? -1.0 : 1.0) * v;
+        if (c != 0) v += gram_at(h.Uu[c], h.NU, x, y);
+        // d2S/dRe v_a dtheta = dA_a/dtheta: 2 Re <S, dA>; d2S/dIm v_a dtheta = i dA: -2 Im <S, dA>
+        if (tx != ty) {
+            const int p = tx ? y : x, j = (tx ? x : y) - 2 * n;
+            const int a = p < n ? p : p - n;
+            const int z = h.zvt[a * P + j];
+            if (z >= 0) v += p < n ? 2.0 * h.Zs[c][z] : -2.0 * h.Zs[c][z + 1];
+        } else if (tx) {
+            const int q = (x - 2 * n) * P + (y - 2 * n);
+            for (int k = h.ttp[q]; k < h.ttp[q + 1]; ++k) v += 2.0 * h.Zs[c][h.ttl[k]];
+        }
+        H += sc[c] * v;
+        if (c == 0) H += cq * h.gs[0][x] * h.gs[0][y];
     }
-    h.Hext[q] = H;
+    if (tx && x == y)
+        for (int g = 0; g < h.ngauss; ++g)
+            if (h.g_slot[g] == x - 2 * n) H += 1.0 / (h.g_sig[g] * h.g_sig[g]);
+    return H;
 }
 
-// z offset of block b in the class sums: the blocks before it with waves
-__device__ inline int hess_zoff(const HessAsm& h, int b) {
-    int z = 0;
-    for (int q = 0; q < b; ++q) {
-        const DBlock& B = h.blocks[q];
-        if (B.nsl > 0) z += B.nsl * 2 * B.nloc + B.nloc * (B.nloc + 1) / 2;
-    }
-    return z;
-}
-
-// second-part terms: every (amplitude, local parameter) entry of the (v, theta) blocks
-// belongs to one thread (the classes added in a fixed order); the (theta, theta) terms
-// of all blocks, which may share parameters, and the Gaussian constraints are gathered
-// in LDS by one thread in block order and then added in parallel
-constexpr int HS_MAXTH = 64;
-__global__ void __launch_bounds__(256) k_hess_second(HessAsm h) {
-    __shared__ double tt[HS_MAXTH * HS_MAXTH];
-    const int n = h.namp, NU = h.NU, P = h.ntheta;
-    double cp, cq;
-    hess_pf(h, cp, cq);
-    const double sc[3] = {cp, -1.0, 1.0};
-    for (int a = threadIdx.x; a < n; a += blockDim.x) {
-        const int b = h.amps[a].block;
-        const DBlock& B = h.blocks[b];
-        if (B.nsl == 0) continue;
-        const int z0 = hess_zoff(h, b) + (a - B.site) * 2 * B.nloc;
-        for (int i = 0; i < B.nloc; ++i) {
-            double re = 0.0, im = 0.0;
-            for (int c = 0; c < 3; ++c) {
-                // d2S/dRe v_a dtheta = dA_a/dtheta: 2 Re Q ; d2S/dIm v_a dtheta = i dA: -2 Im Q
-                re += 2.0 * sc[c] * h.Zs[c][z0 + 2 * i];
-                im += -2.0 * sc[c] * h.Zs[c][z0 + 2 * i + 1];
-            }
-            const int j = 2 * n + B.vars[i];
-            h.Hext[(long long)a * NU + j] += re;
-            h.Hext[(long long)j * NU + a] += re;
-            h.Hext[(long long)(n + a) * NU + j] += im;
-            h.Hext[(long long)j * NU + n + a] += im;
-        }
-    }
-    if (P > HS_MAXTH) return;     // rejected on the host
-    for (int q = threadIdx.x; q < P * P; q += blockDim.x) tt[q] = 0.0;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < 3; ++c) {
-            int zq = 0;
-            for (int b = 0; b < h.nblock; ++b) {
-                const DBlock& B = h.blocks[b];
-                if (B.nsl == 0) continue;
-                zq += B.nsl * 2 * B.nloc;
-                for (int i = 0; i < B.nloc; ++i)
-                    for (int k = i; k < B.nloc; ++k) {
-                        const double rv = 2.0 * sc[c] * h.Zs[c][zq++];
-                        const int j1 = B.vars[i], j2 = B.vars[k];
-                        tt[j1 * P + j2] += rv;
-                        if (j1 != j2) tt[j2 * P + j1] += rv;
-                    }
-            }
-        }
-        for (int g = 0; g < h.ngauss; ++g) {
-            const int j = h.g_slot[g];
-            tt[j * P + j] += 1.0 / (h.g_sig[g] * h.g_sig[g]);
-        }
-    }
-    __syncthreads();
-    for (int q = threadIdx.x; q < P * P; q += blockDim.x) {
-        const int j1 = q / P, j2 = q - j1 * P;
-        h.Hext[(long long)(2 * n + j1) * NU + 2 * n + j2] += tt[q];
-    }
-}
-
-__global__ void __launch_bounds__(256) k_hess_map(HessAsm h) {
-    const int np = 2 * h.nfree + h.ntheta, NU = h.NU;
+__global__ void __launch_bounds__(256) k_hess_out(HessAsm h) {
+    const int np = 2 * h.nfree + h.ntheta;
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (long long)np * np) return;
-    const int r = (int)(q / np), c = (int)(q - (long long)r * np);
+    double cp, cq;
+    hess_pf(h, cp, cq);
+    // the elements (r, c) and (c, r) are the same sum: the matrix is exactly symmetric
+    const int qr = (int)(q / np), qc = (int)(q - (long long)qr * np), r = min(qr, qc), c = max(qr, qc);
     double H = 0.0;
     for (int u = h.map_ptr[r]; u < h.map_ptr[r + 1]; ++u)
         for (int w = h.map_ptr[c]; w < h.map_ptr[c + 1]; ++w)
-            H += h.map_r[u] * h.map_r[w] * h.Hext[(long long)h.map_x[u] * NU + h.map_x[w]];
+            H += h.map_r[u] * h.map_r[w] * hess_ext(h, cp, cq, h.map_x[u], h.map_x[w]);
     h.out[q] = H;
 }
 
@@ -459,101 +600,91 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_zero(do
     return hipGetLastError();
 }
 
-// panel pairs (P, Q, first tile pair, tile pairs) and the tile-pair list (I, J) of the
-// matrix-core Gram of ncol columns; returns the number of tile pairs
-extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_tables(int ncol, int4* pp, int* npp, int2* tiles) {
-    const int npan = (ncol + 63) / 64;
-    const int T1 = (ncol + 15) / 16;        // tiles of a one-panel Gram
+// Tile pairs (I, J) of the Gram of ncol columns, returned count; more than 64 columns: also
+// the panel pairs (their workgroups and partials set by the caller) and each tile pair's panel
+// pair
+extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_tables(int ncol, int2* tiles, GramPair* pairs, int* npair,
+                                                                      int* tpair) {
+    const int T = (ncol + 15) / 16;
+    const bool wide = ncol > 64;
+    const int np = wide ? (T + 7) / 8 : 1;
     int q = 0, y = 0;
-    for (int P = 0; P < npan; ++P)
-        for (int Q = P; Q < npan; ++Q) {
-            const int q0 = q;
-            // one panel: the pairs I <= J of its tiles; several: all 4 x 4 pairs of a panel
-            // pair (tiles past the last column give entries the accumulation skips)
-            for (int I = 0; I < 4; ++I)
-                for (int J = 0; J < 4; ++J) {
-                    const bool use = (npan == 1) ? (I < T1 && J < T1 && I <= J) : true;
-                    if (!use) continue;
-                    if (tiles) tiles[q] = make_int2(4 * P + I, 4 * Q + J);
-                    ++q;
+    for (int P = 0; P < np; ++P)
+        for (int Q = P; Q < np; ++Q, ++y) {
+            const int i1 = wide ? std::min(T, 8 * P + 8) : T, j1 = wide ? std::min(T, 8 * Q + 8) : T, q0 = q;
+            for (int I = 8 * P; I < i1; ++I)
+                for (int J = P == Q ? I : 8 * Q; J < j1; ++J, ++q) {
+                    if (tiles) tiles[q] = make_int2(I, J);
+                    if (tpair) tpair[q] = y;
                 }
-            if (pp) pp[y] = make_int4(P, Q, q0, q - q0);
-            ++y;
+            if (pairs) pairs[y] = GramPair{P, Q, q0, q - q0, P == Q ? (j1 - 8 * P) / 2 + 1 : j1 - 8 * Q, 0, 0, 0};
         }
-    if (npp) *npp = y;
+    if (npair) *npair = y;
     return q;
 }
 
-// workgroups along the rows for a Gram of npp panel pairs (about 2048 in all)
-extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_nwg(int npp) {
-    // environment CTPWA_GRAM_WGS overrides the per-launch workgroup budget (measurements)
-    static const int budget = [] {
+// workgroups of a Gram of up to 64 columns (environment CTPWA_GRAM_WGS overrides it for
+// measurements)
+extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_nwg() {
+    static const int n = [] {
         const char* e = std::getenv("CTPWA_GRAM_WGS");
-        return e ? std::max(32, std::atoi(e)) : 2048;
+        return e ? std::max(32, std::atoi(e) / 4) : 512;
     }();
-    const int cap = std::max(512, budget / 4);
-    return std::max(32, std::min(cap, budget / std::max(1, npp)));
+    return n;
 }
 
-// weighted Gram on the matrix cores: partials [nwg][ntp][256] written (accumulate = 0)
-// or added (accumulate = 1) in part; FP64 input, or FP32 input (f32 = 1)
-extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_gram_panels(const void* X, int f32, int ncol,
-                                                                                     long long ldx, long long nrows,
-                                                                                     const double* Wt, long long nev,
-                                                                                     const int4* pp, int npp, int ntp,
-                                                                                     double* part, int nwg, int accumulate,
+// weighted Gram on the matrix cores of the pieces' rows (rpe rows per event), up to 64 columns:
+// partials [ghi of the last piece][tile pairs][256]; FP64 input, or FP32 input (f32 = 1)
+extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_gram_panels(const void* X, int f32, int ncol, long long ldx, const HessPieces* H,
+                                                                                     int rpe, const double* Wt, double* part,
                                                                                      hipStream_t s) {
-    if (ncol <= 0 || nrows <= 0) return hipSuccess;
-    const dim3 g(nwg, npp), b(64 * GP_WAVES);
-#define GP_LAUNCH(TT, NTT, FF)                                                                                   \
-    hipLaunchKernelGGL((k_gram_panels<TT, NTT, FF>), g, b, gram_panels_lds(f32 != 0, NTT, FF), s, (const TT*)X, ncol, \
-                       ldx, nrows, Wt, nev, pp, ntp, part, accumulate)
-    const int T1 = (ncol + 15) / 16;
-    if (ncol > 64) {
-        if (f32) GP_LAUNCH(float, 4, true); else GP_LAUNCH(double, 4, true);
-    } else if (f32) {
-        switch (T1) {
-        case 1: GP_LAUNCH(float, 1, false); break;
-        case 2: GP_LAUNCH(float, 2, false); break;
-        case 3: GP_LAUNCH(float, 3, false); break;
-        default: GP_LAUNCH(float, 4, false); break;
-        }
-    } else {
-        switch (T1) {
-        case 1: GP_LAUNCH(double, 1, false); break;
-        case 2: GP_LAUNCH(double, 2, false); break;
-        case 3: GP_LAUNCH(double, 3, false); break;
-        default: GP_LAUNCH(double, 4, false); break;
-        }
+    if (ncol <= 0 || H->n <= 0) return hipSuccess;
+    if (ncol > 64) return hipErrorInvalidValue;
+    const dim3 g(H->ghi[H->n - 1]), b(64 * GP_WAVES);
+#define GP_LAUNCH(TT, NTT)                                                                                            \
+    hipLaunchKernelGGL((k_gram_panels<TT, NTT>), g, b, gram_panels_lds(f32 != 0, NTT), s, (const TT*)X, ncol, ldx, *H, rpe, \
+                       Wt, part)
+    switch ((ncol + 15) / 16 + (f32 ? 4 : 0)) {
+    case 1: GP_LAUNCH(double, 1); break;
+    case 2: GP_LAUNCH(double, 2); break;
+    case 3: GP_LAUNCH(double, 3); break;
+    case 4: GP_LAUNCH(double, 4); break;
+    case 5: GP_LAUNCH(float, 1); break;
+    case 6: GP_LAUNCH(float, 2); break;
+    case 7: GP_LAUNCH(float, 3); break;
+    default: GP_LAUNCH(float, 4); break;
     }
 #undef GP_LAUNCH
     return hipGetLastError();
 }
 
-// tot += the Gram from the partials of k_gram_panels (packed upper triangle)
-extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_accum_panels(const double* part, int nwg, int ntp,
-                                                                                      const int2* tiles, int ncol,
-                                                                                      double* tot, hipStream_t s) {
-    const long long E = (long long)ntp * 256;
-    hipLaunchKernelGGL(k_accum_panels, dim3((unsigned)((E + 63) / 64)), dim3(256), 0, s, part, nwg, ntp, tiles, ncol, tot);
+// more than 64 columns, one piece: rows X[col ldx + row], nwg workgroups as set in pairs, then
+// the sums into tot (first: set, else add)
+extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_gram_wide(const void* X, int f32, int ncol, long long ldx, long long nrows, long long nev, const double* Wt,
+                                                                                   const GramPair* pairs, int npair, const int2* tiles,
+                                                                                   const int* tpair, int ntp, int nwg, double* part,
+                                                                                   double* tot, int first, hipStream_t s) {
+    const dim3 g(nwg), b(64 * GW_WAVES);
+    if (f32)
+        hipLaunchKernelGGL(k_gram_wide<float>, g, b, gram_wide_lds<float>(), s, (const float*)X, ncol, ldx, nrows, (int)nev, Wt, pairs,
+                           npair, part);
+    else
+        hipLaunchKernelGGL(k_gram_wide<double>, g, b, gram_wide_lds<double>(), s, (const double*)X, ncol, ldx, nrows, (int)nev, Wt, pairs,
+                           npair, part);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_accum_wide, dim3(4 * ntp), dim3(64 * HA_WAVES), 0, s, part, pairs, tiles, tpair, ncol, tot, first);
     return hipGetLastError();
 }
 
-// waves of the Hessian rows kernel (256 threads per workgroup) over n events: the row
-// count of its column-sum partials
-extern "C" __attribute__((visibility("hidden"))) long long ctpwa_hess_rows_waves(long long n) {
-    return (n + 255) / 256 * 4;
-}
-
-// tot[perm[c]] += the column sums left by the rows kernel over n events, for its ncol
-// summed columns (perm: the rows kernel's put order -> the assembly's order)
-extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_accum_cols(const double* cs, long long ld,
-                                                                                    long long n, int ncol, const int* perm,
-                                                                                    double* tot, hipStream_t s) {
-    const long long nw = ctpwa_hess_rows_waves(n);
-    if (ncol <= 0 || nw <= 0) return hipSuccess;
-    if (nw > ld) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_accum_cols, dim3(ncol), dim3(256), 0, s, cs, ld, (int)nw, perm, tot);
+// a pass's sums (k_hess_accum)
+extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_hess_accum(
+    const HessPieces* H, const HessPieces* HU, const HessTotals* T, const double* gpart, int ntp, const int2* tiles, int ncol,
+    const double* upart, int utp, const int2* utiles, int ucol, const double* zpart, int nz, int nwg, const int* perm,
+    hipStream_t s) {
+    const unsigned nx = (unsigned)(4 * ntp + 4 * utp + (nz + HA_WAVES - 1) / HA_WAVES);
+    hipLaunchKernelGGL(k_hess_accum, dim3(nx, (unsigned)std::max(H->n, HU->n)), dim3(64 * HA_WAVES), 0, s, *H, *HU, *T, gpart,
+                       ntp, tiles, ncol, upart, utp, utiles, ucol, zpart, nz, nwg, perm);
     return hipGetLastError();
 }
 
@@ -564,12 +695,8 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_gram_to
 }
 
 extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_hess_assemble(const HessAsm* h, hipStream_t s) {
-    const long long ne = (long long)h->NU * h->NU;
-    hipLaunchKernelGGL(k_hess_ext, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s, *h);
-    if (h->ntheta > HS_MAXTH) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_hess_second, dim3(1), dim3(256), 0, s, *h);
     const int np = 2 * h->nfree + h->ntheta;
     const long long nm = (long long)np * np;
-    hipLaunchKernelGGL(k_hess_map, dim3((unsigned)((nm + 255) / 256)), dim3(256), 0, s, *h);
+    hipLaunchKernelGGL(k_hess_out, dim3((unsigned)((nm + 255) / 256)), dim3(256), 0, s, *h);
     return hipGetLastError();
 }

@@ -653,4 +653,18 @@ inline Model_ derive(const Plan& P) {
     return M;
 }
 
+// Shape of the generated Hessian (or amplitude Gram) kernel: wave groups and their blocks,
+// Gram columns 2 C and u columns NU, Jacobian type, whether the Gram is fused into it (else
+// it writes Jacobian rows), LDS layout in doubles (S exchange, parameter slots, column-sum
+// slabs of SW columns per wave; the fused form's tile takes the place of all of them)
+struct HessShape {
+    int G = 1, C = 0, NU = 0, SW = 16, nslot = 0;
+    bool fused = false, f32 = false;
+    std::vector<std::vector<int>> blocks;                    // per group
+    std::vector<std::vector<std::pair<int, int>>> slot;      // per parameter of several groups: (group, slot)
+    std::vector<int> owner;                                  // per parameter: the group that writes its columns (-1: none)
+    long long oX = 0, oT = 0, oZ = 0, lds = 0;
+};
+HessShape hess_shape(const Model_& M, bool amps_only);
+
 }  // namespace ctpwa

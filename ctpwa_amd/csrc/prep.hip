@@ -637,25 +637,6 @@ __global__ void k_amplitudes(AuxArgs a, long long e0, long long n, double* __res
     }
 }
 
-// amplitude rows for Grams of the amplitudes (fit fractions, interference): column-major
-// X[col][R], R = p * n + i (polarisation p of event e0 + i), columns Re A_a (a < namp)
-// then Im A_a; A_a = K_a Psi_b sl_u,p without couplings (withK == 0: Psi_b sl_u,p)
-__global__ void k_amp_rows(AuxArgs a, long long e0, long long n, double* __restrict__ X, long long ldx, int withK) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    long long e = e0 + i;
-    for (int am = 0; am < a.namp; ++am) {
-        const DAmp& A = a.amps[am];
-        double2 psi = block_psi(a, A.block, e);
-        double K = withK ? a.table[a.off_rec + (long long)A.rec * REC] : 1.0;
-        for (int p = 0; p < a.npol; ++p) {
-            double2 s = ev_sl(a.st, A.u, p, a.npol, e);
-            X[(long long)am * ldx + p * n + i] = K * (psi.x * s.x - psi.y * s.y);
-            X[(long long)(a.namp + am) * ldx + p * n + i] = K * (psi.x * s.y + psi.y * s.x);
-        }
-    }
-}
-
 // per-event partial-wave intensities: out[b][i] = sum_p |P_b(e, p)|^2 for the nblock
 // partial waves (blocks) and out[nblock][i] = I(e) = sum_p |sum_b P_b|^2, with
 // P_b = Psi_b sum_{a in b} c_a sl_u(a),p and c_a = v_a K_a (src/ComputeResults.cu:57-190)
@@ -820,15 +801,6 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finaliz
                                                                                   hipStream_t stream) {
     hipLaunchKernelGGL(ctpwa::k_finalize, dim3(3 * f->nacc), dim3(ctpwa::ASM_THREADS), ctpwa::assemble_lds_bytes(*f), stream,
                        *f, done);
-    return hipGetLastError();
-}
-
-extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_amp_rows(const ctpwa::AuxArgs* a, long long e0,
-                                                                                  long long n, double* X, long long ldx,
-                                                                                  int withK, hipStream_t stream) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(ctpwa::k_amp_rows, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, stream, *a, e0, n, X, ldx,
-                       withK);
     return hipGetLastError();
 }
 

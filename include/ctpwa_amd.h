@@ -152,11 +152,9 @@ int ctpwa_time_eval_kernel(ctpwa_handle* h, const double* params_dev, int iters,
 long long ctpwa_footprint_bytes(const char* plan_text, long long n_phsp, long long n_data, long long n_bkg,
                                 int precision);
 
-/* device bytes a handle allocates on its first ctpwa_hessian call (the per-chunk
- * Jacobian rows and partial sums it keeps until ctpwa_destroy).  A handle that is alone
- * in the process, with at least 2^20 phase-space and 2^17 data + background events, runs
- * data and background on a second stream with a second buffer set; the estimate counts
- * that set when no handle is live at the time of this call */
+/* device bytes a handle allocates on its first ctpwa_hessian call and keeps until
+ * ctpwa_destroy: partial sums, and with more than 64 Jacobian columns the rows of a pass
+ * (the larger of the two storage forms' needs) */
 long long ctpwa_hessian_workspace_bytes(const char* plan_text, long long n_phsp, long long n_data, long long n_bkg);
 
 /* number of events of a class, and algorithmic bytes the fused kernel must read per
