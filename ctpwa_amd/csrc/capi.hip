@@ -263,14 +263,14 @@ struct GramWS {
     bool ready = false;
     HessShape S;
     hipModule_t mod = nullptr;
-    hipFunction_t fn = nullptr;
+    hipFunction_t fn = nullptr, fn_sum = nullptr, fn_theta = nullptr;
     int nz = 0;                          // summed columns
     int* perm = nullptr;                 // put order -> [Z | u] order
     int target = 0;                      // workgroups of the per-event kernel
     long long chunk = 0, cap = 0;        // events of a class per pass, events per pass
     long long ldJ = 0, ldc = 0;
     void* J = nullptr;
-    double *U = nullptr, *W = nullptr, *z = nullptr;
+    double *U = nullptr, *W = nullptr, *D = nullptr, *z = nullptr;
     GramTabs gJ, gU;
 };
 
@@ -1089,7 +1089,7 @@ static long long up(long long x, long long m) { return (x + m - 1) / m * m; }
 // multiple of 256), events of all classes per pass (cap), workgroups (four waves' registers
 // and the LDS of a CU shared out among the CU's workgroups), and the buffers in doubles
 struct GramSizes {
-    long long chunk, cap, ldJ, ldc, J, U, W, z, part;     // ldJ, ldc: rows of J and of U, W
+    long long chunk, cap, ldJ, ldc, J, U, W, D, z, part;     // ldJ, ldc: rows of J and of U, W, D
     int target, nz;
 };
 // the partials of a Gram: ncol <= 64 at least one workgroup per piece; more columns: two
@@ -1125,7 +1125,9 @@ static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long
     z.chunk = std::max<long long>(256, hess_jbytes() / row / 256 * 256);
     const long long all = n3[0] + n3[1] + n3[2];
     z.cap = std::max<long long>(1, std::min(all, z.chunk));
-    const int per_cu = std::max(1, (int)std::min<long long>(8 / S.G, 160 * 1024 / std::max<long long>(1, S.lds * 8)));
+    // (split rows: one-wave workgroups, as many times over as there are sets; 2 or 8 per CU and
+    // set are 2 % slower)
+    const int per_cu = S.split ? 4 : std::max(1, (int)std::min<long long>(8 / S.G, 160 * 1024 / std::max<long long>(1, S.lds * 8)));
     // (a class smaller than a workgroup's share still gets one)
     z.target = (int)std::min<long long>((long long)ncu * per_cu, std::max<long long>(1, (all + 63) / 64)) + 4;
     z.nz = S.NU > 0 ? hess_nz(M) + S.NU : 0;
@@ -1141,7 +1143,8 @@ static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long
     z.ldc = up(z.cap + 4 * 64, 64);
     z.J = z.ldJ * 2 * S.C;
     z.U = z.ldc * S.NU;
-    z.W = z.ldc * 2;
+    z.W = z.ldc * (S.split && S.NU > 0 ? 2 + 2 * M.P.npol : 2);
+    z.D = S.split ? z.ldc * S.nslot * 2 * M.P.npol : 0;
     int nwg = 0;
     z.part = gram_plan(2 * S.C, ncu, nullptr, &nwg) + (S.NU > 0 ? gram_plan(S.NU, ncu, nullptr, &nwg) : 0);
     return z;
@@ -1159,7 +1162,7 @@ static long long hess_workspace_bytes(const Model_& M0, const long long n3[3], l
         const HessShape S = hess_shape(M, false);
         const GramSizes z = gram_sizes(M, S, n3, 256);
         const long long nG = (long long)(2 * S.C) * (2 * S.C + 1) / 2, nUu = (long long)S.NU * (S.NU + 1) / 2;
-        long long w = 3 * (nG + nUu + z.nz) + (S.f32 ? z.J / 2 : z.J) + z.U + z.W + z.z + z.part;
+        long long w = 3 * (nG + nUu + z.nz) + (S.f32 ? z.J / 2 : z.J) + z.U + z.W + z.D + z.z + z.part;
         w += (long long)M.P.ntheta * M.P.ntheta * 4 + (long long)M.P.namp * M.P.ntheta;      // index tables
         w += (long long)M.customs.size() * M.ncf2() * ntot;   // second-order Custom factor rows
         most = std::max(most, w);
@@ -1172,7 +1175,7 @@ static long long agram_workspace_bytes(const Model_& M, long long n) {
     const long long n3[3] = {n, 0, 0};
     const HessShape S = hess_shape(M, true);
     const GramSizes z = gram_sizes(M, S, n3, 256);
-    return (z.J + z.U + z.W + z.z + z.part + (long long)M.P.namp * (2 * M.P.namp + 1)) * 8;
+    return (z.J + z.U + z.W + z.D + z.z + z.part + (long long)M.P.namp * (2 * M.P.namp + 1)) * 8;
 }
 
 // nwg > 0: the fused form's workgroups, each with its tile pairs' sums
@@ -1201,6 +1204,10 @@ static void gramws_setup(ctpwa_handle* h, GramWS& w, bool amps_only, const long 
     std::vector<int> perm;
     w.mod = compile_eval(h->device, generate_hess_kernel(M, &perm, amps_only));
     HIPCHECK(hipModuleGetFunction(&w.fn, w.mod, amps_only ? "ctpwa_amp_gram" : w.S.fused ? "ctpwa_hess_fused" : "ctpwa_hess_rows"));
+    if (w.S.split && !amps_only) {
+        HIPCHECK(hipModuleGetFunction(&w.fn_sum, w.mod, "ctpwa_hess_sum"));
+        HIPCHECK(hipModuleGetFunction(&w.fn_theta, w.mod, "ctpwa_hess_theta"));
+    }
     if ((int)perm.size() != z.nz) throw std::runtime_error("Hessian: summed-column count mismatch");
     w.perm = h->upload(perm);
     w.nz = z.nz;
@@ -1213,6 +1220,7 @@ static void gramws_setup(ctpwa_handle* h, GramWS& w, bool amps_only, const long 
     if (!w.S.fused) {
         w.J = h->alloc<unsigned char>((size_t)z.J * (w.S.f32 ? sizeof(float) : sizeof(double)));
         w.U = h->alloc<double>((size_t)z.U);
+        w.D = h->alloc<double>((size_t)z.D);
         // the amplitude Gram weights every row by one
         w.W = amps_only ? h->upload(std::vector<double>((size_t)z.W, 1.0)) : h->alloc<double>((size_t)z.W);
     }
@@ -1308,8 +1316,11 @@ static void gramws_run(ctpwa_handle* h, GramWS& w, const bool use[3], HessTotals
         double* gp = w.gJ.part;
         double* upart = w.gU.part;
         void* args[] = {&h->table, (void*)&h->slp, &h->inv, &h->invf, &h->ntot, &h->wts, &h->wc[1], &h->wc[2], &h->pw[1], &h->pw[2],
-                        &H, &w.J, &w.ldJ, &w.U, &w.W, &w.ldc, &gp, &upart, &w.z, &nwg, (void*)&cfr, &h->ntot, &withK};
-        HIPCHECK(hipModuleLaunchKernel(w.fn, nwg, 1, 1, 64 * w.S.G, 1, 1, 0, s, args, nullptr));
+                        &H, &w.J, &w.ldJ, &w.U, &w.W, &w.D, &w.ldc, &gp, &upart, &w.z, &nwg, (void*)&cfr, &h->ntot, &withK};
+        if (w.fn_sum) HIPCHECK(hipModuleLaunchKernel(w.fn_sum, nwg, 1, 1, 64 * (unsigned)w.S.sum_blocks.size(), 1, 1, 0, s, args, nullptr));
+        if (w.S.split) HIPCHECK(hipModuleLaunchKernel(w.fn, nwg, w.S.G, 1, 64, 1, 1, 0, s, args, nullptr));
+        else HIPCHECK(hipModuleLaunchKernel(w.fn, nwg, 1, 1, 64 * w.S.G, 1, 1, 0, s, args, nullptr));
+        if (w.fn_theta) HIPCHECK(hipModuleLaunchKernel(w.fn_theta, nwg, 1, 1, 64, 1, 1, 0, s, args, nullptr));
         for (int c = 0; c < 3; ++c) T.first[c] = !seen[c];
         for (int k = 0; k < H.n; ++k) seen[H.cls[k]] = true;
         // Grams of up to 64 columns: one launch for all pieces, summed with the columns below;

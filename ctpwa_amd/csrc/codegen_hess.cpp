@@ -26,13 +26,22 @@
 // scratch at 10 amplitudes, 7 KB at 149.  A parameter whose blocks lie in several groups is
 // summed through LDS slots in group order by one of them.
 //
-// Two forms:
+// Three forms:
 //  * fused (FP64 Jacobian of up to 64 real columns): J and u of the 64 events go into an LDS
 //    tile and straight into the FP64 matrix cores, whose tile pairs are shared out among the
 //    waves; nothing per event is written.  Written to memory and read back by the Gram
 //    kernel, the 40-column Jacobian of 3.05M events moved 3.9 GB (getHessian 1.31 ms).
 //  * rows: J (FP64, or FP32 in the mixed form), u and the weights are written to memory,
 //    column-major, for the Gram kernels.
+//  * split rows, for more than 24 amplitudes.  A workgroup of eight waves that runs the code
+//    of all 149 amplitudes for its 64 events fetches 600 KB of instructions per step (64 KB
+//    cache for two CUs), and each wave's 19 amplitudes spill: 6.9 ms for 600k events.  Here
+//    ctpwa_hess_sum forms S and the weights (eight wave groups, 0.2 ms); then every workgroup
+//    is one wave with one set of about eleven amplitudes (blockIdx.y), whose 30-50 KB of code
+//    stay cached while all workgroups of the set run (1.5 ms, of which 0.8 ms are the FP64
+//    instructions); then ctpwa_hess_theta adds up the parameters that several sets share
+//    (0.4 ms).  Sets of 7 to 15 amplitudes are within 3 %, single blocks 6 % slower: more
+//    parameters are shared then.
 #include <algorithm>
 #include <map>
 #include <set>
@@ -65,6 +74,8 @@ __device__ __forceinline__ double frcp(double x) {
 // that the 16 columns x 2 rows that half a wave reads lie in different banks and every
 // address is a lane offset plus a constant
 __device__ __forceinline__ double& xe(double* xs, int c, int r8) { return *(double*)((char*)xs + (c * 528 + r8)); }
+// element of a column at a lane's byte offset
+template <typename T> __device__ __forceinline__ T& at(T* col, unsigned off) { return *(T*)((char*)col + off); }
 __device__ __forceinline__ void wsync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -116,6 +127,9 @@ HessShape hess_shape(const Model_& M, bool amps_only) {
     int sets = 1;
     for (int k = 1; k < n; ++k) sets += pars(bl[k]) != pars(bl[k - 1]);
     int G = P.namp <= 4 ? 1 : P.namp <= (H.f32 ? 12 : 8) ? 2 : P.namp <= 24 ? 4 : 8;
+    H.fused = !H.f32 && 2 * H.C <= 64;
+    H.split = !H.fused && P.namp > 24;
+    if (H.split) G = (P.namp + 10) / 11;
     for (;; G /= 2) {
         G = std::max(1, std::min(G, n));
         // cuts: the largest group's cost (FP64 instructions) as small as possible; between
@@ -168,7 +182,15 @@ HessShape hess_shape(const Model_& M, bool amps_only) {
             load[o]++;
         }
         H.G = G;
-        H.fused = !H.f32 && 2 * H.C <= 64;
+        if (H.split) {
+            H.SW = 16;
+            H.lds = amps_only ? 0 : H.SW * 66;
+            // the summing kernel's wave groups: the same order of blocks, cut by amplitudes
+            H.sum_blocks.assign(std::min(8, n), {});
+            for (int k = 0, a = 0; k < n; a += P.blocks[bl[k++]].nsl)
+                H.sum_blocks[std::min<size_t>(H.sum_blocks.size() - 1, (size_t)a * H.sum_blocks.size() / P.namp)].push_back(bl[k]);
+            return H;
+        }
         const long long X = G > 1 && !amps_only ? (long long)G * 2 * NP * 64 : 0, T = (long long)H.nslot * 2 * NP * 64;
         // (the fused tile: a column of weights, then J of every polarisation, or u)
         const int GTn = (2 * H.C + 15) / 16;
@@ -199,7 +221,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
     const HessShape H = hess_shape(M, amps_only);
     const bool fused = H.fused, ahead = fused && 2 * H.C <= 48;
     const int NP = P.npol, NA = P.namp, NT = amps_only ? 0 : P.ntheta;
-    const int C = H.C, NUX = H.NU, G = H.G, SW = H.SW;
+    const int C = H.C, NUX = H.NU, SW = H.SW;
     const int GT = (2 * C + 15) / 16, UT = (NUX + 15) / 16;     // tiles of the two Grams
     const int NG2 = GT * (GT + 1) / 2, NU2 = UT * (UT + 1) / 2;
     std::ostringstream src;
@@ -233,15 +255,27 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
     const std::string SIG =
         "    const double* __restrict__ tab, const void* __restrict__ slv, const double* __restrict__ inv,\n"
         "    const float* __restrict__ invf, long long ld, const double* __restrict__ wts, double w1, double w2,\n"
-        "    int pw1, int pw2, HessPieces H, " + std::string(JT) + "* __restrict__ J, long long ldJ, double* __restrict__ U, double* __restrict__ W,\n"
+        "    int pw1, int pw2, HessPieces H, " + std::string(JT) + "* __restrict__ J, long long ldJ, double* __restrict__ U, double* __restrict__ W, double* __restrict__ D,\n"
         "    long long ldc, double* __restrict__ gpart, double* __restrict__ upart, double* __restrict__ zpart, int nwg,\n"
         "    const double* __restrict__ cfr, long long cld, int withK";
-    const std::string CALL = "tab, slv, inv, invf, ld, wts, w1, w2, pw1, pw2, H, J, ldJ, U, W, ldc, gpart, upart, zpart, nwg, cfr, cld, withK";
+    const std::string CALL = "tab, slv, inv, invf, ld, wts, w1, w2, pw1, pw2, H, J, ldJ, U, W, D, ldc, gpart, upart, zpart, nwg, cfr, cld, withK";
     std::vector<int> order_cols;
     std::ostringstream bodies;
-    for (int g = 0; g < G; ++g) {
+    // the generated functions: the groups, and in the split form the sets, the parameter
+    // columns and the groups of the summing kernel
+    enum Kind { GROUP, SET, THETA, SUM };
+    struct Body { Kind kind; int g, waves; std::vector<int> blocks; };
+    std::vector<Body> todo;
+    for (int g = 0; g < H.G; ++g) todo.push_back({H.split ? SET : GROUP, g, H.split ? 1 : H.G, H.blocks[g]});
+    if (H.split && !amps_only) {
+        todo.push_back({THETA, 0, 1, {}});
+        for (size_t g = 0; g < H.sum_blocks.size(); ++g) todo.push_back({SUM, (int)g, (int)H.sum_blocks.size(), H.sum_blocks[g]});
+    }
+    for (const Body& body : todo) {
         std::ostringstream o;
-        const std::vector<int>& blocks = H.blocks[g];
+        const std::vector<int>& blocks = body.blocks;
+        const int g = body.g, G = body.waves;
+        const Kind kind = body.kind;
         const int col0 = (int)order_cols.size();           // this wave's first summed column
         auto nput = [&]() { return (int)order_cols.size() - col0; };
         // what the group reads
@@ -278,7 +312,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                 for (int k = 0; k < (amps_only ? 2 : ncfr); ++k)
                     inputs.push_back({"double", "ncf" + std::to_string(c) + "_" + std::to_string(k),
                                       "cfr[" + std::to_string((long long)c * ncfr + k) + "LL * cld + e]"});
-        if (!amps_only) inputs.push_back({"double", "nwload", "(cls != 0 && wvar) ? wts[e] : wconst"});
+        if (!amps_only && (kind == GROUP || kind == SUM)) inputs.push_back({"double", "nwload", "(cls != 0 && wvar) ? wts[e] : wconst"});
         for (const Input& in : inputs) {
             if (!ahead) o << "  const " << in.type << " " << in.name << " = " << in.src << ";\n";
             if (in.type == SLT) continue;
@@ -314,6 +348,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
             o << "    long long z_" << ph << " = 0;\n    asm volatile(\"\" : \"+s\"(z_" << ph << "));\n"
               << "    const double* __restrict__ tb_" << ph << " = tab + z_" << ph << ";\n"
               << (inner ? "    int l8 = lane * 8;\n" : "    l8 = lane * 8;\n") << "    asm volatile(\"\" : \"+v\"(l8));\n    (void)l8;\n";
+            if (!fused) o << "    lj = ldJ; lc = ldc; lu = cls != 0 ? ldc : 0;\n    asm volatile(\"\" : \"+s\"(lj), \"+s\"(lc), \"+s\"(lu));\n";
         };
         auto rec = [&](int ph, long long rr, int comp) {
             std::ostringstream q;
@@ -346,19 +381,23 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
         };
         auto sn = [&](int u, int p) { return "s" + std::to_string(u) + "_" + std::to_string(p); };
         auto jstore = [&](int col, int p, const std::string& v, const char* ind) {
-            o << ind << "J[" << col << "LL * ldJ + jr" << p << "] = (" << JT << ")(" << v << ");\n";
+            o << ind << "at(J" << p << " + " << col << "LL * lj, ro * (unsigned)sizeof(" << JT << ")) = (" << JT << ")(" << v << ");\n";
         };
         auto gsync = [&]() { o << (G > 1 ? "  __syncthreads();\n" : "  wsync();\n"); };
 
         // ---- phase 1: block products, amplitudes, S, I, weights ---------------------------
+        const bool first = amps_only || kind == GROUP || kind == SUM, stores = !fused && kind != SUM;
         phase_vars(1, false);
         if (fused)
             for (int b : blocks)
                 for (int c = 0; c < P.blocks[b].nsl; ++c)
                     o << "  double F" << P.blocks[b].site + c << "r, F" << P.blocks[b].site + c << "i;\n";
         if (!amps_only)
-            for (int p = 0; p < NP; ++p) o << "  double S" << p << "r = 0.0, S" << p << "i = 0.0;\n";
+            for (int p = 0; p < NP; ++p)
+                for (int c = 0; c < 2; ++c)
+                    o << "  double S" << p << (c ? "i" : "r") << " = " << (first ? std::string("0.0") : "at(Wk + " + std::to_string(2 + 2 * p + c) + "LL * lc, wo)") << ";\n";
         for (int b : blocks) {
+            if (!first) break;
             const PBlock& B = P.blocks[b];
             o << "  {\n";
             phase_vars(1, true);
@@ -378,7 +417,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                       << sn(u, p) << "x;\n";
                     if (!amps_only)
                         o << "        S" << p << "r += vr * ar - vi * ai; S" << p << "i += vr * ai + vi * ar;\n";
-                    if (!fused) {
+                    if (stores) {
                         jstore(a, p, "ar", "        ");
                         jstore(C + a, p, "ai", "        ");
                     }
@@ -403,20 +442,30 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                     }
             }
             // a lane past the end: S = 0 makes every sum it hands in zero
-            o << "  if (!live) {";
-            for (int p = 0; p < NP; ++p) o << " S" << p << "r = 0.0; S" << p << "i = 0.0;";
-            o << " }\n  double I = 0.0;\n";
+            if (first) {
+                o << "  if (!live) {";
+                for (int p = 0; p < NP; ++p) o << " S" << p << "r = 0.0; S" << p << "i = 0.0;";
+                o << " }\n";
+            }
+            o << "  double I = 0.0;\n";
             for (int p = 0; p < NP; ++p) o << "  I += S" << p << "r * S" << p << "r + S" << p << "i * S" << p << "i;\n";
-            o << "  const double we = (cls == 0) ? 1.0 : wload;\n"
+            if (!first) o << "  const double alpha = at(Wk, wo);\n";
+            else o << "  const double we = (cls == 0) ? 1.0 : wload;\n"
                  "  double alpha, beta;\n"
                  "  if (cls == 0) { alpha = 1.0; beta = 0.0; }\n"
                  "  else if (I == 0.0) { alpha = 0.0; beta = 0.0; }\n"
                  "  else { const double iI = frcp(I); alpha = we * iI; beta = -alpha * iI; }\n";
-            if (!fused && g == 0) o << "  W[wr] = alpha; W[ldc + wr] = beta;\n";
-            if (!fused) o << "  const bool ust = cls != 0;   // wave-uniform: a scalar branch around each u store\n";
+            if (!fused && first && g == 0) o << "  at(Wk, wo) = alpha; at(Wk + lc, wo) = beta;\n";
+            if (kind == SUM) {
+                for (int p = 0; p < NP && g == 0; ++p)
+                    o << "  at(Wk + " << 2 + 2 * p << "LL * lc, wo) = S" << p << "r; at(Wk + " << 3 + 2 * p << "LL * lc, wo) = S" << p << "i;\n";
+                if (G > 1) o << "  __syncthreads();\n";      // every wave has read the exchanged S
+            }
+        }
+        if (!amps_only && kind != SUM) {
 
             // ---- phase 2: u, derivative columns and second-part scalars --------------------
-            o << "  double* zs = sm + " << H.oZ + (long long)g * SW * 66 << ";\n";
+            o << "  double* zs = sm + " << (H.split ? 0 : H.oZ + (long long)g * SW * 66) << ";\n";
             auto flush = [&](const char* ind) {
                 o << ind << "zf" << (nput() - 1) / SW << " += col_part(zs, l8 >> 3);\n";
             };
@@ -427,7 +476,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
             };
             auto ustore = [&](const std::string& v, int x, const char* ind) {
                 put(v, col_u0 + x, ind);
-                if (!fused) o << ind << "if (ust) U[" << x << "LL * ldc + wr] = " << v << ";\n";
+                if (!fused) o << ind << (kind == GROUP ? "if (cls != 0) " : "") << "at(Uk + " << x << "LL * lu, wo) = " << v << ";\n";
             };
             // a parameter's finished derivative columns
             auto theta_cols = [&](int j) {
@@ -444,7 +493,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                 }
             };
             phase_vars(2, false);
-            if (g == 0) put("alpha * I", col_I, "  ");
+            if (g == 0 && kind != SET) put("alpha * I", col_I, "  ");
             std::vector<int> last(NT, -1);
             for (size_t k = 0; k < blocks.size(); ++k)
                 for (int j : M.bvars[blocks[k]]) last[j] = (int)k;
@@ -562,6 +611,10 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                       << "      const double Fr = K * psr, Fi = K * psi_;\n"
                       // g_a = conj(F_a) T_u: dI/dRe v_a = 2 Re g, dI/dIm v_a = 2 Im g
                       << "      const double gr = Fr * t" << u << "r + Fi * t" << u << "i, gi = Fr * t" << u << "i - Fi * t" << u << "r;\n";
+                    for (int p = 0; p < NP && kind == SET; ++p) {
+                        jstore(a, p, "Fr * " + sn(u, p) + "x - Fi * " + sn(u, p) + "y", "      ");
+                        jstore(C + a, p, "Fr * " + sn(u, p) + "y + Fi * " + sn(u, p) + "x", "      ");
+                    }
                     ustore("2.0 * gr", a, "      ");
                     ustore("2.0 * gi", NA + a, "      ");
                     for (int i = 0; i < nl; ++i) {
@@ -592,6 +645,9 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                         o << "      }\n";
                     }
                     o << "    }\n";
+                    // (regions of one amplitude: scheduling a whole block at once takes the
+                    // compiler five times as long and keeps no fewer registers)
+                    if (kind == SET) o << "    __builtin_amdgcn_sched_barrier(0);\n";
                 }
                 // R_ik = sum_a Re(v_a d2F_ik conj(T_u)), d2F_ik = K_ik Psi - K_i P1_k - K_k P1_i + K P2_ik
                 {
@@ -612,7 +668,11 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                     if (last[j] != (int)kb) continue;
                     if (H.slot[j].empty()) { theta_cols(j); continue; }
                     for (const auto& s : H.slot[j])
-                        if (s.first == g)
+                        if (s.first == g && kind == SET)
+                            for (int p = 0; p < NP; ++p)
+                                o << "  at(Dk + " << s.second * 2 * NP + 2 * p << "LL * lc, wo) = dS" << j << "_" << p << "r; at(Dk + " << s.second * 2 * NP + 2 * p + 1
+                                  << "LL * lc, wo) = dS" << j << "_" << p << "i;\n";
+                        else if (s.first == g)
                             for (int p = 0; p < NP; ++p)
                                 o << "  sm[" << H.oT + ((long long)s.second * 2 * NP + 2 * p) * 64 << " + lane] = dS" << j << "_" << p << "r; sm["
                                   << H.oT + ((long long)s.second * 2 * NP + 2 * p + 1) * 64 << " + lane] = dS" << j << "_" << p << "i;\n";
@@ -623,20 +683,22 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
             // the slots are written again only after the next iteration's first barrier.)
             if (G > 1) o << "  __syncthreads();\n";
             for (int j = 0; j < NT; ++j) {
-                if (H.slot[j].empty() || H.owner[j] != g) continue;
+                if (H.slot[j].empty() || (H.split ? kind != THETA : H.owner[j] != g)) continue;
+                if (H.split) phase_vars(3 + j, false);
                 for (int p = 0; p < NP; ++p)
                     for (int c = 0; c < 2; ++c) {
                         o << "  " << (open_[j] ? "" : "double ") << "dS" << j << "_" << p << (c ? "i" : "r") << " = ";
                         for (size_t k = 0; k < H.slot[j].size(); ++k)
-                            o << (k ? " + " : "") << "sm[" << H.oT + ((long long)H.slot[j][k].second * 2 * NP + 2 * p + c) * 64 << " + lane]";
+                            if (H.split) o << (k ? " + " : "") << "at(Dk + " << H.slot[j][k].second * 2 * NP + 2 * p + c << "LL * lc, wo)";
+                            else o << (k ? " + " : "") << "sm[" << H.oT + ((long long)H.slot[j][k].second * 2 * NP + 2 * p + c) * 64 << " + lane]";
                         o << ";\n";
                     }
                 theta_cols(j);
             }
             // parameters of no block with waves: zero columns
-            if (g == 0)
+            if (g == 0 && kind != SET)
                 for (int j = 0; j < NT; ++j)
-                    if (H.owner[j] < 0) {
+                    if (H.owner[j] < 0 && H.slot[j].empty()) {
                         for (int p = 0; p < NP; ++p) o << "  const double dS" << j << "_" << p << "r = 0.0, dS" << j << "_" << p << "i = 0.0;\n";
                         theta_cols(j);
                     }
@@ -725,7 +787,8 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
         }
         // the function: declarations, the loop over the workgroup's events, the partial sums
         const int ncols = nput(), nflush = (ncols + SW - 1) / SW;
-        bodies << "__device__ __forceinline__ void hess_g" << g << "(\n" << SIG << ", double* __restrict__ sm)\n{\n"
+        static const char* const fname[] = {"hess_g", "hess_g", "hess_t", "hess_s"};
+        bodies << "__device__ __forceinline__ void " << fname[kind] << g << "(\n" << SIG << ", double* __restrict__ sm)\n{\n"
                << "  const " << SLT << "* __restrict__ sl = (const " << SLT << "*)slv;\n"
                << "  const int lane = threadIdx.x & 63, wg = blockIdx.x;\n"
                   "  int k = 0;\n  while (k + 1 < H.n && wg >= H.wg0[k + 1]) ++k;\n"
@@ -736,6 +799,18 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                   "  const double wconst = cls == 1 ? w1 : w2;\n"
                   "  const bool wvar = cls == 1 ? pw1 != 0 : cls == 2 && pw2 != 0;\n";
         for (int f = 0; f < nflush; ++f) bodies << "  double zf" << f << " = 0.0;\n";
+        if (!fused) {
+            // rows: uniform column addresses plus a 32-bit lane offset.  The column strides pass
+            // through empty asm statements (phase_vars), or hundreds of column addresses are
+            // formed before the loop and kept in spilled registers.  Phase space has no u.  In
+            // the sets its stores go to one column that nothing reads: a branch around each
+            // store would cut the block's code into pieces that the compiler schedules and
+            // allocates badly (2.5 KB of scratch per lane).  Groups of a smaller model take the
+            // branch (305k events of the 10-amplitude model, mixed: 132 us, without 141 us).
+            bodies << "  long long lj = ldJ, lc = ldc, lu = ldc;\n  (void)lj; (void)lc; (void)lu;\n";
+            for (int p = 0; p < NP; ++p) bodies << "  " << JT << "* __restrict__ J" << p << " = J + H.row0[k] + " << p << " * cnt;\n";
+            if (!amps_only) bodies << "  double *__restrict__ Uk = U + H.w0[k], *__restrict__ Wk = W + H.w0[k], *__restrict__ Dk = D + H.w0[k];\n";
+        }
         if (fused) {
             for (int q = 0; q < NG2; ++q) bodies << "  d4 ag" << q << " = (d4){0.0, 0.0, 0.0, 0.0};\n";
             for (int q = 0; q < NU2; ++q) bodies << "  d4 au" << q << " = (d4){0.0, 0.0, 0.0, 0.0};\n";
@@ -755,9 +830,9 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
                   "  const long long r = live ? t0 + lane : b1 - 1;\n"
                   "  const long long e = pe0 + r;\n  (void)e;\n";
         if (!fused) {
-            for (int p = 0; p < NP; ++p) bodies << "  const long long jr" << p << " = H.row0[k] + " << p << " * cnt + r;\n";
             // (the u and weight entries of lanes past the end go to the piece's padding)
-            if (!amps_only) bodies << "  const long long wr = H.w0[k] + t0 + lane;\n";
+            bodies << "  const unsigned ro = (unsigned)r;\n";
+            if (!amps_only) bodies << "  const unsigned wo = (unsigned)(t0 + lane) * 8u;\n";
         }
         bodies << o.str() << "  }\n";
         if (fused) {
@@ -795,17 +870,25 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
     if (!amps_only && (int)order_cols.size() != NZ + 1 + NUX) throw std::runtime_error("Hessian generator: summed-column count mismatch");
     if (perm) *perm = order_cols;
     src << bodies.str();
-    const char* name = amps_only ? "ctpwa_amp_gram" : fused ? "ctpwa_hess_fused" : "ctpwa_hess_rows";
-    src << "extern \"C\" __global__ void __launch_bounds__(" << 64 * G << (G < 8 && (!fused || 2 * C <= 48) ? ", 2" : "") << ") " << name << "(\n" << SIG << ")\n{\n"
-        << "  __shared__ __attribute__((aligned(16))) double sm[" << std::max<long long>(H.lds, 2) << "];\n";
-    if (G == 1) src << "  hess_g0(" << CALL << ", sm);\n";
-    else {
-        src << "  switch (__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) {\n";
-        for (int g = 0; g < G; ++g)
-            src << "  " << (g + 1 < G ? "case " + std::to_string(g) : std::string("default")) << ": hess_g" << g << "(" << CALL << ", sm); break;\n";
-        src << "  }\n";
+    // a kernel of n functions, one per wave of the workgroup or (sets) per blockIdx.y
+    auto kernel = [&](const char* name, const char* fn, int n, bool sets, long long lds, const char* bounds) {
+        src << "extern \"C\" __global__ void __launch_bounds__(" << (sets ? 64 : 64 * n) << bounds << ") " << name << "(\n" << SIG << ")\n{\n"
+            << "  __shared__ __attribute__((aligned(16))) double sm[" << std::max<long long>(lds, 2) << "];\n";
+        if (n == 1) {
+            src << "  " << fn << "0(" << CALL << ", sm);\n}\n";
+            return;
+        }
+        src << "  switch (" << (sets ? "blockIdx.y" : "__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))") << ") {\n";
+        for (int g = 0; g < n; ++g)
+            src << "  " << (g + 1 < n ? "case " + std::to_string(g) : std::string("default")) << ": " << fn << g << "(" << CALL << ", sm); break;\n";
+        src << "  }\n}\n";
+    };
+    kernel(amps_only ? "ctpwa_amp_gram" : fused ? "ctpwa_hess_fused" : "ctpwa_hess_rows", "hess_g", H.G, H.split, H.lds,
+           H.split || (H.G < 8 && (!fused || 2 * C <= 48)) ? ", 2" : "");
+    if (H.split && !amps_only) {
+        kernel("ctpwa_hess_theta", "hess_t", 1, true, H.lds, "");
+        kernel("ctpwa_hess_sum", "hess_s", (int)H.sum_blocks.size(), false, (long long)H.sum_blocks.size() * 2 * NP * 64, "");
     }
-    src << "}\n";
     return src.str();
 }
 

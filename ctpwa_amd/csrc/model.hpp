@@ -659,8 +659,9 @@ inline Model_ derive(const Plan& P) {
 // slabs of SW columns per wave; the fused form's tile takes the place of all of them)
 struct HessShape {
     int G = 1, C = 0, NU = 0, SW = 16, nslot = 0;
-    bool fused = false, f32 = false;
-    std::vector<std::vector<int>> blocks;                    // per group
+    bool fused = false, f32 = false, split = false;
+    std::vector<std::vector<int>> blocks;                    // per group (split: per set)
+    std::vector<std::vector<int>> sum_blocks;                // split: per wave group of the summing kernel
     std::vector<std::vector<std::pair<int, int>>> slot;      // per parameter of several groups: (group, slot)
     std::vector<int> owner;                                  // per parameter: the group that writes its columns (-1: none)
     long long oX = 0, oT = 0, oZ = 0, lds = 0;
