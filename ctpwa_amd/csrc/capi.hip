@@ -39,7 +39,7 @@ extern "C" hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs*, unsigned int*
 extern "C" hipError_t ctpwa_launch_prep_batch(const double* const*, double* const*, const ctpwa::PrepArgs*, int,
                                               const ctpwa::PrepArgs*, int, const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_finalize_batch(const ctpwa::FinArgs*, int, int, size_t, const int*, hipStream_t);
-extern "C" hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs*, long long, long long, double*, int, hipStream_t);
+extern "C" hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs*, int, long long, long long, double*, int, hipStream_t);
 
 
 extern "C" hipError_t ctpwa_launch_zero(double*, long long, hipStream_t);
@@ -1582,7 +1582,7 @@ static int aux_call(ctpwa_handle* h, const double* params_dev, int cls, double* 
             e = hipModuleLaunchKernel(h->fn_aux, (unsigned)((n + 255) / 256), 1, 1, 256, 1, 1, 0, s, args, nullptr);
         }
     } else if (e == hipSuccess) {
-        e = ctpwa_launch_aux(&h->aux, h->off[cls], h->n[cls], out_dev, intensity, s);
+        e = ctpwa_launch_aux(&h->aux, (int)h->M.P.blocks.size(), h->off[cls], h->n[cls], out_dev, intensity, s);
     }
     if (e != hipSuccess) return fail(hipGetErrorString(e));
     return 0;

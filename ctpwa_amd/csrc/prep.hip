@@ -586,21 +586,50 @@ __global__ void __launch_bounds__(ASM_THREADS) k_assemble_batch(const FinArgs* _
 // generic per-event amplitudes and intensities
 // ---------------------------------------------------------------------------
 
-__device__ inline double2 block_psi(const AuxArgs& a, int b, long long e) {
-    const DBlock& B = a.blocks[b];
+// The model's tables are the same for every event, and nothing writes them while these
+// kernels run: reads through the constant address space become scalar loads, shared by the
+// wave and free of the vector memory counter.  As vector loads, each of a block's five
+// dependent table reads waited behind the kernel's own output stores.  With them, one pass
+// over all polarisations instead of one each, and one-wave workgroups, the partial amplitudes
+// of 1M events (11 waves, 120 MB read, 352 MB written) take 140 us instead of 197: 3.4 TB/s,
+// bound by writing eleven streams to memory (half the events, which the last-level cache
+// takes, 45 us).  Two or four events per thread, which walk the tables once, and nontemporal
+// stores change nothing.
+__device__ __forceinline__ int uni(const int* p) { return *(const __attribute__((address_space(4))) int*)(unsigned long long)p; }
+__device__ __forceinline__ double uni(const double* p) { return *(const __attribute__((address_space(4))) double*)(unsigned long long)p; }
+
+__device__ __forceinline__ double post_inv(const EvStore& s, int i, long long e) {
+    if (s.mixed) {
+        const int m = uni(s.imap + i);
+        return (m >= 0) ? s.inv[(long long)m * s.ld + e] : (double)s.invf[(long long)(-m - 1) * s.ld + e];
+    }
+    return s.inv[(long long)i * s.ld + e];
+}
+__device__ __forceinline__ double2 post_sl(const EvStore& s, int u, int p, int npol, long long e) {
+    if (p < s.nps) return ev_sl_row(s, (long long)u * s.nps + p, e);
+    const double2 m = ev_sl_row(s, (long long)u * s.nps + (npol - 1 - p), e);
+    const double g = (double)uni(s.psign + u);
+    return make_double2(g * m.x, -g * m.y);
+}
+
+__device__ __forceinline__ double2 block_psi(const AuxArgs& a, int b, long long e) {
+    const DBlock* B = a.blocks + b;
     double pr = 1.0, pi = 0.0;
-    for (int d = 0; d < B.nden; ++d) {
-        const DDen& D = a.dens[B.den0 + d];
-        const DDenTerms& DT = a.dterms[B.den0 + d];
+    const int nden = uni(&B->nden), den0 = uni(&B->den0);
+    for (int d = den0; d < den0 + nden; ++d) {
+        const int rec = uni(&a.dens[d].rec);
+        const DDenTerms* DT = a.dterms + d;
+        const int nre = uni(&DT->nre), nt = nre + uni(&DT->nim), t0 = uni(&DT->t0);
         double dr = 0.0, di = 0.0;
-        for (int t = 0; t < DT.nre + DT.nim; ++t) {
-            const DTerm& T = a.terms[DT.t0 + t];
-            double c = (T.coef < 0) ? T.cval : a.table[a.off_rec + (long long)(D.rec + T.coef) * REC];
-            double x = (T.inv < 0) ? 1.0 : ev_inv(a.st, T.inv, e);
-            if (t < DT.nre) dr += c * x; else di += c * x;
+        for (int t = 0; t < nt; ++t) {
+            const DTerm* T = a.terms + t0 + t;
+            const int coef = uni(&T->coef), inv = uni(&T->inv);
+            const double c = (coef < 0) ? uni(&T->cval) : uni(a.table + a.off_rec + (long long)(rec + coef) * REC);
+            const double x = (inv < 0) ? 1.0 : post_inv(a.st, inv, e);
+            if (t < nre) dr += c * x; else di += c * x;
         }
         double xr = dr, xi = di;                          // table lineshape: the factor itself
-        if (!DT.stat) {
+        if (!uni(&DT->stat)) {
             const double q = 1.0 / (dr * dr + di * di);
             xr = dr * q;                                  // 1 / (dr - i di)
             xi = di * q;
@@ -609,8 +638,8 @@ __device__ inline double2 block_psi(const AuxArgs& a, int b, long long e) {
         pr = nr; pi = ni;
     }
     // Custom lineshape factors (written for this parameter point by the Custom kernel)
-    for (int q = a.bcp[b]; q < a.bcp[b + 1]; ++q) {
-        const double* f = a.cfb + (long long)a.bcl[q] * a.ncf * a.cld + e;
+    for (int q = uni(a.bcp + b); q < uni(a.bcp + b + 1); ++q) {
+        const double* f = a.cfb + (long long)uni(a.bcl + q) * a.ncf * a.cld + e;
         const double fr = f[0], fi = f[a.cld];
         const double nr = pr * fr - pi * fi, ni = pr * fi + pi * fr;
         pr = nr; pi = ni;
@@ -618,17 +647,56 @@ __device__ inline double2 block_psi(const AuxArgs& a, int b, long long e) {
     return make_double2(pr, pi);
 }
 
+// NP > 0: the model's polarisation count, known at compile time (registers, unrolled);
+// 0: any count
+template <int NP> struct PolArr { double r[NP], i[NP]; };
+template <> struct PolArr<0> { double r[MAXPOL], i[MAXPOL]; };
+
+// w += P_b(e, p0 + p) of NP polarisations (those below npol), or of all npol (NP = 0, p0 = 0)
+template <int NP>
+__device__ __forceinline__ void add_block(const AuxArgs& a, int b, long long e, int p0, int npol, PolArr<NP>& w) {
+    const int np = NP ? NP : npol;
+    const int nsl = uni(&a.blocks[b].nsl), site = uni(&a.blocks[b].site);
+    if (nsl <= 0) return;
+    const double2 psi = block_psi(a, b, e);
+    PolArr<NP> y;
+#pragma unroll NP ? NP : 1
+    for (int p = 0; p < np; ++p) { y.r[p] = 0.0; y.i[p] = 0.0; }
+    for (int am = site; am < site + nsl; ++am) {
+        const double cr = uni(a.table + a.off_c + 2 * am), ci = uni(a.table + a.off_c + 2 * am + 1);
+        const int u = uni(&a.amps[am].u);
+#pragma unroll NP ? NP : 1
+        for (int p = 0; p < np; ++p) {
+            if (NP && p0 + p >= npol) continue;
+            const double2 s = post_sl(a.st, u, p0 + p, npol, e);
+            y.r[p] += cr * s.x - ci * s.y;
+            y.i[p] += cr * s.y + ci * s.x;
+        }
+    }
+#pragma unroll NP ? NP : 1
+    for (int p = 0; p < np; ++p) {
+        w.r[p] += psi.x * y.r[p] - psi.y * y.i[p];
+        w.i[p] += psi.x * y.i[p] + psi.y * y.r[p];
+    }
+}
+
 // A[e][p][a] = K_a Psi_b(e) sl_u,p(e)  (interleaved complex), events [e0, e0 + n)
-__global__ void k_amplitudes(AuxArgs a, long long e0, long long n, double* __restrict__ out) {
+__global__ void __launch_bounds__(128) k_amplitudes(AuxArgs a, long long e0, long long n, double* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     long long e = e0 + i;
+    int block = -1;
+    double2 psi = make_double2(0.0, 0.0);
     for (int am = 0; am < a.namp; ++am) {
-        const DAmp& A = a.amps[am];
-        double2 psi = block_psi(a, A.block, e);
-        double K = a.table[a.off_rec + (long long)A.rec * REC];
+        const DAmp* A = a.amps + am;
+        if (uni(&A->block) != block) {
+            block = uni(&A->block);
+            psi = block_psi(a, block, e);
+        }
+        const double K = uni(a.table + a.off_rec + (long long)uni(&A->rec) * REC);
+        const int u = uni(&A->u);
         for (int p = 0; p < a.npol; ++p) {
-            double2 s = ev_sl(a.st, A.u, p, a.npol, e);
+            double2 s = post_sl(a.st, u, p, a.npol, e);
             double r = K * (psi.x * s.x - psi.y * s.y), im = K * (psi.x * s.y + psi.y * s.x);
             long long o = ((i * a.npol + p) * a.namp + am) * 2;
             out[o] = r;
@@ -643,94 +711,67 @@ __global__ void k_amplitudes(AuxArgs a, long long e0, long long n, double* __res
 // partial wave w = blocks wblk[wptr[w] .. wptr[w+1]) (a block and its identical-particle
 // permuted copies): out[w][i] = sum_pol |sum over the wave's blocks P_b|^2,
 // out[nwave][i] = the total intensity
-__global__ void k_partial_int(AuxArgs a, const int* __restrict__ wptr, const int* __restrict__ wblk, int nwave,
-                              long long e0, long long n, double* __restrict__ out) {
+template <int NP>
+__global__ void __launch_bounds__(64) k_partial_int(AuxArgs a, const int* __restrict__ wptr, const int* __restrict__ wblk, int nwave,
+                                                     long long e0, long long n, double* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    long long e = e0 + i;
-    double Sr[MAXPOL], Si[MAXPOL], Wr[MAXPOL], Wi[MAXPOL];
-    for (int p = 0; p < a.npol; ++p) { Sr[p] = 0.0; Si[p] = 0.0; }
+    const long long e = e0 + i;
+    const int npol = NP ? NP : a.npol;
+    PolArr<NP> S, W;
+#pragma unroll NP ? NP : 1
+    for (int p = 0; p < npol; ++p) { S.r[p] = 0.0; S.i[p] = 0.0; }
     for (int w = 0; w < nwave; ++w) {
-        for (int p = 0; p < a.npol; ++p) { Wr[p] = 0.0; Wi[p] = 0.0; }
-        for (int k = wptr[w]; k < wptr[w + 1]; ++k) {
-            const DBlock& B = a.blocks[wblk[k]];
-            if (B.nsl <= 0) continue;
-            double2 psi = block_psi(a, wblk[k], e);
-            for (int p = 0; p < a.npol; ++p) {
-                double yr = 0.0, yi = 0.0;
-                for (int c = 0; c < B.nsl; ++c) {
-                    const int am = B.site + c;
-                    const double cr = a.table[a.off_c + 2 * am], ci = a.table[a.off_c + 2 * am + 1];
-                    double2 s = ev_sl(a.st, a.amps[am].u, p, a.npol, e);
-                    yr += cr * s.x - ci * s.y;
-                    yi += cr * s.y + ci * s.x;
-                }
-                Wr[p] += psi.x * yr - psi.y * yi;
-                Wi[p] += psi.x * yi + psi.y * yr;
-            }
-        }
+#pragma unroll NP ? NP : 1
+        for (int p = 0; p < npol; ++p) { W.r[p] = 0.0; W.i[p] = 0.0; }
+        for (int k = uni(wptr + w); k < uni(wptr + w + 1); ++k) add_block<NP>(a, uni(wblk + k), e, 0, npol, W);
         double v = 0.0;
-        for (int p = 0; p < a.npol; ++p) {
-            v += Wr[p] * Wr[p] + Wi[p] * Wi[p];
-            Sr[p] += Wr[p];
-            Si[p] += Wi[p];
+#pragma unroll NP ? NP : 1
+        for (int p = 0; p < npol; ++p) {
+            v += W.r[p] * W.r[p] + W.i[p] * W.i[p];
+            S.r[p] += W.r[p];
+            S.i[p] += W.i[p];
         }
         out[(long long)w * n + i] = v;
     }
     double I = 0.0;
-    for (int p = 0; p < a.npol; ++p) I += Sr[p] * Sr[p] + Si[p] * Si[p];
+#pragma unroll NP ? NP : 1
+    for (int p = 0; p < npol; ++p) I += S.r[p] * S.r[p] + S.i[p] * S.i[p];
     out[(long long)nwave * n + i] = I;
 }
 
 // coherent partial-wave amplitudes: out[w][i][p] = sum over the wave's blocks of P_b
 // (couplings applied), interleaved complex, events [e0, e0 + n)
-__global__ void k_partial_amp(AuxArgs a, const int* __restrict__ wptr, const int* __restrict__ wblk, int nwave,
-                              long long e0, long long n, double2* __restrict__ out) {
+template <int NP>
+__global__ void __launch_bounds__(64) k_partial_amp(AuxArgs a, const int* __restrict__ wptr, const int* __restrict__ wblk, int nwave,
+                                                     long long e0, long long n, double2* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    long long e = e0 + i;
-    for (int w = 0; w < nwave; ++w) {
-        for (int p = 0; p < a.npol; ++p) {
-            double wr = 0.0, wi = 0.0;
-            for (int k = wptr[w]; k < wptr[w + 1]; ++k) {
-                const DBlock& B = a.blocks[wblk[k]];
-                if (B.nsl <= 0) continue;
-                double2 psi = block_psi(a, wblk[k], e);
-                double yr = 0.0, yi = 0.0;
-                for (int c = 0; c < B.nsl; ++c) {
-                    const int am = B.site + c;
-                    const double cr = a.table[a.off_c + 2 * am], ci = a.table[a.off_c + 2 * am + 1];
-                    double2 s = ev_sl(a.st, a.amps[am].u, p, a.npol, e);
-                    yr += cr * s.x - ci * s.y;
-                    yi += cr * s.y + ci * s.x;
-                }
-                wr += psi.x * yr - psi.y * yi;
-                wi += psi.x * yi + psi.y * yr;
-            }
-            out[((long long)w * n + i) * a.npol + p] = make_double2(wr, wi);
+    const long long e = e0 + i;
+    for (int p0 = 0; p0 < a.npol; p0 += NP)
+        for (int w = 0; w < nwave; ++w) {
+            PolArr<NP> W;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) { W.r[p] = 0.0; W.i[p] = 0.0; }
+            for (int k = uni(wptr + w); k < uni(wptr + w + 1); ++k) add_block<NP>(a, uni(wblk + k), e, p0, a.npol, W);
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+                if (p0 + p < a.npol) out[((long long)w * n + i) * a.npol + p0 + p] = make_double2(W.r[p], W.i[p]);
         }
-    }
 }
 
-__global__ void k_intensity(AuxArgs a, long long e0, long long n, double* __restrict__ out) {
+template <int NP>
+__global__ void __launch_bounds__(64) k_intensity(AuxArgs a, int nblock, long long e0, long long n, double* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    long long e = e0 + i;
-    double Sr[MAXPOL], Si[MAXPOL];
-    for (int p = 0; p < a.npol; ++p) { Sr[p] = 0.0; Si[p] = 0.0; }
-    for (int am = 0; am < a.namp; ++am) {
-        const DAmp& A = a.amps[am];
-        double2 psi = block_psi(a, A.block, e);
-        double cr = a.table[a.off_c + 2 * am], ci = a.table[a.off_c + 2 * am + 1];
-        double yr = cr * psi.x - ci * psi.y, yi = cr * psi.y + ci * psi.x;
-        for (int p = 0; p < a.npol; ++p) {
-            double2 s = ev_sl(a.st, A.u, p, a.npol, e);
-            Sr[p] += yr * s.x - yi * s.y;
-            Si[p] += yr * s.y + yi * s.x;
-        }
-    }
+    const int npol = NP ? NP : a.npol;
+    PolArr<NP> S;
+#pragma unroll NP ? NP : 1
+    for (int p = 0; p < npol; ++p) { S.r[p] = 0.0; S.i[p] = 0.0; }
+    for (int b = 0; b < nblock; ++b) add_block<NP>(a, b, e0 + i, 0, npol, S);
     double I = 0.0;
-    for (int p = 0; p < a.npol; ++p) I += Sr[p] * Sr[p] + Si[p] * Si[p];
+#pragma unroll NP ? NP : 1
+    for (int p = 0; p < npol; ++p) I += S.r[p] * S.r[p] + S.i[p] * S.i[p];
     out[i] = I;
 }
 
@@ -804,13 +845,26 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finaliz
     return hipGetLastError();
 }
 
+// the polarisation count at compile time up to four; more: any count at once (MORE = 0), or in
+// groups of MORE
+#define POST_LAUNCH(K, MORE, npol, n, ...)                                                               \
+    do {                                                                                                 \
+        const dim3 g_((unsigned)((n + 63) / 64)), b_(64);                                                \
+        switch (npol) {                                                                                  \
+        case 1: hipLaunchKernelGGL(ctpwa::K<1>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
+        case 2: hipLaunchKernelGGL(ctpwa::K<2>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
+        case 3: hipLaunchKernelGGL(ctpwa::K<3>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
+        case 4: hipLaunchKernelGGL(ctpwa::K<4>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
+        default: hipLaunchKernelGGL(ctpwa::K<MORE>, g_, b_, 0, stream, __VA_ARGS__);                     \
+        }                                                                                                \
+    } while (0)
+
 extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_partial_int(const ctpwa::AuxArgs* a, const int* wptr,
                                                                                      const int* wblk, int nwave,
                                                                                      long long e0, long long n, double* out,
                                                                                      hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(ctpwa::k_partial_int, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, stream, *a, wptr, wblk,
-                       nwave, e0, n, out);
+    POST_LAUNCH(k_partial_int, 0, a->npol, n, *a, wptr, wblk, nwave, e0, n, out);
     return hipGetLastError();
 }
 
@@ -819,17 +873,15 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_partial
                                                                                      long long e0, long long n, double* out,
                                                                                      hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(ctpwa::k_partial_amp, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, stream, *a, wptr, wblk,
-                       nwave, e0, n, (double2*)out);
+    POST_LAUNCH(k_partial_amp, 4, a->npol, n, *a, wptr, wblk, nwave, e0, n, (double2*)out);
     return hipGetLastError();
 }
 
-extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs* a, long long e0, long long n, double* out, int intensity,
-                                        hipStream_t stream) {
+extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs* a, int nblock, long long e0,
+                                                                             long long n, double* out, int intensity,
+                                                                             hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    int bs = 128;
-    long long nb = (n + bs - 1) / bs;
-    if (intensity) hipLaunchKernelGGL(ctpwa::k_intensity, dim3((unsigned)nb), dim3(bs), 0, stream, *a, e0, n, out);
-    else hipLaunchKernelGGL(ctpwa::k_amplitudes, dim3((unsigned)nb), dim3(bs), 0, stream, *a, e0, n, out);
+    if (intensity) POST_LAUNCH(k_intensity, 0, a->npol, n, *a, nblock, e0, n, out);
+    else hipLaunchKernelGGL(ctpwa::k_amplitudes, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, stream, *a, e0, n, out);
     return hipGetLastError();
 }
