@@ -34,9 +34,9 @@ extern "C" hipError_t ctpwa_launch_to_mixed(const double2*, const double*, long 
                                              double*, float*, long long, long long, hipStream_t);
 extern "C" hipError_t ctpwa_launch_polsym(const double2*, long long, long long, long long, int, unsigned long long*,
                                           hipStream_t);
-extern "C" hipError_t ctpwa_launch_prep(const double*, double*, const ctpwa::PrepArgs*, int, int, hipStream_t);
+extern "C" hipError_t ctpwa_launch_prep(const double*, double*, const ctpwa::PrepArgs*, int, hipStream_t);
 extern "C" hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs*, unsigned int*, hipStream_t);
-extern "C" hipError_t ctpwa_launch_prep_batch(const double* const*, double* const*, const ctpwa::PrepArgs*, int,
+extern "C" hipError_t ctpwa_launch_prep_batch(const double* const*, double* const*, const ctpwa::PrepArgs*,
                                               const ctpwa::PrepArgs*, int, const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_finalize_batch(const ctpwa::FinArgs*, int, int, size_t, const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs*, int, long long, long long, double*, int, hipStream_t);
@@ -833,28 +833,7 @@ extern "C" int ctpwa_create(const char* plan_text, const double* phsp, long long
         h->prep = PrepArgs{d_blocks, d_res, d_nodes2, d_topos2, d_slcL, d_slc0, d_dens, d_amps,
                            (int)dens.size(), P.namp, P.nfree, P.ntheta,
                            (long long)M.off_v(), (long long)M.off_c(), (long long)M.off_rec(),
-                           (long long)M.off_th(), (long long)M.off_lth(), 0, nullptr, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        {
-            std::vector<char> blob;
-            auto put = [&](const void* p, size_t n) -> int {
-                size_t o = (blob.size() + 15) / 16 * 16;
-                blob.resize(o + (n + 15) / 16 * 16, 0);
-                if (n) std::memcpy(blob.data() + o, p, n);
-                return (int)o;
-            };
-            h->prep.o_blocks = put(blocks.data(), blocks.size() * sizeof(DBlock));
-            h->prep.o_res = put(res.data(), res.size() * sizeof(DRes));
-            h->prep.o_nodes = put(nodes.data(), nodes.size() * sizeof(DNode));
-            h->prep.o_topos = put(topos.data(), topos.size() * sizeof(DTopo));
-            h->prep.o_slcL = put(slcL.data(), slcL.size() * sizeof(int));
-            h->prep.o_slc0 = put(slc0.data(), slc0.size() * sizeof(int));
-            h->prep.o_dens = put(dens.data(), dens.size() * sizeof(DDen));
-            h->prep.o_amps = put(amps.data(), amps.size() * sizeof(DAmp));
-            if (blob.size() <= 48 * 1024) {
-                h->prep.meta = h->upload(blob);
-                h->prep.meta_bytes = (int)blob.size();
-            }
-        }
+                           (long long)M.off_th(), (long long)M.off_lth(), 0};
         h->fin = FinArgs{};
         h->fin.part = h->part;
         h->fin.nwg = h->nwg;
@@ -1027,7 +1006,7 @@ extern "C" int ctpwa_nll_grad(ctpwa_handle* h, const double* params_dev, double*
     if (!h || !params_dev || !out_dev) return fail("ctpwa_nll_grad: NULL argument");
     DeviceGuard g(h->device);
     hipStream_t s = (hipStream_t)stream;
-    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 2, s);
+    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, 2, s);
     if (e == hipSuccess) e = launch_custom(h, s);
     if (e == hipSuccess) e = launch_eval(h, s);
     if (e == hipSuccess) {
@@ -1050,7 +1029,7 @@ extern "C" int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev,
     double* scr = scratch_lookup(h->device);
     if (!scr) return fail("ctpwa_nll_grad_noalloc: no scratch address for this device");
     hipStream_t s = (hipStream_t)stream;
-    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 2, s);
+    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, 2, s);
     if (e == hipSuccess) e = launch_custom(h, s);
     if (e == hipSuccess) e = launch_eval(h, s, scr);
     if (e == hipSuccess) {
@@ -1460,7 +1439,7 @@ static void build_fixed_gram(ctpwa_handle* h) {
     // the table's coefficient records depend on theta only (none free): any couplings do
     double* p0 = h->upload(std::vector<double>((size_t)std::max(1, 2 * P.nfree), 0.0));
     double2* G = h->alloc<double2>((size_t)P.namp * P.namp);
-    HIPCHECK(ctpwa_launch_prep(p0, h->table, &h->prep, h->M.maxloc, 0, s));
+    HIPCHECK(ctpwa_launch_prep(p0, h->table, &h->prep, 0, s));
     HIPCHECK(launch_custom(h, s));
     class_gram(h, 0, 0, (double*)G, s);
     h->d_gram = G;
@@ -1474,7 +1453,7 @@ extern "C" int ctpwa_amplitude_gram(ctpwa_handle* h, const double* params_dev, i
     DeviceGuard g(h->device);
     hipStream_t s = (hipStream_t)stream;
     try {
-        HIPCHECK(ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 0, s));
+        HIPCHECK(ctpwa_launch_prep(params_dev, h->table, &h->prep, 0, s));
         HIPCHECK(launch_custom(h, s));
         class_gram(h, cls, 1, out_dev, s);
         return 0;
@@ -1488,7 +1467,7 @@ extern "C" int ctpwa_partial_intensities(ctpwa_handle* h, const double* params_d
     if (cls < 0 || cls > 2) return fail("ctpwa_partial_intensities: class must be 0 (phsp), 1 (data) or 2 (bkg)");
     DeviceGuard g(h->device);
     hipStream_t s = (hipStream_t)stream;
-    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 0, s);
+    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, 0, s);
     if (e == hipSuccess) e = launch_custom(h, s);
     if (e == hipSuccess)
         e = ctpwa_launch_partial_int(&h->aux, h->wave_ptr, h->wave_blk, h->M.P.nwave, h->off[cls], h->n[cls],
@@ -1502,7 +1481,7 @@ extern "C" int ctpwa_partial_amplitudes(ctpwa_handle* h, const double* params_de
     if (cls < 0 || cls > 2) return fail("ctpwa_partial_amplitudes: class must be 0 (phsp), 1 (data) or 2 (bkg)");
     DeviceGuard g(h->device);
     hipStream_t s = (hipStream_t)stream;
-    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 0, s);
+    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, 0, s);
     if (e == hipSuccess) e = launch_custom(h, s);
     if (e == hipSuccess)
         e = ctpwa_launch_partial_amp(&h->aux, h->wave_ptr, h->wave_blk, h->M.P.nwave, h->off[cls], h->n[cls],
@@ -1532,7 +1511,7 @@ extern "C" int ctpwa_hessian(ctpwa_handle* h, const double* params_dev, double* 
         const Model_& M = h->M;
         const Plan& P = M.P;
         const HessShape& S = h->hess.S;
-        HIPCHECK(ctpwa_launch_prep(params_dev, h->table, &h->prep, M.maxloc, 3, s));
+        HIPCHECK(ctpwa_launch_prep(params_dev, h->table, &h->prep, 3, s));
         if (h->fn_custom2) {
             void* args[] = {&h->table, &h->inv, &h->invf, &h->ntot, &h->cfb2};
             unsigned grid = (unsigned)std::min<long long>(16384, (h->ntot + 63) / 64);
@@ -1571,7 +1550,7 @@ static int aux_call(ctpwa_handle* h, const double* params_dev, int cls, double* 
     if (cls < 0 || cls > 2) return fail("event class must be 0, 1 or 2");
     DeviceGuard g(h->device);
     hipStream_t s = (hipStream_t)stream;
-    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 0, s);
+    hipError_t e = ctpwa_launch_prep(params_dev, h->table, &h->prep, 0, s);
     if (e == hipSuccess) e = launch_custom(h, s);
     if (e == hipSuccess && h->fn_aux) {
         // generated kernel of the model (Custom lineshapes)
@@ -1605,7 +1584,7 @@ extern "C" int ctpwa_time_eval_kernel(ctpwa_handle* h, const double* params_dev,
     std::vector<hipEvent_t> ev(2 * (size_t)iters, nullptr);
     hipError_t e = hipSuccess;
     for (size_t i = 0; i < ev.size() && e == hipSuccess; ++i) e = hipEventCreate(&ev[i]);
-    if (e == hipSuccess) e = ctpwa_launch_prep(params_dev, h->table, &h->prep, h->M.maxloc, 0, s);
+    if (e == hipSuccess) e = ctpwa_launch_prep(params_dev, h->table, &h->prep, 0, s);
     if (e == hipSuccess) e = launch_custom(h, s);
     for (int i = 0; i < iters && e == hipSuccess; ++i) {
         e = hipEventRecord(ev[2 * i], s);
@@ -1730,7 +1709,7 @@ static void batch_launches_graph(ctpwa_batch* b, const ctpwa_handle* h0, int row
     const int* d_hdr = (const int*)(b->dev + b->o_hdr);
     unsigned int* d_ctr = (unsigned int*)(b->dev + b->o_ctr);
     HIPCHECK(ctpwa_launch_prep_batch((const double* const*)(b->dev + b->o_params), (double* const*)(b->dev + b->o_tables),
-                                     &h0->prep, h0->M.maxloc, (const PrepArgs*)(b->dev + b->o_preps), rows, d_hdr, s));
+                                     &h0->prep, (const PrepArgs*)(b->dev + b->o_preps), rows, d_hdr, s));
     const EvalJob* d_jobs = (const EvalJob*)(b->dev + b->o_jobs);
     void* args[] = {&d_jobs, &d_hdr, &d_ctr};
     HIPCHECK(hipModuleLaunchKernel(h0->fn_group_p, b->persist, 1, 1, h0->M.wgs, 1, 1, 0, s, args, nullptr));
@@ -1818,7 +1797,7 @@ extern "C" int ctpwa_batch_nll_grad(ctpwa_batch* b, ctpwa_handle* const* hs, con
             // one batched prep launch, each job's Custom factors, one grouped launch whose
             // workgroups are shared out among the jobs, one batched reduction and assembly
             HIPCHECK(ctpwa_launch_prep_batch((const double* const*)(b->dev + b->o_params),
-                                             (double* const*)(b->dev + b->o_tables), &h0->prep, h0->M.maxloc, nullptr, n,
+                                             (double* const*)(b->dev + b->o_tables), &h0->prep, nullptr, n,
                                              nullptr, s));
             for (int j = 0; j < n; ++j) HIPCHECK(launch_custom(hs[j], s));
             const EvalJob* d_jobs = (const EvalJob*)(b->dev + b->o_jobs);

@@ -75,17 +75,7 @@ struct PrepArgs {
     long long off_th;        // theta values (read by Custom lineshapes in the fused kernel)
     long long off_lth;       // theta of the last NLL / Hessian evaluation (ctpwa_last_theta)
     int remember;            // this launch writes theta to off_lth as well
-    // the same tables packed in one blob (16-byte aligned sections) that the prep kernel
-    // copies to LDS before use; meta_bytes == 0: read the tables from global memory
-    const void* meta;
-    int meta_bytes;
-    int o_blocks, o_res, o_nodes, o_topos, o_slcL, o_slc0, o_dens, o_amps;
 };
-
-// dynamic LDS of the prep kernels: the staged model tables, then the parameter vector
-inline size_t prep_lds_bytes(const PrepArgs& a) {
-    return (size_t)a.meta_bytes + sizeof(double) * (size_t)(2 * a.nfree + a.ntheta);
-}
 
 // one term of a gradient contraction in the final assembly
 //   theta entries: idx >= 0  -> scale * dcoef * C[idx]          (propagator coefficient)

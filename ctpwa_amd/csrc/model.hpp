@@ -229,7 +229,6 @@ struct Model_ {
     std::vector<std::vector<int>> block_customs;  // [block] -> custom indices
     std::vector<CTerm> cterms;                    // Custom theta-gradient accumulators
     std::vector<double> tabs;                     // table lineshapes, concatenated
-    int maxloc = 0;
     // Propagators equal by construction (same kinematic node, lineshape and parameter
     // sources) within one wave group: den_canon[d] is the first of them.  The fused kernel
     // evaluates and accumulates the first only.
@@ -475,7 +474,6 @@ inline Model_ derive(const Plan& P) {
             for (int s : r.slots)
                 if (s >= 0 && std::find(vars.begin(), vars.end(), s) == vars.end()) vars.push_back(s);
         if ((int)vars.size() > Model_::NLOC) throw std::runtime_error("more than 8 free parameters in one block");
-        M.maxloc = std::max(M.maxloc, (int)vars.size());
         M.bvars.push_back(vars);
         std::vector<int> res_at(nn, -1);
         for (size_t r = 0; r < B.res.size(); ++r) {

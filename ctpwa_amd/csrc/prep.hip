@@ -3,8 +3,8 @@
 //  k_prep      params -> coefficient table: couplings v_a, c_a = v_a K_a, amplitude
 //              numerators K_a and every propagator-denominator coefficient, each with
 //              its first and second derivatives over the block's free parameters
-//              (forward-mode jets).  One thread per item; runs in microseconds.
-//  k_reduce, k_assemble  per-workgroup partial sums -> NLL and gradient in the fit-parameter
+//              (forward-mode jets).  One wave per item; runs in microseconds.
+//  k_finalize  per-workgroup partial sums -> NLL and gradient in the fit-parameter
 //              layout [Re p, Im p, theta], following the assembly of the reference's
 //              NLLFunction::forward/backward (src/Analysis.cu:1134-1261): phase-space
 //              mean, N_eff log term, NaN/Inf -> 1e30 with zero gradient, Gaussian
@@ -16,106 +16,77 @@
 namespace ctpwa {
 
 // ---------------------------------------------------------------------------
-// forward-mode jet over NV block-local variables: value, gradient and (when H)
-// Hessian.  NV is the smallest of 1/2/4/8 that holds the model's largest block, so
-// the jets stay in registers.
+// forward-mode jet over a block's NLOC = 8 local variables, spread over a wave: every lane
+// carries the value and the derivatives of one component, lane i d/dx_i, or with second
+// derivatives lane 8 i + k d/dx_i, d/dx_k and d2/dx_i dx_k.  An item is one chain of
+// dependent operations, and one thread with all components issued them one after the other
+// (149 amplitudes with second derivatives: 69 us, now 11 us).
 // ---------------------------------------------------------------------------
-template <int NV, bool H>
-struct DJ {
-    double v, g[NV], h[H ? NV : 1][H ? NV : 1];
-};
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jc(double c) {
-    DJ<NV, H> r;
-    r.v = c;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) r.g[i] = 0.0;
-    if constexpr (H) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) r.h[i][k] = 0.0;
-    }
+static_assert(NLOC == 8, "one wave holds the 8 x 8 second derivatives");
+template <bool H> struct DJ { double v, g, gk, h; };
+template <> struct DJ<false> { double v, g; };
+template <bool H> __device__ __forceinline__ int jet_i() { return H ? threadIdx.x >> 3 : threadIdx.x; }
+template <bool H>
+__device__ inline DJ<H> jc(double c) {
+    if constexpr (H) return {c, 0.0, 0.0, 0.0};
+    else return {c, 0.0};
+}
+template <bool H>
+__device__ inline DJ<H> jv(double c, int i) {
+    DJ<H> r = jc<H>(c);
+    r.g = jet_i<H>() == i ? 1.0 : 0.0;
+    if constexpr (H) r.gk = (int)(threadIdx.x & 7) == i ? 1.0 : 0.0;
     return r;
 }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jv(double c, int i) {
-    DJ<NV, H> r = jc<NV, H>(c);
-#pragma unroll
-    for (int k = 0; k < NV; ++k) if (k == i) r.g[k] = 1.0;
-    return r;
-}
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jadd(const DJ<NV, H>& a, const DJ<NV, H>& b) {
-    DJ<NV, H> r;
+template <bool H>
+__device__ inline DJ<H> jadd(const DJ<H>& a, const DJ<H>& b) {
+    DJ<H> r;
     r.v = a.v + b.v;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) r.g[i] = a.g[i] + b.g[i];
-    if constexpr (H) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) r.h[i][k] = a.h[i][k] + b.h[i][k];
-    }
+    r.g = a.g + b.g;
+    if constexpr (H) { r.gk = a.gk + b.gk; r.h = a.h + b.h; }
     return r;
 }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jscale(const DJ<NV, H>& a, double c) {
-    DJ<NV, H> r;
+template <bool H>
+__device__ inline DJ<H> jscale(const DJ<H>& a, double c) {
+    DJ<H> r;
     r.v = a.v * c;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) r.g[i] = a.g[i] * c;
-    if constexpr (H) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) r.h[i][k] = a.h[i][k] * c;
-    }
+    r.g = a.g * c;
+    if constexpr (H) { r.gk = a.gk * c; r.h = a.h * c; }
     return r;
 }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jsub(const DJ<NV, H>& a, const DJ<NV, H>& b) { return jadd(a, jscale(b, -1.0)); }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jmul(const DJ<NV, H>& a, const DJ<NV, H>& b) {
-    DJ<NV, H> r;
+template <bool H>
+__device__ inline DJ<H> jsub(const DJ<H>& a, const DJ<H>& b) { return jadd(a, jscale(b, -1.0)); }
+template <bool H>
+__device__ inline DJ<H> jmul(const DJ<H>& a, const DJ<H>& b) {
+    DJ<H> r;
     r.v = a.v * b.v;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) r.g[i] = a.g[i] * b.v + a.v * b.g[i];
+    r.g = a.g * b.v + a.v * b.g;
     if constexpr (H) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int k = 0; k < NV; ++k)
-                r.h[i][k] = a.h[i][k] * b.v + a.v * b.h[i][k] + a.g[i] * b.g[k] + a.g[k] * b.g[i];
+        r.gk = a.gk * b.v + a.v * b.gk;
+        r.h = a.h * b.v + a.v * b.h + a.g * b.gk + a.gk * b.g;
     }
     return r;
 }
 // f(a) given f, f', f''
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jfun(const DJ<NV, H>& a, double f, double d1, double d2) {
-    DJ<NV, H> r;
+template <bool H>
+__device__ inline DJ<H> jfun(const DJ<H>& a, double f, double d1, double d2) {
+    DJ<H> r;
     r.v = f;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) r.g[i] = d1 * a.g[i];
-    if constexpr (H) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) r.h[i][k] = d1 * a.h[i][k] + d2 * a.g[i] * a.g[k];
-    }
+    r.g = d1 * a.g;
+    if constexpr (H) { r.gk = d1 * a.gk; r.h = d1 * a.h + d2 * a.g * a.gk; }
     return r;
 }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jinv(const DJ<NV, H>& a) { double x = a.v; return jfun(a, 1.0 / x, -1.0 / (x * x), 2.0 / (x * x * x)); }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jdiv(const DJ<NV, H>& a, const DJ<NV, H>& b) { return jmul(a, jinv(b)); }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jsqrt(const DJ<NV, H>& a) { double s = sqrt(a.v); return jfun(a, s, 0.5 / s, -0.25 / (s * a.v)); }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jlog(const DJ<NV, H>& a) { return jfun(a, log(a.v), 1.0 / a.v, -1.0 / (a.v * a.v)); }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jpowi(const DJ<NV, H>& a, int n) {
-    if (n == 0) return jc<NV, H>(1.0);
+template <bool H>
+__device__ inline DJ<H> jinv(const DJ<H>& a) { double x = a.v; return jfun(a, 1.0 / x, -1.0 / (x * x), 2.0 / (x * x * x)); }
+template <bool H>
+__device__ inline DJ<H> jdiv(const DJ<H>& a, const DJ<H>& b) { return jmul(a, jinv(b)); }
+template <bool H>
+__device__ inline DJ<H> jsqrt(const DJ<H>& a) { double s = sqrt(a.v); return jfun(a, s, 0.5 / s, -0.25 / (s * a.v)); }
+template <bool H>
+__device__ inline DJ<H> jlog(const DJ<H>& a) { return jfun(a, log(a.v), 1.0 / a.v, -1.0 / (a.v * a.v)); }
+template <bool H>
+__device__ inline DJ<H> jpowi(const DJ<H>& a, int n) {
+    if (n == 0) return jc<H>(1.0);
     if (n == 1) return a;
     double x = a.v, xn2 = 1.0;
     for (int i = 0; i < n - 2; ++i) xn2 *= x;
@@ -123,8 +94,8 @@ __device__ inline DJ<NV, H> jpowi(const DJ<NV, H>& a, int n) {
     return jfun(a, xn, n * xn1, n * (n - 1.0) * xn2);
 }
 // N_L(z) with z = q0 d as a jet in q0
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jbfpoly(int L, const DJ<NV, H>& q0, double d) {
+template <bool H>
+__device__ inline DJ<H> jbfpoly(int L, const DJ<H>& q0, double d) {
     double c[7];
     int deg = 0;
     switch (L) {
@@ -134,140 +105,128 @@ __device__ inline DJ<NV, H> jbfpoly(int L, const DJ<NV, H>& q0, double d) {
     case 4: c[0] = 11025; c[1] = 1575; c[2] = 135; c[3] = 10; c[4] = 1; deg = 4; break;
     case 5: c[0] = 893025; c[1] = 99225; c[2] = 6300; c[3] = 315; c[4] = 15; c[5] = 1; deg = 5; break;
     case 6: c[0] = 540326025; c[1] = 6185025; c[2] = 363825; c[3] = 17325; c[4] = 630; c[5] = 21; c[6] = 1; deg = 6; break;
-    default: return jc<NV, H>(1.0);
+    default: return jc<H>(1.0);
     }
-    DJ<NV, H> z = jscale(q0, d);
-    DJ<NV, H> z2 = jmul(z, z);
-    DJ<NV, H> r = jc<NV, H>(c[deg]);          // Horner in z^2
-    for (int i = deg - 1; i >= 0; --i) r = jadd(jmul(r, z2), jc<NV, H>(c[i]));
+    DJ<H> z = jscale(q0, d);
+    DJ<H> z2 = jmul(z, z);
+    DJ<H> r = jc<H>(c[deg]);          // Horner in z^2
+    for (int i = deg - 1; i >= 0; --i) r = jadd(jmul(r, z2), jc<H>(c[i]));
     return r;
 }
 // breakup momentum (src/AmpGen.cu:2733-2737) and computeQ0AD (include/ResModel.cuh:88-97)
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jbreakup(const DJ<NV, H>& m, const DJ<NV, H>& m1, const DJ<NV, H>& m2) {
-    DJ<NV, H> s = jadd(m1, m2), d = jsub(m1, m2);
-    DJ<NV, H> mm = jmul(m, m);
-    DJ<NV, H> q2 = jmul(jsub(mm, jmul(s, s)), jsub(mm, jmul(d, d)));
-    if (q2.v <= 0.0) return jc<NV, H>(0.0);
+template <bool H>
+__device__ inline DJ<H> jbreakup(const DJ<H>& m, const DJ<H>& m1, const DJ<H>& m2) {
+    DJ<H> s = jadd(m1, m2), d = jsub(m1, m2);
+    DJ<H> mm = jmul(m, m);
+    DJ<H> q2 = jmul(jsub(mm, jmul(s, s)), jsub(mm, jmul(d, d)));
+    if (q2.v <= 0.0) return jc<H>(0.0);
     return jdiv(jsqrt(q2), jscale(m, 2.0));
 }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> jq0ad(const DJ<NV, H>& m0, const DJ<NV, H>& m1, const DJ<NV, H>& m2) {
-    DJ<NV, H> s = jadd(m1, m2), d = jsub(m1, m2);
-    DJ<NV, H> m0s = jmul(m0, m0);
-    DJ<NV, H> q2 = jdiv(jmul(jsub(m0s, jmul(s, s)), jsub(m0s, jmul(d, d))), jscale(m0s, 4.0));
-    if (q2.v < 0.0) return jc<NV, H>(0.0);
+template <bool H>
+__device__ inline DJ<H> jq0ad(const DJ<H>& m0, const DJ<H>& m1, const DJ<H>& m2) {
+    DJ<H> s = jadd(m1, m2), d = jsub(m1, m2);
+    DJ<H> m0s = jmul(m0, m0);
+    DJ<H> q2 = jdiv(jmul(jsub(m0s, jmul(s, s)), jsub(m0s, jmul(d, d))), jscale(m0s, 4.0));
+    if (q2.v < 0.0) return jc<H>(0.0);
     return jsqrt(q2);
 }
 
-__device__ inline int local_index(const DBlock& B, int slot) {
+// a model table in the constant address space (nothing writes it while a kernel reads it)
+#define CTAB(T) __attribute__((address_space(4))) T
+__device__ inline int local_index(const CTAB(DBlock)& B, int slot) {
     for (int i = 0; i < B.nloc; ++i) if (B.vars[i] == slot) return i;
     return -1;
 }
-template <int NV, bool H>
-__device__ inline DJ<NV, H> res_param(const DRes& R, int p, const DBlock& B, const double* theta) {
-    if (p >= R.np) return jc<NV, H>(0.0);
+template <bool H>
+__device__ inline DJ<H> res_param(const CTAB(DRes)& R, int p, const CTAB(DBlock)& B, const double* theta) {
+    if (p >= R.np) return jc<H>(0.0);
     int s = R.slot[p];
-    if (s < 0) return jc<NV, H>(R.p[p]);
-    return jv<NV, H>(theta[s], local_index(B, s));
+    if (s < 0) return jc<H>(R.p[p]);
+    return jv<H>(theta[s], local_index(B, s));
 }
 // mass used in q0 for a daughter: configured mass, else the mass parameter of the
 // block's resonance that occupies it (src/AmpGen.cu:1664-1731)
-template <int NV, bool H>
-__device__ inline DJ<NV, H> q0_dmass(double cfg, int ref, const DBlock& B, const DRes* res, const double* theta) {
-    if (cfg > 0) return jc<NV, H>(cfg);
+template <bool H>
+__device__ inline DJ<H> q0_dmass(double cfg, int ref, const CTAB(DBlock)& B, const CTAB(DRes)* res, const double* theta) {
+    if (cfg > 0) return jc<H>(cfg);
     // a final-state particle configured with mass 0: the reference falls back to the
     // event mass here, which is 0 for a massless particle (up to rounding)
-    if (ref >= 0) return jc<NV, H>(0.0);
+    if (ref >= 0) return jc<H>(0.0);
     int kk = -ref - 1;
     for (int r = 0; r < B.nres; ++r) {
-        const DRes& R = res[B.res0 + r];
-        if (R.node == kk && R.np > 0) return res_param<NV, H>(R, 0, B, theta);
+        const CTAB(DRes)& R = res[B.res0 + r];
+        if (R.node == kk && R.np > 0) return res_param<H>(R, 0, B, theta);
     }
-    return jc<NV, H>(1.0);   // unreachable: the host rejects event-dependent q0
+    return jc<H>(1.0);   // unreachable: the host rejects event-dependent q0
 }
-template <int NV, bool H>
-__device__ inline void store(double* t, const DJ<NV, H>& x) {
-    t[0] = x.v;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) t[1 + i] = x.g[i];
-    if constexpr (H) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int k = 0; k < NV; ++k) t[1 + NLOC + i * NLOC + k] = x.h[i][k];
-    }
+// the wave's lanes hold the record's components side by side
+template <bool H>
+__device__ inline void store(double* t, const DJ<H>& x) {
+    const int lane = threadIdx.x;
+    if (lane == 0) t[0] = x.v;
+    if (H ? (lane & 7) == 0 : lane < NLOC) t[1 + jet_i<H>()] = x.g;
+    if constexpr (H) t[1 + NLOC + lane] = x.h;
 }
 
-template <int NV, bool H>
+template <bool H>
 __device__ __forceinline__ void prep_body(const double* __restrict__ gparams, double* __restrict__ table, PrepArgs a) {
-    using J = DJ<NV, H>;
-    extern __shared__ uint4 smeta[];
-    // the parameter vector goes to LDS behind the model tables (meta_bytes is a multiple of
-    // 16), loaded in the same phase as the tables, so the item's chain starts with both
-    // in LDS instead of waiting for a dependent global load of its parameters
-    double* params = (double*)((char*)smeta + a.meta_bytes);
-    for (int i = threadIdx.x; i < 2 * a.nfree + a.ntheta; i += blockDim.x) params[i] = gparams[i];
-    if (a.meta_bytes > 0) {
-        // the model tables are read many times with dependent indices: stage them in LDS
-        const uint4* src = (const uint4*)a.meta;
-        for (int i = threadIdx.x; i < a.meta_bytes / 16; i += blockDim.x) smeta[i] = src[i];
-        const char* base = (const char*)smeta;
-        a.blocks = (const DBlock*)(base + a.o_blocks);
-        a.res = (const DRes*)(base + a.o_res);
-        a.nodes = (const DNode*)(base + a.o_nodes);
-        a.topos = (const DTopo*)(base + a.o_topos);
-        a.slcL = (const int*)(base + a.o_slcL);
-        a.slc0 = (const int*)(base + a.o_slc0);
-        a.dens = (const DDen*)(base + a.o_dens);
-        a.amps = (const DAmp*)(base + a.o_amps);
-    }
-    __syncthreads();
+    using J = DJ<H>;
+    // the model's tables are read with wave-uniform, dependent indices: scalar loads.  (Each
+    // workgroup copying all tables to LDS first took 21 us at 149 amplitudes, this 11 us; 8 us
+    // at 10 amplitudes either way, which is the launch and cold instruction and table reads.)
+    const double* params = gparams;
+    const CTAB(DBlock)* blocks = (const CTAB(DBlock)*)a.blocks;
+    const CTAB(DRes)* res = (const CTAB(DRes)*)a.res;
+    const CTAB(DNode)* nodes = (const CTAB(DNode)*)a.nodes;
+    const CTAB(DTopo)* topos = (const CTAB(DTopo)*)a.topos;
+    const CTAB(DDen)* dens = (const CTAB(DDen)*)a.dens;
+    const CTAB(DAmp)* amps = (const CTAB(DAmp)*)a.amps;
+    const CTAB(int)* slcL = (const CTAB(int)*)a.slcL;
+    const CTAB(int)* slc0 = (const CTAB(int)*)a.slc0;
     // one item (denominator or amplitude record) per workgroup: the items' chains of
     // dependent jet arithmetic then run on different compute units at the same time instead
     // of one after another in a single divergent wave
     int item = blockIdx.x;
-    const double* theta = params + 2 * a.nfree;
+    const double* __restrict__ theta = params + 2 * a.nfree;
     if (blockIdx.x == 0)
         for (int j = threadIdx.x; j < a.ntheta; j += blockDim.x) {
             table[a.off_th + j] = theta[j];
             if (a.remember) table[a.off_lth + j] = theta[j];
         }
-    if (threadIdx.x != 0) return;
     if (item < a.nden) {
-        const DDen& D = a.dens[item];
-        const DBlock& B = a.blocks[D.block];
-        const DRes& R = a.res[B.res0 + D.res];
-        const DTopo& T = a.topos[B.topo];
-        const DNode& n = a.nodes[T.node0 + R.node];
-        J m0 = (R.np > 0) ? res_param<NV, H>(R, 0, B, theta) : jc<NV, H>(1.0);
-        J q0 = jq0ad(m0, q0_dmass<NV, H>(n.md1, n.d1ref, B, a.res, theta), q0_dmass<NV, H>(n.md2, n.d2ref, B, a.res, theta));
+        const CTAB(DDen)& D = dens[item];
+        const CTAB(DBlock)& B = blocks[D.block];
+        const CTAB(DRes)& R = res[B.res0 + D.res];
+        const CTAB(DTopo)& T = topos[B.topo];
+        const CTAB(DNode)& n = nodes[T.node0 + R.node];
+        J m0 = (R.np > 0) ? res_param<H>(R, 0, B, theta) : jc<H>(1.0);
+        J q0 = jq0ad(m0, q0_dmass<H>(n.md1, n.d1ref, B, res, theta), q0_dmass<H>(n.md2, n.d2ref, B, res, theta));
         double* t = table + a.off_rec + (long long)D.rec * REC;
         J m02 = jmul(m0, m0);
         switch (R.model) {
         case 0: {   // BWR: D = m0^2 - s - i g0 m0^2 N_L(q0 d')/q0^(2L+1) * E
-            J g0 = res_param<NV, H>(R, 1, B, theta);
+            J g0 = res_param<H>(R, 1, B, theta);
             double dp = n.has_bf ? n.bf_d : 0.0;
-            J N0 = (dp != 0.0) ? jbfpoly(n.lmin, q0, dp) : jc<NV, H>(1.0);
+            J N0 = (dp != 0.0) ? jbfpoly(n.lmin, q0, dp) : jc<H>(1.0);
             J b = jdiv(jmul(jmul(g0, m02), N0), jpowi(q0, 2 * n.lmin + 1));
             store(t, m02);
             store(t + REC, b);
             break;
         }
         case 1: {   // BW: D = m0^2 - s - i m0 g0
-            J g0 = res_param<NV, H>(R, 1, B, theta);
+            J g0 = res_param<H>(R, 1, B, theta);
             store(t, m02);
             store(t + REC, jmul(m0, g0));
             break;
         }
         case 3: {   // Flatte: D = m0^2 - s + sum b_i rho_im,i - i sum b_i rho_re,i, b_i = m0 g_i / 2
             store(t, m02);
-            for (int i = 0; i < R.nch; ++i) store(t + (1 + i) * REC, jscale(jmul(m0, res_param<NV, H>(R, 1 + i, B, theta)), 0.5));
+            for (int i = 0; i < R.nch; ++i) store(t + (1 + i) * REC, jscale(jmul(m0, res_param<H>(R, 1 + i, B, theta)), 0.5));
             break;
         }
         case 4: {   // Gounaris-Sakurai (src/ResModel.cu:484-561)
             const double pi = 3.14159265358979323846;
-            J g0 = res_param<NV, H>(R, 1, B, theta);
+            J g0 = res_param<H>(R, 1, B, theta);
             double mpi = R.nch > 0 ? R.ch[0] : 0.1396;
             J q02 = jmul(q0, q0), q03 = jmul(q02, q0);
             J logA = jlog(jscale(jadd(m0, jscale(q0, 2.0)), 1.0 / (2.0 * mpi)));
@@ -275,7 +234,7 @@ __device__ __forceinline__ void prep_body(const double* __restrict__ gparams, do
             J dh0 = jadd(jmul(h0, jsub(jinv(jscale(q02, 8.0)), jinv(jscale(m02, 2.0)))), jinv(jscale(m02, 2.0 * pi)));
             J c1 = jdiv(jmul(g0, m02), q03);
             J c3 = jdiv(jmul(jmul(g0, m02), dh0), q0);
-            J one_c3 = jadd(jc<NV, H>(1.0), c3);
+            J one_c3 = jadd(jc<H>(1.0), c3);
             store(t, jmul(one_c3, m02));
             store(t + REC, jscale(one_c3, -1.0));
             store(t + 2 * REC, c1);
@@ -288,42 +247,43 @@ __device__ __forceinline__ void prep_body(const double* __restrict__ gparams, do
     }
     item -= a.nden;
     if (item >= a.namp) return;
-    const DAmp& A = a.amps[item];
-    const DBlock& B = a.blocks[A.block];
-    const DTopo& T = a.topos[B.topo];
-    const int* Ls = a.slcL + (long long)(a.slc0[B.topo] + A.slc) * MAXNODE;
-    J K = jc<NV, H>(1.0);
+    const CTAB(DAmp)& A = amps[item];
+    const CTAB(DBlock)& B = blocks[A.block];
+    const CTAB(DTopo)& T = topos[B.topo];
+    const CTAB(int)* Ls = slcL + (long long)(slc0[B.topo] + A.slc) * MAXNODE;
+    J K = jc<H>(1.0);
     for (int k = 0; k < T.nn; ++k) {
-        const DNode& n = a.nodes[T.node0 + k];
+        const CTAB(DNode)& n = nodes[T.node0 + k];
         int L = Ls[k];
         int r = -1;
-        for (int i = 0; i < B.nres; ++i) if (a.res[B.res0 + i].node == k) { r = i; break; }
-        J m1 = q0_dmass<NV, H>(n.md1, n.d1ref, B, a.res, theta), m2 = q0_dmass<NV, H>(n.md2, n.d2ref, B, a.res, theta);
+        for (int i = 0; i < B.nres; ++i) if (res[B.res0 + i].node == k) { r = i; break; }
+        J m1 = q0_dmass<H>(n.md1, n.d1ref, B, res, theta), m2 = q0_dmass<H>(n.md2, n.d2ref, B, res, theta);
         if (k == 0 || r < 0) {
             if (n.has_bf && L >= 1 && L <= 6) {
-                J q0 = jbreakup(jc<NV, H>(n.mm > 0 ? n.mm : 1.0), m1, m2);
+                J q0 = jbreakup(jc<H>(n.mm > 0 ? n.mm : 1.0), m1, m2);
                 K = jmul(K, jsqrt(jbfpoly(L, q0, n.bf_d)));
             }
             continue;
         }
-        const DRes& R = a.res[B.res0 + r];
+        const CTAB(DRes)& R = res[B.res0 + r];
         // BW, Custom and the table lineshapes (Hist, Interp) carry no automatic barrier
         if (R.model == 1 || R.model == 5 || R.model == 6 || R.model == 7) continue;
-        J m0 = (R.np > 0) ? res_param<NV, H>(R, 0, B, theta) : jc<NV, H>(1.0);
+        J m0 = (R.np > 0) ? res_param<H>(R, 0, B, theta) : jc<H>(1.0);
         J q0 = jq0ad(m0, m1, m2);
         if (n.has_bf && L >= 1 && L <= 6) K = jmul(K, jsqrt(jbfpoly(L, q0, n.bf_d)));
         if (R.model == 4) {                                // GS numerator 1 + d(m0) g0 / m0
             const double pi = 3.14159265358979323846;
-            J g0 = res_param<NV, H>(R, 1, B, theta);
+            J g0 = res_param<H>(R, 1, B, theta);
             double mpi = R.nch > 0 ? R.ch[0] : 0.1396;
             J q02 = jmul(q0, q0), q03 = jmul(q02, q0);
             J logA = jlog(jscale(jadd(m0, jscale(q0, 2.0)), 1.0 / (2.0 * mpi)));
-            J dv = jadd(jsub(jmul(jscale(jdiv(jc<NV, H>(mpi * mpi), q02), 3.0 / pi), logA), jmul(jc<NV, H>(mpi * mpi / pi), jdiv(m0, q03))),
+            J dv = jadd(jsub(jmul(jscale(jdiv(jc<H>(mpi * mpi), q02), 3.0 / pi), logA), jmul(jc<H>(mpi * mpi / pi), jdiv(m0, q03))),
                          jdiv(m0, jscale(q0, 2.0 * pi)));
-            K = jmul(K, jadd(jc<NV, H>(1.0), jdiv(jmul(dv, g0), m0)));
+            K = jmul(K, jadd(jc<H>(1.0), jdiv(jmul(dv, g0), m0)));
         }
     }
     store(table + a.off_rec + (long long)A.rec * REC, K);
+    if (threadIdx.x != 0) return;
     double pr = params[A.freeidx] * A.ratio, pi_ = params[a.nfree + A.freeidx] * A.ratio;
     table[a.off_v + 2 * item] = pr;
     table[a.off_v + 2 * item + 1] = pi_;
@@ -331,14 +291,13 @@ __device__ __forceinline__ void prep_body(const double* __restrict__ gparams, do
     table[a.off_c + 2 * item + 1] = pi_ * K.v;
 }
 
-template <int NV, bool H>
+template <bool H>
 __global__ void __launch_bounds__(64) k_prep(const double* __restrict__ params, double* __restrict__ table, PrepArgs a) {
-    prep_body<NV, H>(params, table, a);
+    prep_body<H>(params, table, a);
 }
 
 // many likelihoods of one model: blockIdx.y selects the likelihood (its parameters and
 // coefficient table); the model tables in `a` are the same for all of them
-template <int NV, bool H>
 // one workgroup row per job.  hdr (graph replays; NULL otherwise): hdr[0] is the number
 // of jobs, rows at or beyond it leave at once, and each job's prep arguments come from
 // args[row] (its own handle's model tables) instead of `a`
@@ -347,7 +306,7 @@ __global__ void __launch_bounds__(64) k_prep_batch(const double* const* __restri
     if (hdr && (int)blockIdx.y >= hdr[0]) return;
     if (args) a = args[blockIdx.y];
     a.remember = 1;                 // NLL evaluations: each table keeps its theta as the last evaluated one
-    prep_body<NV, H>(params[blockIdx.y], tables[blockIdx.y], a);
+    prep_body<false>(params[blockIdx.y], tables[blockIdx.y], a);
 }
 
 // ---------------------------------------------------------------------------
@@ -355,21 +314,22 @@ __global__ void __launch_bounds__(64) k_prep_batch(const double* const* __restri
 // ---------------------------------------------------------------------------
 
 constexpr int RED_THREADS = 256;
-constexpr int ASM_THREADS = 256;
+constexpr int ASM_THREADS = 1024;
 
-// this thread's share of class c's total of accumulator column col: the class's
+// this lane's share of class c's total of accumulator column col: the class's
 // workgroup partials in a fixed order, or, for the phase space with a stored Gram (no free
 // resonance parameter), the column from G and c_a = v_a K_a:
 //   col 0: sum_a Re(conj(c_a) (G c)_a) = sum_e I(e);  col 1 + 2a / 2 + 2a: Re / Im (G c)_a
-// (sum_e conj(Psi_a sl_a) S, the fused kernel's accX_a); a tree sum over the workgroup
-// follows, so the result does not depend on timing
+// (sum_e conj(Psi_a sl_a) S, the fused kernel's accX_a); a butterfly over the wave follows, so
+// the result depends neither on timing nor on the kernel that sums
 __device__ __forceinline__ double class_share(const FinArgs& f, int c, int col) {
-    double s = 0.0;
+    const int lane = threadIdx.x & 63;
     if (c == 0 && f.gram) {
+        double s = 0.0;
         const int n = f.namp;
         const double2* cv = (const double2*)(f.table + f.off_c);
         if (col == 0) {
-            for (int a = threadIdx.x; a < n; a += RED_THREADS) {
+            for (int a = lane; a < n; a += 64) {
                 double gr = 0.0, gi = 0.0;
                 for (int b = 0; b < n; ++b) {
                     const double2 G = f.gram[(long long)a * n + b], cb = cv[b];
@@ -381,51 +341,42 @@ __device__ __forceinline__ double class_share(const FinArgs& f, int c, int col) 
             }
         } else {
             const int a = (col - 1) >> 1, im = (col - 1) & 1;
-            for (int b = threadIdx.x; b < n; b += RED_THREADS) {
+            for (int b = lane; b < n; b += 64) {
                 const double2 G = f.gram[(long long)a * n + b], cb = cv[b];
                 s += im ? (G.x * cb.y + G.y * cb.x) : (G.x * cb.x - G.y * cb.y);
             }
         }
         return s;
     }
+    // four loads in flight per lane
     const double* src = f.part + (long long)col * f.nwg;
-    for (int g = f.g0[c] + threadIdx.x; g < f.g1[c]; g += RED_THREADS) s += src[g];
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    int g = f.g0[c] + lane;
+    for (; g + 192 < f.g1[c]; g += 256) {
+        s0 += src[g];
+        s1 += src[g + 64];
+        s2 += src[g + 128];
+        s3 += src[g + 192];
+    }
+    for (; g < f.g1[c]; g += 64) s0 += src[g];
+    return (s0 + s1) + (s2 + s3);
+}
+// the wave's (class, column) pair of the totals, the sum in every lane
+__device__ __forceinline__ double pair_total(const FinArgs& f, int pair) {
+    const int c = pair / f.nacc, col = pair - c * f.nacc;
+    double s = class_share(f, c, col);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     return s;
 }
 
-// fixed-order sum over a workgroup of RED_THREADS threads, valid in thread 0: a butterfly
-// within each wave (lane 0 always adds in the same order), then the wave sums in wave order
-// through LDS (one barrier instead of one per tree level)
-__device__ __forceinline__ double wg_sum(double v, double* sh) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double t = 0.0;
-    if (threadIdx.x == 0) {
-        t = sh[0];
-        for (int k = 1; k < RED_THREADS / 64; ++k) t += sh[k];
-    }
-    return t;
-}
-
-// stage 1: one workgroup per (class, accumulator column); fixed summation order
-__global__ void __launch_bounds__(RED_THREADS) k_reduce(FinArgs f) {
-    __shared__ double sh[RED_THREADS / 64];
-    int pair = blockIdx.x;
-    int c = pair / f.nacc, col = pair - c * f.nacc;
-    const double tot = wg_sum(class_share(f, c, col), sh);
-    if (threadIdx.x == 0) f.totals[pair] = tot;
-}
-
+// stage 1: one wave per (class, accumulator column); fixed summation order
 __global__ void __launch_bounds__(RED_THREADS) k_reduce_batch(const FinArgs* __restrict__ fins, const int* __restrict__ hdr) {
     if (hdr && (int)blockIdx.y >= hdr[0]) return;
     const FinArgs& f = fins[blockIdx.y];
-    if ((int)blockIdx.x >= 3 * f.nacc) return;      // the whole workgroup leaves together
-    __shared__ double sh[RED_THREADS / 64];
-    int pair = blockIdx.x;
-    int c = pair / f.nacc, col = pair - c * f.nacc;
-    const double tot = wg_sum(class_share(f, c, col), sh);
-    if (threadIdx.x == 0) f.totals[pair] = tot;
+    const int pair = blockIdx.x * (RED_THREADS / 64) + (threadIdx.x >> 6);
+    if (pair >= 3 * f.nacc) return;
+    const double tot = pair_total(f, pair);
+    if ((threadIdx.x & 63) == 0) f.totals[pair] = tot;
 }
 
 // stage 2: NLL and gradient from the class totals.  Every global read happens first, in
@@ -478,7 +429,9 @@ __device__ __forceinline__ void assemble_prefill(const FinArgs& f) {
     for (int k = tid; k <= f.nfree; k += ASM_THREADS) L.cpp[k] = f.cpp[k];
     for (int k = tid; k <= f.ntheta; k += ASM_THREADS) L.thp[k] = f.thp[k];
 }
-// the assembly proper, after assemble_prefill and a barrier
+// the assembly proper, after assemble_prefill and a barrier; SHARED: the totals come from other
+// workgroups of this launch (coherent loads)
+template <bool SHARED>
 __device__ __forceinline__ void assemble_main(const FinArgs& f) {
     const AsmLds L = asm_lds(f);
     double* C = L.C;
@@ -491,15 +444,17 @@ __device__ __forceinline__ void assemble_main(const FinArgs& f) {
     const int* cpp = L.cpp;
     const int* thp = L.thp;
     int tid = threadIdx.x;
-    const double* tot = f.totals;            // tot[c * nacc + col]
+    auto tot = [&](int i) {                  // i = c * nacc + col
+        return SHARED ? __hip_atomic_load(f.totals + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : f.totals[i];
+    };
     double Np = f.Np, Neff = f.Wd - f.Wb;
-    double pf = (Np > 0) ? tot[0] / Np : 0.0;
+    double pf = (Np > 0) ? tot(0) / Np : 0.0;
     if (!(pf > 1e-30) || isinf(pf)) pf = 1e-30;
     double cp = (Np > 0) ? Neff / (pf * Np) : 0.0;
     const double* theta = f.params + 2 * f.nfree;
     for (int col = tid; col < f.nacc; col += ASM_THREADS)
-        C[col] = -tot[f.nacc + col] + tot[2 * f.nacc + col] + cp * tot[col];
-    double loss = -tot[f.nacc] + tot[2 * f.nacc] + Neff * log(pf);
+        C[col] = -tot(f.nacc + col) + tot(2 * f.nacc + col) + cp * tot(col);
+    double loss = -tot(f.nacc) + tot(2 * f.nacc) + Neff * log(pf);
     for (int g = 0; g < f.ngauss; ++g) {
         double d = theta[f.g_slot[g]] - f.g_mu[g];
         loss += d * d / (2.0 * f.g_sig[g] * f.g_sig[g]);
@@ -546,34 +501,32 @@ __device__ __forceinline__ void assemble_main(const FinArgs& f) {
 __device__ __forceinline__ void assemble_body(const FinArgs& f) {
     assemble_prefill(f);
     __syncthreads();
-    assemble_main(f);
+    assemble_main<false>(f);
 }
 
-__global__ void __launch_bounds__(ASM_THREADS) k_assemble(FinArgs f) { assemble_body(f); }
-
-// k_reduce and k_assemble in one launch: every workgroup sums one (class, accumulator)
-// over the class's workgroup partials (the order of k_reduce), and the workgroup that
-// finishes last, found by a device-scope counter, runs the assembly on the totals and
-// resets the counter for the next evaluation.  Results are those of the two kernels.
-static_assert(RED_THREADS == ASM_THREADS, "one workgroup size for both parts");
+// Reduction and assembly in one launch: every wave sums one (class, accumulator) over the
+// class's workgroup partials, and the workgroup that finishes last, found by a device-scope
+// counter, runs the assembly on the totals and resets the counter for the next evaluation.
+// Bound by latency: cold reads of the partials and tables, and the handover.  Sixteen waves to
+// a workgroup (one workgroup and one count per sum, each with the assembly's inputs, took
+// 37 us at 149 amplitudes, 11 us at 10; now 12 and 9); the totals go through coherent stores and loads
+// and a wait instead of agent-scope fences, which write back and invalidate the L2 cache.
 __global__ void __launch_bounds__(ASM_THREADS) k_finalize(FinArgs f, unsigned int* __restrict__ done) {
-    __shared__ double sh[RED_THREADS / 64];
     __shared__ int last;
-    const int pair = blockIdx.x;
-    const int c = pair / f.nacc, col = pair - c * f.nacc;
+    const int pair = blockIdx.x * (ASM_THREADS / 64) + (threadIdx.x >> 6);
     // the assembly's inputs that need no totals, loaded by every workgroup while its
     // reduction loads are in flight (any workgroup may turn out to be the last)
     assemble_prefill(f);
-    const double tot = wg_sum(class_share(f, c, col), sh);
-    if (threadIdx.x == 0) {
-        f.totals[pair] = tot;
-        __threadfence();                                   // the total is visible before the count
-        last = atomicAdd(done, 1u) == gridDim.x - 1;
+    if (pair < 3 * f.nacc) {
+        const double tot = pair_total(f, pair);
+        if ((threadIdx.x & 63) == 0) __hip_atomic_store(f.totals + pair, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's total is visible before the count
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(done, 1u) == gridDim.x - 1;
     __syncthreads();
     if (!last) return;
-    __threadfence();                                       // every total is visible to this workgroup
-    assemble_main(f);
+    assemble_main<true>(f);
     if (threadIdx.x == 0) *done = 0u;
 }
 
@@ -777,36 +730,24 @@ __global__ void __launch_bounds__(64) k_intensity(AuxArgs a, int nblock, long lo
 
 }  // namespace ctpwa
 
-template <int NV, bool H>
+template <bool H>
 static hipError_t launch_prep_t(const double* params, double* table, const ctpwa::PrepArgs* a, int remember,
                                 hipStream_t stream) {
     int items = a->nden + a->namp;
     ctpwa::PrepArgs b = *a;
     b.remember = remember;
-    hipLaunchKernelGGL((ctpwa::k_prep<NV, H>), dim3(items), dim3(64), ctpwa::prep_lds_bytes(*a), stream, params, table, b);
+    hipLaunchKernelGGL((ctpwa::k_prep<H>), dim3(items), dim3(64), 0, stream, params, table, b);
     return hipGetLastError();
 }
 
-// nv: largest number of free parameters in one block; flags: bit 0 also second
+// flags: bit 0 also second
 // derivatives (Hessian), bit 1 theta is also stored as the last evaluated theta (the
 // NLL and Hessian entry points; the per-event outputs leave it)
 extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_prep(const double* params, double* table,
-                                                                              const ctpwa::PrepArgs* a, int nv,
-                                                                              int flags, hipStream_t stream) {
+                                                                              const ctpwa::PrepArgs* a, int flags,
+                                                                              hipStream_t stream) {
     const int hess = flags & 1, rem = (flags >> 1) & 1;
-    if (nv <= 1) return hess ? launch_prep_t<1, true>(params, table, a, rem, stream) : launch_prep_t<1, false>(params, table, a, rem, stream);
-    if (nv <= 2) return hess ? launch_prep_t<2, true>(params, table, a, rem, stream) : launch_prep_t<2, false>(params, table, a, rem, stream);
-    if (nv <= 4) return hess ? launch_prep_t<4, true>(params, table, a, rem, stream) : launch_prep_t<4, false>(params, table, a, rem, stream);
-    return hess ? launch_prep_t<8, true>(params, table, a, rem, stream) : launch_prep_t<8, false>(params, table, a, rem, stream);
-}
-
-template <int NV, bool H>
-static hipError_t launch_prep_batch_t(const double* const* params, double* const* tables, const ctpwa::PrepArgs* a,
-                                      const ctpwa::PrepArgs* args, int rows, const int* hdr, hipStream_t stream) {
-    int items = a->nden + a->namp;
-    hipLaunchKernelGGL((ctpwa::k_prep_batch<NV, H>), dim3(items, rows), dim3(64), ctpwa::prep_lds_bytes(*a), stream, params,
-                       tables, *a, args, hdr);
-    return hipGetLastError();
+    return hess ? launch_prep_t<true>(params, table, a, rem, stream) : launch_prep_t<false>(params, table, a, rem, stream);
 }
 
 // rows: workgroup rows launched (the job count, or with hdr a bound on the job count hdr[0]
@@ -814,14 +755,14 @@ static hipError_t launch_prep_batch_t(const double* const* params, double* const
 // device (a then only gives the launch shape)
 extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_prep_batch(const double* const* params,
                                                                                     double* const* tables,
-                                                                                    const ctpwa::PrepArgs* a, int nv,
+                                                                                    const ctpwa::PrepArgs* a,
                                                                                     const ctpwa::PrepArgs* args, int rows,
                                                                                     const int* hdr, hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
-    if (nv <= 1) return launch_prep_batch_t<1, false>(params, tables, a, args, rows, hdr, stream);
-    if (nv <= 2) return launch_prep_batch_t<2, false>(params, tables, a, args, rows, hdr, stream);
-    if (nv <= 4) return launch_prep_batch_t<4, false>(params, tables, a, args, rows, hdr, stream);
-    return launch_prep_batch_t<8, false>(params, tables, a, args, rows, hdr, stream);
+    const int items = a->nden + a->namp;
+    hipLaunchKernelGGL(ctpwa::k_prep_batch, dim3(items, rows), dim3(64), 0, stream, params, tables, *a,
+                       args, hdr);
+    return hipGetLastError();
 }
 
 // fins: device array of the jobs' arguments; rows and hdr as above; max_nacc: the largest
@@ -830,7 +771,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finaliz
                                                                                         int max_nacc, size_t lds_bytes,
                                                                                         const int* hdr, hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(ctpwa::k_reduce_batch, dim3(3 * max_nacc, rows), dim3(ctpwa::RED_THREADS), 0, stream, fins, hdr);
+    hipLaunchKernelGGL(ctpwa::k_reduce_batch, dim3((3 * max_nacc + 3) / 4, rows), dim3(ctpwa::RED_THREADS), 0, stream, fins, hdr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(ctpwa::k_assemble_batch, dim3(rows), dim3(ctpwa::ASM_THREADS), lds_bytes, stream, fins, hdr);
@@ -840,7 +781,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finaliz
 // done: a device counter that is zero between evaluations (reset by the kernel itself)
 extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs* f, unsigned int* done,
                                                                                   hipStream_t stream) {
-    hipLaunchKernelGGL(ctpwa::k_finalize, dim3(3 * f->nacc), dim3(ctpwa::ASM_THREADS), ctpwa::assemble_lds_bytes(*f), stream,
+    hipLaunchKernelGGL(ctpwa::k_finalize, dim3((3 * f->nacc + 15) / 16), dim3(ctpwa::ASM_THREADS), ctpwa::assemble_lds_bytes(*f), stream,
                        *f, done);
     return hipGetLastError();
 }
