@@ -35,7 +35,7 @@ extern "C" hipError_t ctpwa_launch_to_mixed(const double2*, const double*, long 
 extern "C" hipError_t ctpwa_launch_polsym(const double2*, long long, long long, long long, int, unsigned long long*,
                                           hipStream_t);
 extern "C" hipError_t ctpwa_launch_prep(const double*, double*, const ctpwa::PrepArgs*, int, hipStream_t);
-extern "C" hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs*, unsigned int*, hipStream_t);
+extern "C" hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_prep_batch(const double* const*, double* const*, const ctpwa::PrepArgs*,
                                               const ctpwa::PrepArgs*, int, const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_finalize_batch(const ctpwa::FinArgs*, int, int, size_t, const int*, hipStream_t);
@@ -836,6 +836,7 @@ extern "C" int ctpwa_create(const char* plan_text, const double* phsp, long long
                            (long long)M.off_th(), (long long)M.off_lth(), 0};
         h->fin = FinArgs{};
         h->fin.part = h->part;
+        h->fin.done = h->fin_done;
         h->fin.nwg = h->nwg;
         h->fin.nacc = h->nacc;
         for (int c = 0; c < 3; ++c) { h->fin.g0[c] = h->g0[c]; h->fin.g1[c] = h->g1[c]; }
@@ -1012,7 +1013,7 @@ extern "C" int ctpwa_nll_grad(ctpwa_handle* h, const double* params_dev, double*
     if (e == hipSuccess) {
         h->fin.params = params_dev;
         h->fin.out = out_dev;
-        e = ctpwa_launch_finalize(&h->fin, h->fin_done, s);
+        e = ctpwa_launch_finalize(&h->fin, s);
     }
     if (e != hipSuccess) return fail(std::string("ctpwa_nll_grad: ") + hipGetErrorString(e));
     return 0;
@@ -1038,7 +1039,7 @@ extern "C" int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev,
         f.totals = scr + (size_t)h->nacc * (size_t)std::max(1, h->nwg);
         f.params = params_dev;
         f.out = out_dev;
-        e = ctpwa_launch_finalize(&f, h->fin_done, s);
+        e = ctpwa_launch_finalize(&f, s);
     }
     if (e != hipSuccess) return fail(std::string("ctpwa_nll_grad_noalloc: ") + hipGetErrorString(e));
     return 0;

@@ -106,6 +106,7 @@ struct FinArgs {
     const double* params;
     double* out;             // [1 + 2 nfree + ntheta]
     double* totals;          // [3][nacc] scratch (kept for inspection)
+    unsigned int* done;      // counts finished workgroups; zero between evaluations
     // no free resonance parameter: the phase-space totals come from the stored amplitude
     // Gram G[a][b] = sum_e sum_p conj(A'_a) A'_b (amplitudes without couplings or theta
     // coefficients) and the table's c_a (offset off_c) instead of per-event partials

@@ -313,7 +313,6 @@ __global__ void __launch_bounds__(64) k_prep_batch(const double* const* __restri
 // final assembly
 // ---------------------------------------------------------------------------
 
-constexpr int RED_THREADS = 256;
 constexpr int ASM_THREADS = 1024;
 
 // this lane's share of class c's total of accumulator column col: the class's
@@ -369,17 +368,7 @@ __device__ __forceinline__ double pair_total(const FinArgs& f, int pair) {
     return s;
 }
 
-// stage 1: one wave per (class, accumulator column); fixed summation order
-__global__ void __launch_bounds__(RED_THREADS) k_reduce_batch(const FinArgs* __restrict__ fins, const int* __restrict__ hdr) {
-    if (hdr && (int)blockIdx.y >= hdr[0]) return;
-    const FinArgs& f = fins[blockIdx.y];
-    const int pair = blockIdx.x * (RED_THREADS / 64) + (threadIdx.x >> 6);
-    if (pair >= 3 * f.nacc) return;
-    const double tot = pair_total(f, pair);
-    if ((threadIdx.x & 63) == 0) f.totals[pair] = tot;
-}
-
-// stage 2: NLL and gradient from the class totals.  Every global read happens first, in
+// NLL and gradient from the class totals.  Every global read happens first, in
 // parallel over the threads: the gradient entries' weights (scale times their table
 // coefficient), accumulator indices and row pointers (assemble_prefill, which needs no
 // totals and so runs in k_finalize before a workgroup's reduction, off the last
@@ -429,9 +418,8 @@ __device__ __forceinline__ void assemble_prefill(const FinArgs& f) {
     for (int k = tid; k <= f.nfree; k += ASM_THREADS) L.cpp[k] = f.cpp[k];
     for (int k = tid; k <= f.ntheta; k += ASM_THREADS) L.thp[k] = f.thp[k];
 }
-// the assembly proper, after assemble_prefill and a barrier; SHARED: the totals come from other
+// the assembly proper, after assemble_prefill and a barrier; the totals come from other
 // workgroups of this launch (coherent loads)
-template <bool SHARED>
 __device__ __forceinline__ void assemble_main(const FinArgs& f) {
     const AsmLds L = asm_lds(f);
     double* C = L.C;
@@ -445,7 +433,7 @@ __device__ __forceinline__ void assemble_main(const FinArgs& f) {
     const int* thp = L.thp;
     int tid = threadIdx.x;
     auto tot = [&](int i) {                  // i = c * nacc + col
-        return SHARED ? __hip_atomic_load(f.totals + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : f.totals[i];
+        return __hip_atomic_load(f.totals + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     double Np = f.Np, Neff = f.Wd - f.Wb;
     double pf = (Np > 0) ? tot(0) / Np : 0.0;
@@ -498,12 +486,6 @@ __device__ __forceinline__ void assemble_main(const FinArgs& f) {
     }
 }
 
-__device__ __forceinline__ void assemble_body(const FinArgs& f) {
-    assemble_prefill(f);
-    __syncthreads();
-    assemble_main<false>(f);
-}
-
 // Reduction and assembly in one launch: every wave sums one (class, accumulator) over the
 // class's workgroup partials, and the workgroup that finishes last, found by a device-scope
 // counter, runs the assembly on the totals and resets the counter for the next evaluation.
@@ -511,7 +493,7 @@ __device__ __forceinline__ void assemble_body(const FinArgs& f) {
 // a workgroup (one workgroup and one count per sum, each with the assembly's inputs, took
 // 37 us at 149 amplitudes, 11 us at 10; now 12 and 9); the totals go through coherent stores and loads
 // and a wait instead of agent-scope fences, which write back and invalidate the L2 cache.
-__global__ void __launch_bounds__(ASM_THREADS) k_finalize(FinArgs f, unsigned int* __restrict__ done) {
+__device__ __forceinline__ void finalize_body(const FinArgs& f) {
     __shared__ int last;
     const int pair = blockIdx.x * (ASM_THREADS / 64) + (threadIdx.x >> 6);
     // the assembly's inputs that need no totals, loaded by every workgroup while its
@@ -523,16 +505,19 @@ __global__ void __launch_bounds__(ASM_THREADS) k_finalize(FinArgs f, unsigned in
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's total is visible before the count
     __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(done, 1u) == gridDim.x - 1;
+    if (threadIdx.x == 0) last = atomicAdd(f.done, 1u) == gridDim.x - 1;
     __syncthreads();
     if (!last) return;
-    assemble_main<true>(f);
-    if (threadIdx.x == 0) *done = 0u;
+    assemble_main(f);
+    if (threadIdx.x == 0) *f.done = 0u;
 }
+__global__ void __launch_bounds__(ASM_THREADS) k_finalize(FinArgs f) { finalize_body(f); }
+// many likelihoods, one per blockIdx.y.  (Separate launches for the sums and the assemblies
+// took 4.7 + 6.2 us for 24 likelihoods of 10 amplitudes, together 9.5 us.)
 
-__global__ void __launch_bounds__(ASM_THREADS) k_assemble_batch(const FinArgs* __restrict__ fins, const int* __restrict__ hdr) {
-    if (hdr && (int)blockIdx.x >= hdr[0]) return;
-    assemble_body(fins[blockIdx.x]);
+__global__ void __launch_bounds__(ASM_THREADS) k_finalize_batch(const FinArgs* __restrict__ fins, const int* __restrict__ hdr) {
+    if (hdr && (int)blockIdx.y >= hdr[0]) return;
+    finalize_body(fins[blockIdx.y]);
 }
 
 // ---------------------------------------------------------------------------
@@ -771,18 +756,14 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finaliz
                                                                                         int max_nacc, size_t lds_bytes,
                                                                                         const int* hdr, hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(ctpwa::k_reduce_batch, dim3((3 * max_nacc + 3) / 4, rows), dim3(ctpwa::RED_THREADS), 0, stream, fins, hdr);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(ctpwa::k_assemble_batch, dim3(rows), dim3(ctpwa::ASM_THREADS), lds_bytes, stream, fins, hdr);
+    hipLaunchKernelGGL(ctpwa::k_finalize_batch, dim3((3 * max_nacc + 15) / 16, rows), dim3(ctpwa::ASM_THREADS), lds_bytes, stream,
+                       fins, hdr);
     return hipGetLastError();
 }
 
-// done: a device counter that is zero between evaluations (reset by the kernel itself)
-extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs* f, unsigned int* done,
-                                                                                  hipStream_t stream) {
-    hipLaunchKernelGGL(ctpwa::k_finalize, dim3((3 * f->nacc + 15) / 16), dim3(ctpwa::ASM_THREADS), ctpwa::assemble_lds_bytes(*f), stream,
-                       *f, done);
+extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs* f, hipStream_t stream) {
+    hipLaunchKernelGGL(ctpwa::k_finalize, dim3((3 * f->nacc + 15) / 16), dim3(ctpwa::ASM_THREADS), ctpwa::assemble_lds_bytes(*f),
+                       stream, *f);
     return hipGetLastError();
 }
 
