@@ -623,18 +623,14 @@ extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_tables(int ncol,
     return q;
 }
 
-// workgroups of a Gram of up to 64 columns whose rows take `bytes` (environment CTPWA_GRAM_WGS
-// overrides it for measurements).  Two per CU while the rows, just written, are still mostly in
-// the last-level cache (256 MB): more workgroups only mean more partials (Hessian in the mixed
-// form, 40 columns: 50 MB 131 against 143 us with three per CU, 345 MB 389 against 424 us).
-// Three when they come from memory, whose latency two waves per SIMD do not cover (576 MB 721
-// against 646 us, 960 MB 1162 against 1010 us; 62 columns, 595 MB 1694 against 1513 us).
-extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_nwg(long long bytes) {
+// workgroups of a Gram of up to 64 columns (environment CTPWA_GRAM_WGS overrides it for
+// measurements)
+extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_nwg() {
     static const int n = [] {
         const char* e = std::getenv("CTPWA_GRAM_WGS");
-        return e ? std::max(32, std::atoi(e) / 4) : 0;
+        return e ? std::max(32, std::atoi(e) / 4) : 512;
     }();
-    return n ? n : bytes > (450LL << 20) ? 768 : 512;
+    return n;
 }
 
 // weighted Gram on the matrix cores of the pieces' rows (rpe rows per event), up to 64 columns:
