@@ -44,7 +44,7 @@ extern "C" hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs*, int, long long, lo
 
 extern "C" hipError_t ctpwa_launch_zero(double*, long long, hipStream_t);
 extern "C" int ctpwa_gram_tables(int, int2*, ctpwa::GramPair*, int*, int*);
-extern "C" int ctpwa_gram_nwg();
+extern "C" int ctpwa_gram_nwg(int, int);
 extern "C" hipError_t ctpwa_launch_gram_panels(const void*, int, int, long long, const ctpwa::HessPieces*, int, const double*,
                                                 double*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_gram_wide(const void*, int, int, long long, long long, long long, const double*,
@@ -1074,11 +1074,11 @@ struct GramSizes {
 };
 // the partials of a Gram: ncol <= 64 at least one workgroup per piece; more columns: two
 // workgroups per CU shared out among the panel pairs by a wave's tile pairs
-static long long gram_plan(int ncol, int ncu, std::vector<GramPair>* pairs, int* nwg) {
+static long long gram_plan(int ncol, bool f32, int ncu, std::vector<GramPair>* pairs, int* nwg) {
     int np = 0;
     const int ntp = ctpwa_gram_tables(ncol, nullptr, nullptr, &np, nullptr);
     if (ncol <= 64) {
-        *nwg = ctpwa_gram_nwg() + 4;
+        *nwg = ctpwa_gram_nwg(f32, ncol);
         return (long long)*nwg * ntp * 256;
     }
     std::vector<GramPair> pp((size_t)np);
@@ -1108,8 +1108,10 @@ static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long
     // (split rows: one-wave workgroups, as many times over as there are sets; 2 or 8 per CU and
     // set are 2 % slower)
     const int per_cu = S.split ? 4 : std::max(1, (int)std::min<long long>(8 / S.G, 160 * 1024 / std::max<long long>(1, S.lds * 8)));
-    // (a class smaller than a workgroup's share still gets one)
-    z.target = (int)std::min<long long>((long long)ncu * per_cu, std::max<long long>(1, (all + 63) / 64)) + 4;
+    // never more than fit on the chip at once (four workgroups over, for classes smaller than
+    // a share, ran as a second round: the mixed form's Gram of 3.05M events 611 us, not 310);
+    // at least one for each of up to four pieces
+    z.target = (int)std::max<long long>(4, std::min<long long>((long long)ncu * per_cu, (all + 63) / 64 + 3));
     z.nz = S.NU > 0 ? hess_nz(M) + S.NU : 0;
     z.z = (long long)z.nz * z.target;
     if (S.fused) {
@@ -1126,7 +1128,7 @@ static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long
     z.W = z.ldc * (S.split && S.NU > 0 ? 2 + 2 * M.P.npol : 2);
     z.D = S.split ? z.ldc * S.nslot * 2 * M.P.npol : 0;
     int nwg = 0;
-    z.part = gram_plan(2 * S.C, ncu, nullptr, &nwg) + (S.NU > 0 ? gram_plan(S.NU, ncu, nullptr, &nwg) : 0);
+    z.part = gram_plan(2 * S.C, S.f32, ncu, nullptr, &nwg) + (S.NU > 0 ? gram_plan(S.NU, false, ncu, nullptr, &nwg) : 0);
     return z;
 }
 static int device_cus(int device) {
@@ -1159,14 +1161,14 @@ static long long agram_workspace_bytes(const Model_& M, long long n) {
 }
 
 // nwg > 0: the fused form's workgroups, each with its tile pairs' sums
-static void gram_setup(ctpwa_handle* h, GramTabs& g, int ncol, int nwg) {
+static void gram_setup(ctpwa_handle* h, GramTabs& g, int ncol, bool f32, int nwg) {
     g.ncol = ncol;
     g.ntp = ctpwa_gram_tables(ncol, nullptr, nullptr, &g.npp, nullptr);
     std::vector<int2> tiles((size_t)g.ntp);
     std::vector<int> tpair((size_t)g.ntp);
     ctpwa_gram_tables(ncol, tiles.data(), nullptr, &g.npp, tpair.data());
     std::vector<GramPair> pp;
-    long long part = gram_plan(ncol, device_cus(h->device), &pp, &g.nwg);
+    long long part = gram_plan(ncol, f32, device_cus(h->device), &pp, &g.nwg);
     if (nwg > 0) {
         g.nwg = nwg;
         part = (long long)nwg * g.ntp * 256;
@@ -1204,8 +1206,8 @@ static void gramws_setup(ctpwa_handle* h, GramWS& w, bool amps_only, const long 
         // the amplitude Gram weights every row by one
         w.W = amps_only ? h->upload(std::vector<double>((size_t)z.W, 1.0)) : h->alloc<double>((size_t)z.W);
     }
-    gram_setup(h, w.gJ, 2 * w.S.C, w.S.fused ? z.target : 0);
-    if (w.S.NU > 0) gram_setup(h, w.gU, w.S.NU, w.S.fused ? z.target : 0);
+    gram_setup(h, w.gJ, 2 * w.S.C, w.S.f32, w.S.fused ? z.target : 0);
+    if (w.S.NU > 0) gram_setup(h, w.gU, w.S.NU, false, w.S.fused ? z.target : 0);
     w.ready = true;
 }
 

@@ -476,7 +476,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
             };
             auto ustore = [&](const std::string& v, int x, const char* ind) {
                 put(v, col_u0 + x, ind);
-                if (!fused) o << ind << (kind == GROUP ? "if (cls != 0) " : "") << "at(Uk + " << x << "LL * lu, wo) = " << v << ";\n";
+                if (!fused) o << ind << (kind == GROUP && NA <= 12 ? "if (cls != 0) " : "") << "at(Uk + " << x << "LL * lu, wo) = " << v << ";\n";
             };
             // a parameter's finished derivative columns
             auto theta_cols = [&](int j) {

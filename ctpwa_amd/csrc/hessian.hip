@@ -75,7 +75,7 @@ inline size_t gram_panels_lds(bool f32, int NT) {
 // NT: tiles of the columns; the NT (NT + 1) / 2 tile pairs I <= J.  With the pair count fixed
 // at compile time every pair's product is unconditional.
 template <typename T, int NT>
-__global__ void __launch_bounds__(64 * GP_WAVES)
+__global__ void __launch_bounds__(64 * GP_WAVES, sizeof(T) == 4 && NT < 4 ? 3 : 2)
 k_gram_panels(const T* __restrict__ X0, int ncol, long long ldx, HessPieces H, int rpe, const double* __restrict__ Wt0,
               double* __restrict__ part) {
     constexpr int R = GP<T>::R, ST = R + 1;
@@ -624,13 +624,15 @@ extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_tables(int ncol,
 }
 
 // workgroups of a Gram of up to 64 columns (environment CTPWA_GRAM_WGS overrides it for
-// measurements)
-extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_nwg() {
+// measurements): as many as fit on the chip at once by their registers, three per CU for up to
+// three tiles of FP32 columns, else two.  One more runs as a second round (four over 512: 611 us
+// for the FP32 rows of 3.05M events, 378 us without, with three per CU 325 us).
+extern "C" __attribute__((visibility("hidden"))) int ctpwa_gram_nwg(int f32, int ncol) {
     static const int n = [] {
         const char* e = std::getenv("CTPWA_GRAM_WGS");
-        return e ? std::max(32, std::atoi(e) / 4) : 512;
+        return e ? std::max(32, std::atoi(e) / 4) : 0;
     }();
-    return n;
+    return n ? n : f32 && ncol <= 48 ? 768 : 512;
 }
 
 // weighted Gram on the matrix cores of the pieces' rows (rpe rows per event), up to 64 columns:
