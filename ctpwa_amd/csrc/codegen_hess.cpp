@@ -186,7 +186,8 @@ HessShape hess_shape(const Model_& M, bool amps_only) {
             H.SW = 16;
             H.lds = amps_only ? 0 : H.SW * 66;
             // the summing kernel's wave groups: the same order of blocks, cut by amplitudes
-            H.sum_blocks.assign(std::min(8, n), {});
+            // (as many as have room to exchange their shares of S in LDS)
+            H.sum_blocks.assign(std::min({8, n, std::max(1, 159 / NP)}), {});
             for (int k = 0, a = 0; k < n; a += P.blocks[bl[k++]].nsl)
                 H.sum_blocks[std::min<size_t>(H.sum_blocks.size() - 1, (size_t)a * H.sum_blocks.size() / P.namp)].push_back(bl[k]);
             return H;

@@ -362,6 +362,8 @@ inline void assign_groups(Model_& M) {
     for (size_t d = 0; d < M.dens.size(); ++d) key[d] = den_key(M, (int)d);
     const int n = (int)bl.size();
     int G = P.namp <= 24 ? 1 : std::min(8, (P.namp + 18) / 19);
+    // (the two exchange buffers, G shares of S for 64 events each, have to fit in LDS)
+    while (G > 1 && 2LL * G * 2 * P.npol * 64 * 8 > 159 * 1024) --G;
     G = std::max(1, std::min(G, n));
     M.bgroup.assign(P.blocks.size(), 0);
     if (G > 1) {
