@@ -30,7 +30,8 @@
 //  * fused (FP64 Jacobian of up to 64 real columns): J and u of the 64 events go into an LDS
 //    tile and straight into the FP64 matrix cores, whose tile pairs are shared out among the
 //    waves; nothing per event is written.  Written to memory and read back by the Gram
-//    kernel, the 40-column Jacobian of 3.05M events moved 3.9 GB (getHessian 1.31 ms).
+//    kernel, the 40-column Jacobian of 3.05M events moved 3.9 GB (getHessian 1.31 ms,
+//    fused 0.79 ms).
 //  * rows: J (FP64, or FP32 in the mixed form), u and the weights are written to memory,
 //    column-major, for the Gram kernels.
 //  * split rows, for more than 24 amplitudes.  A workgroup of eight waves that runs the code
@@ -126,6 +127,9 @@ HessShape hess_shape(const Model_& M, bool amps_only) {
     const int n = (int)bl.size();
     int sets = 1;
     for (int k = 1; k < n; ++k) sets += pars(bl[k]) != pars(bl[k - 1]);
+    // about five amplitudes to a group.  FP64, 10 amplitudes, 3.05M events: four groups 818 us,
+    // two 827; amplitude Gram, 1M events: 108 against 124.  FP32 rows hold less per event: 10
+    // amplitudes, 305k events: two 126 us, four 134; 20 amplitudes, 360k events: two 492, four 445
     int G = P.namp <= 4 ? 1 : P.namp <= (H.f32 ? 12 : 8) ? 2 : P.namp <= 24 ? 4 : 8;
     H.fused = !H.f32 && 2 * H.C <= 64;
     H.split = !H.fused && P.namp > 24;

@@ -29,8 +29,6 @@
 
 namespace ctpwa {
 
-
-
 // Weighted Gram of a column-major matrix X[column][row] (column stride ldx) on the matrix
 // cores:
 //   G[a][b] = sum_rows w(row) X[a][row] X[b][row],  w(row) = Wt[row mod nev]
