@@ -36,8 +36,8 @@ extern "C" hipError_t ctpwa_launch_polsym(const double2*, long long, long long, 
                                           hipStream_t);
 extern "C" hipError_t ctpwa_launch_prep(const double*, double*, const ctpwa::PrepArgs*, int, hipStream_t);
 extern "C" hipError_t ctpwa_launch_finalize(const ctpwa::FinArgs*, hipStream_t);
-extern "C" hipError_t ctpwa_launch_prep_batch(const double* const*, double* const*, const ctpwa::PrepArgs*,
-                                              const ctpwa::PrepArgs*, int, const int*, hipStream_t);
+extern "C" hipError_t ctpwa_launch_prep_batch(const double* const*, double* const*, const ctpwa::PrepArgs*, int, int,
+                                              const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_finalize_batch(const ctpwa::FinArgs*, int, int, size_t, const int*, hipStream_t);
 extern "C" hipError_t ctpwa_launch_aux(const ctpwa::AuxArgs*, int, long long, long long, double*, int, hipStream_t);
 
@@ -1630,6 +1630,7 @@ struct ctpwa_batch {
     bool pending = false;
     size_t o_hdr = 0, o_ctr = 0, o_jobs = 0, o_fins = 0, o_params = 0, o_tables = 0, o_preps = 0;
     int max_nacc = 0;              // of the uploaded list
+    int max_items = 0;             // coefficient records of a job's prep
     size_t max_lds = 0;
     // Graph replays (opt-in, environment CTPWA_BATCH_GRAPH=1): the descriptors on the device
     // belong to `key`, a list of (handle serial, params, out); a call with the same list
@@ -1643,7 +1644,7 @@ struct ctpwa_batch {
     int rows = 0;
     hipStream_t cs = nullptr;      // capture stream
     hipModule_t gmod = nullptr;
-    std::map<int, hipGraphExec_t> execs;
+    std::map<std::pair<int, int>, hipGraphExec_t> execs;   // by (rows, max_items)
     int persist = 0;               // workgroups of the persistent grouped kernel
 };
 
@@ -1712,7 +1713,7 @@ static void batch_launches_graph(ctpwa_batch* b, const ctpwa_handle* h0, int row
     const int* d_hdr = (const int*)(b->dev + b->o_hdr);
     unsigned int* d_ctr = (unsigned int*)(b->dev + b->o_ctr);
     HIPCHECK(ctpwa_launch_prep_batch((const double* const*)(b->dev + b->o_params), (double* const*)(b->dev + b->o_tables),
-                                     &h0->prep, (const PrepArgs*)(b->dev + b->o_preps), rows, d_hdr, s));
+                                     (const PrepArgs*)(b->dev + b->o_preps), b->max_items, rows, d_hdr, s));
     const EvalJob* d_jobs = (const EvalJob*)(b->dev + b->o_jobs);
     void* args[] = {&d_jobs, &d_hdr, &d_ctr};
     HIPCHECK(hipModuleLaunchKernel(h0->fn_group_p, b->persist, 1, 1, h0->M.wgs, 1, 1, 0, s, args, nullptr));
@@ -1764,11 +1765,12 @@ extern "C" int ctpwa_batch_nll_grad(ctpwa_batch* b, ctpwa_handle* const* hs, con
             const double** pp = (const double**)(b->host + b->o_params);
             double** tp = (double**)(b->host + b->o_tables);
             PrepArgs* pa = (PrepArgs*)(b->host + b->o_preps);
-            int max_nacc = 0;
+            int max_nacc = 0, max_items = 0;
             size_t max_lds = 0;
             for (int j = 0; j < n; ++j) {
                 ctpwa_handle* h = hs[j];
                 max_nacc = std::max(max_nacc, h->nacc);
+                max_items = std::max(max_items, h->prep.nden + h->prep.namp);
                 max_lds = std::max(max_lds, assemble_lds_bytes(h->fin));
                 jobs[j] = EvalJob{h->table, h->slp, h->inv, h->invf, h->wts, h->part, h->wg_cls, h->wg_rng, h->cfb,
                                   h->ntot, h->wc[1], h->wc[2], h->nwg, h->pw[1], h->pw[2], wg};
@@ -1788,6 +1790,7 @@ extern "C" int ctpwa_batch_nll_grad(ctpwa_batch* b, ctpwa_handle* const* hs, con
             HIPCHECK(hipEventRecord(b->copied, s));
             b->pending = true;
             b->max_nacc = max_nacc;
+            b->max_items = max_items;
             b->max_lds = max_lds;
             if (graph) {
                 b->key.swap(key);
@@ -1798,10 +1801,13 @@ extern "C" int ctpwa_batch_nll_grad(ctpwa_batch* b, ctpwa_handle* const* hs, con
         }
         if (!graph) {
             // one batched prep launch, each job's Custom factors, one grouped launch whose
-            // workgroups are shared out among the jobs, one batched reduction and assembly
+            // workgroups are shared out among the jobs, one batched reduction and assembly.
+            // Every job's coefficients come from its own handle's model tables: handles that
+            // share a kernel may differ in fixed masses, widths, ratios and constraints, which
+            // the kernel's source does not hold.
             HIPCHECK(ctpwa_launch_prep_batch((const double* const*)(b->dev + b->o_params),
-                                             (double* const*)(b->dev + b->o_tables), &h0->prep, nullptr, n,
-                                             nullptr, s));
+                                             (double* const*)(b->dev + b->o_tables),
+                                             (const PrepArgs*)(b->dev + b->o_preps), b->max_items, n, nullptr, s));
             for (int j = 0; j < n; ++j) HIPCHECK(launch_custom(hs[j], s));
             const EvalJob* d_jobs = (const EvalJob*)(b->dev + b->o_jobs);
             void* args[] = {&d_jobs, &n};
@@ -1819,7 +1825,8 @@ extern "C" int ctpwa_batch_nll_grad(ctpwa_batch* b, ctpwa_handle* const* hs, con
             b->persist = std::max(1, per_cu) * std::max(1, ncu);
             b->gmod = h0->mod;
         }
-        auto it = b->execs.find(b->rows);
+        const auto shape = std::make_pair(b->rows, b->max_items);
+        auto it = b->execs.find(shape);
         if (it == b->execs.end()) {
             hipGraph_t graph_ = nullptr;
             hipGraphExec_t exec = nullptr;
@@ -1835,7 +1842,7 @@ extern "C" int ctpwa_batch_nll_grad(ctpwa_batch* b, ctpwa_handle* const* hs, con
             hipError_t e = hipGraphInstantiate(&exec, graph_, nullptr, nullptr, 0);
             (void)hipGraphDestroy(graph_);
             HIPCHECK(e);
-            it = b->execs.emplace(b->rows, exec).first;
+            it = b->execs.emplace(shape, exec).first;
         }
         HIPCHECK(hipGraphLaunch(it->second, s));
         return 0;

@@ -296,15 +296,15 @@ __global__ void __launch_bounds__(64) k_prep(const double* __restrict__ params, 
     prep_body<H>(params, table, a);
 }
 
-// many likelihoods of one model: blockIdx.y selects the likelihood (its parameters and
-// coefficient table); the model tables in `a` are the same for all of them
-// one workgroup row per job.  hdr (graph replays; NULL otherwise): hdr[0] is the number
-// of jobs, rows at or beyond it leave at once, and each job's prep arguments come from
-// args[row] (its own handle's model tables) instead of `a`
+// many likelihoods that share a fused kernel: blockIdx.y selects the likelihood, its
+// parameters, its coefficient table and its own handle's model tables (args: a kernel's
+// source does not hold fixed masses and the like).  hdr (graph replays; NULL otherwise):
+// hdr[0] is the number of jobs, rows at or beyond it leave at once.  The grid has as many
+// items as the largest job.
 __global__ void __launch_bounds__(64) k_prep_batch(const double* const* __restrict__ params, double* const* __restrict__ tables,
-                                                   PrepArgs a, const PrepArgs* __restrict__ args, const int* __restrict__ hdr) {
+                                                   const PrepArgs* __restrict__ args, const int* __restrict__ hdr) {
     if (hdr && (int)blockIdx.y >= hdr[0]) return;
-    if (args) a = args[blockIdx.y];
+    PrepArgs a = args[blockIdx.y];
     a.remember = 1;                 // NLL evaluations: each table keeps its theta as the last evaluated one
     prep_body<false>(params[blockIdx.y], tables[blockIdx.y], a);
 }
@@ -735,18 +735,16 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_prep(co
     return hess ? launch_prep_t<true>(params, table, a, rem, stream) : launch_prep_t<false>(params, table, a, rem, stream);
 }
 
-// rows: workgroup rows launched (the job count, or with hdr a bound on the job count hdr[0]
-// on the device, extra rows leave); args: NULL, or the jobs' own prep arguments on the
-// device (a then only gives the launch shape)
+// args: the jobs' prep arguments on the device; items: the largest job's coefficient records;
+// rows: workgroup rows launched (the job count, or with hdr a bound on the job count hdr[0] on
+// the device, extra rows leave)
 extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_prep_batch(const double* const* params,
                                                                                     double* const* tables,
-                                                                                    const ctpwa::PrepArgs* a,
-                                                                                    const ctpwa::PrepArgs* args, int rows,
-                                                                                    const int* hdr, hipStream_t stream) {
+                                                                                    const ctpwa::PrepArgs* args, int items,
+                                                                                    int rows, const int* hdr,
+                                                                                    hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
-    const int items = a->nden + a->namp;
-    hipLaunchKernelGGL(ctpwa::k_prep_batch, dim3(items, rows), dim3(64), 0, stream, params, tables, *a,
-                       args, hdr);
+    hipLaunchKernelGGL(ctpwa::k_prep_batch, dim3(items, rows), dim3(64), 0, stream, params, tables, args, hdr);
     return hipGetLastError();
 }
 

@@ -87,8 +87,9 @@ int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev, double* ou
 /* Hessian in the same layout: device [(2 n_free + n_theta)^2], row-major. */
 int ctpwa_hessian(ctpwa_handle* h, const double* params_dev, double* hess_dev, void* stream);
 
-/* Many likelihoods of one model (same plan and precision; e.g. the toy fits of an
- * ensemble) evaluated together: one batched prep launch, one grouped per-event launch
+/* Many likelihoods of one model (same generated kernel: same structure and precision, while
+ * fixed masses, widths and ratios may differ; e.g. the toy fits of an ensemble) evaluated
+ * together: one batched prep launch, one grouped per-event launch
  * whose workgroups are shared out among the likelihoods, one batched reduction.  Each
  * likelihood's result is bit-identical to ctpwa_nll_grad on its own (same partition of
  * its events, same summation order).  Replaces the per-fit NLLFunction::forward/backward
