@@ -498,10 +498,14 @@ static Partition partition(const ctpwa_handle* h, bool scan_phsp, long long targ
 }
 
 // The fused kernel's workgroups.  One wave per event (groups == 1): about 1024 (four
-// 128-thread workgroups per CU), at least 256 events each.  Wave groups: one workgroup per
-// CU (its eight waves hold all the registers of a CU's two waves per SIMD) with at least
-// 128 events; 1024 of them, four rounds of workgroups, took 512 us instead of 496 at 1.5M
-// events and 149 amplitudes, and left four times the partial sums to add up.
+// 128-thread workgroups per CU), at least 256 events each.  Wave groups: as many as the chip
+// holds at once by the compiled kernel's registers and LDS, at least 128 events each.  Two
+// groups of at most 256 registers (25 to 32 amplitudes) fit four times on a CU: one workgroup
+// per CU left half of the SIMDs idle (1.4M events, FP64: 26 amplitudes 147 us, four per CU
+// 94; 3M events of 25 amplitudes 270 and 144; as one wave 101 and 181).  More of them than
+// fit run as further rounds: 31 amplitudes, whose 302 registers allow two per CU, 200 us with
+// four and 193 with two; 149 amplitudes, one per CU, 512 us with four and 496 with one, which
+// also leaves a quarter of the partial sums to add up.
 static void setup_partition(ctpwa_handle* h, bool scan_phsp) {
     const long long nev = (scan_phsp ? h->n[0] : 0) + h->n[1] + h->n[2];
     // relative cost of a data or background event: the workgroups of each class get events
@@ -521,9 +525,11 @@ static void setup_partition(ctpwa_handle* h, bool scan_phsp) {
     const long long t1 = std::min<long long>(1024, std::max<long long>(1, (nev + 255) / 256));
     Partition R;
     if (M.groups > 1) {
-        int ncu = 0;
+        int ncu = 0, per_cu = 0;
         HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
-        const long long t = std::min<long long>(std::max(4, std::min(ncu, 1024)), std::max<long long>(1, (nev + 127) / 128));
+        HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, h->fn_eval, M.wgs, 0));
+        const int fit = ncu * std::max(1, per_cu);
+        const long long t = std::min<long long>(std::max(4, std::min(fit, 1024)), std::max<long long>(1, (nev + 127) / 128));
         // (a class too small for a workgroup of its own still gets one)
         for (long long k = t;; --k) {
             R = partition(h, scan_phsp, k, M.ev_step(), wcost, true);
@@ -823,6 +829,12 @@ extern "C" int ctpwa_create(const char* plan_text, const double* phsp, long long
         h->table = h->alloc<double>(M.table_size());
         HIPCHECK(hipMemset(h->table, 0, M.table_size() * sizeof(double)));
 
+        h->src = generate_eval_kernel(M);
+        h->mod = compile_eval(device, h->src);
+        HIPCHECK(hipModuleGetFunction(&h->fn_eval, h->mod, "ctpwa_eval"));
+        HIPCHECK(hipModuleGetFunction(&h->fn_group, h->mod, "ctpwa_eval_group"));
+        HIPCHECK(hipModuleGetFunction(&h->fn_group_p, h->mod, "ctpwa_eval_group_persist"));
+
         h->nacc = M.nacc();
         const bool use_gram = fixed_gram_applies(h);
         setup_partition(h, !use_gram);
@@ -930,11 +942,6 @@ extern "C" int ctpwa_create(const char* plan_text, const double* phsp, long long
             h->wave_blk = h->upload(wblk);
         }
 
-        h->src = generate_eval_kernel(M);
-        h->mod = compile_eval(device, h->src);
-        HIPCHECK(hipModuleGetFunction(&h->fn_eval, h->mod, "ctpwa_eval"));
-        HIPCHECK(hipModuleGetFunction(&h->fn_group, h->mod, "ctpwa_eval_group"));
-        HIPCHECK(hipModuleGetFunction(&h->fn_group_p, h->mod, "ctpwa_eval_group_persist"));
         if (!M.customs.empty()) {
             HIPCHECK(hipModuleGetFunction(&h->fn_aux, h->mod, "ctpwa_aux"));
             HIPCHECK(hipModuleGetFunction(&h->fn_custom, h->mod, "ctpwa_custom"));

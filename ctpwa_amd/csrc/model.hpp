@@ -345,13 +345,17 @@ inline std::string den_key(const Model_& M, int d) {
 // Wave groups of the fused kernel and the equal propagators within each.
 //
 // One thread that carries every accumulator of an event needs about 2 x (2 namp) vector
-// registers for them; past some 24 amplitudes they no longer fit and go to scratch (149
-// amplitudes, FP64: 6.27 ms per evaluation of 1.5M events, 0.25 TB/s).  Such a model's
-// blocks are shared out among the waves of a workgroup, at most 8 of them with about 19
-// amplitudes each: what one wave then holds is what the kernel of a 20-amplitude model
-// holds (0.50 ms, 3.2 TB/s; two waves per SIMD, about 500 FP64 instructions per wave and
-// iteration).  6 groups of 25 amplitudes spill (1.14 ms), and so do 10 of 15, whose ten
-// waves leave each only 168 registers (1.37 ms).
+// registers for them; past some 24 amplitudes it takes more than the 256 of two waves per
+// SIMD, past some 30 they no longer fit at all and go to scratch (149 amplitudes, FP64: 6.27
+// ms per evaluation of 1.5M events, 0.25 TB/s).  Such a model's blocks are shared out among
+// the waves of a workgroup, up to 8 of them with up to 19 amplitudes each, which is what the
+// kernel of a 20-amplitude model holds (149 amplitudes: 0.50 ms, 3.2 TB/s; two waves per SIMD,
+// about 500 FP64 instructions per wave and iteration).  There 6 groups of 25 amplitudes spill
+// more (1.14 ms), and so do 10 of 15, whose ten waves leave each only 168 registers (1.37 ms).
+// Above 152 amplitudes the eight groups grow and spill more again (197 amplitudes, 360k events:
+// 0.33 ms, as one wave 2.4 ms).  1.4M events, FP64, as one wave and in groups: 26 amplitudes
+// 101 and 94 us, 32 amplitudes 114 and 99, 40 amplitudes 141 and 125, 57 amplitudes 1004
+// and 228.
 // Blocks stay in plan order, so that a group's SL tensors, amplitudes and accumulators are
 // contiguous; the cuts minimise the largest group's cost in FP64 instructions.
 inline void assign_groups(Model_& M) {
