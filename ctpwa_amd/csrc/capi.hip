@@ -497,6 +497,15 @@ static Partition partition(const ctpwa_handle* h, bool scan_phsp, long long targ
     return R;
 }
 
+// scratch of ctpwa_nll_grad_noalloc in doubles, and what its contract (include/ctpwa_amd.h)
+// counts for a handle: accumulators of every propagator, workgroups of 256 events.  What it
+// accepts is a matter of the model and the event counts, not of the kernel's split.
+static const size_t NOALLOC_DOUBLES = (size_t)1 << 18;
+static size_t noalloc_contract(const ctpwa_handle* h) {
+    const size_t nacc = 1 + 2 * (size_t)h->M.P.namp + (size_t)h->M.nth_all + h->M.cterms.size();
+    return nacc * (size_t)std::max(1, h->noalloc_nwg) + 3 * nacc;
+}
+
 // The fused kernel's workgroups.  One wave per event (groups == 1): about 1024 (four
 // 128-thread workgroups per CU), at least 256 events each.  Wave groups: as many as the chip
 // holds at once by the compiled kernel's registers and LDS, at least 128 events each.  Two
@@ -529,15 +538,15 @@ static void setup_partition(ctpwa_handle* h, bool scan_phsp) {
         HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
         HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, h->fn_eval, M.wgs, 0));
         const int fit = ncu * std::max(1, per_cu);
-        const long long t = std::min<long long>(std::max(4, std::min(fit, 1024)), std::max<long long>(1, (nev + 127) / 128));
+        long long t = std::min<long long>(std::max(4, std::min(fit, 1024)), std::max<long long>(1, (nev + 127) / 128));
+        h->noalloc_nwg = (int)partition(h, scan_phsp, t1, 128, wcost, false).cls.size();
+        // (some hundred amplitudes: a handle within the contract has to fit into the scratch)
+        if (noalloc_contract(h) <= NOALLOC_DOUBLES) t = std::min<long long>(t, (long long)NOALLOC_DOUBLES / h->nacc - 3);
         // (a class too small for a workgroup of its own still gets one)
         for (long long k = t;; --k) {
             R = partition(h, scan_phsp, k, M.ev_step(), wcost, true);
             if ((long long)R.cls.size() <= t || k <= 1) break;
         }
-        // what ctpwa_nll_grad_noalloc accepts is a matter of the model and the event counts
-        // (include/ctpwa_amd.h), not of this kernel's split
-        h->noalloc_nwg = (int)partition(h, scan_phsp, t1, 128, wcost, false).cls.size();
     } else {
         R = partition(h, scan_phsp, t1, M.ev_step(), wcost, false);
         h->noalloc_nwg = (int)R.cls.size();
@@ -565,7 +574,6 @@ static bool constant_weights(const double* w, long long n, double* c) {
 // Every evaluation overwrites what it reads (each workgroup writes its partial row, the
 // reduction writes the totals), so nothing needs clearing between calls; calls that
 // overlap on one GPU share the array and race.
-static const size_t NOALLOC_DOUBLES = (size_t)1 << 18;
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 static std::mutex g_scratch_mu;
 static std::map<int, double*> g_scratch;
@@ -1028,8 +1036,7 @@ extern "C" int ctpwa_nll_grad(ctpwa_handle* h, const double* params_dev, double*
 
 extern "C" int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev, double* out_dev, void* stream) {
     if (!h || !params_dev || !out_dev) return fail("ctpwa_nll_grad_noalloc: NULL argument");
-    const size_t nacc = 1 + 2 * (size_t)h->M.P.namp + (size_t)h->M.nth_all + h->M.cterms.size();
-    const size_t need = nacc * (size_t)std::max({1, h->nwg, h->noalloc_nwg}) + 3 * nacc;
+    const size_t need = std::max(noalloc_contract(h), (size_t)h->nacc * (size_t)std::max(1, h->nwg) + 3 * (size_t)h->nacc);
     if (need > NOALLOC_DOUBLES)
         return fail("ctpwa_nll_grad_noalloc: the evaluation needs " + std::to_string(need) +
                     " doubles of scratch, more than the " + std::to_string(NOALLOC_DOUBLES) + " it holds");
