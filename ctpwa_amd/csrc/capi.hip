@@ -1070,13 +1070,15 @@ static int hess_nz(const Model_& M) {
     }
     return nz;
 }
-// bytes of Jacobian rows per pass (environment CTPWA_HESS_JBYTES overrides it for measurements)
-static long long hess_jbytes() {
+// bytes of rows per pass: 2 GiB of Jacobian rows, 256 MiB of the amplitude Gram's, which a
+// handle keeps besides (environment CTPWA_HESS_JBYTES overrides it for measurements)
+static long long hess_jbytes(bool amps_only) {
+    const long long most = amps_only ? 256LL << 20 : 2LL << 30;
     if (const char* e = std::getenv("CTPWA_HESS_JBYTES")) {
         long long v = std::atoll(e);
-        if (v >= (1LL << 20)) return v;
+        if (v >= (1LL << 20)) return amps_only ? std::min(v, most) : v;
     }
-    return 2LL << 30;
+    return most;
 }
 static long long up(long long x, long long m) { return (x + m - 1) / m * m; }
 // Sizes of a GramWS for the classes' event counts: events of one class per pass (chunk, a
@@ -1116,7 +1118,7 @@ static long long gram_plan(int ncol, bool f32, int ncu, std::vector<GramPair>* p
 static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long n3[3], int ncu) {
     GramSizes z{};
     const long long row = (long long)M.P.npol * 2 * S.C * 8;
-    z.chunk = std::max<long long>(256, hess_jbytes() / row / 256 * 256);
+    z.chunk = std::max<long long>(256, hess_jbytes(S.NU == 0) / row / 256 * 256);
     const long long all = n3[0] + n3[1] + n3[2];
     z.cap = std::max<long long>(1, std::min(all, z.chunk));
     // (split rows: one-wave workgroups, as many times over as there are sets; 2 or 8 per CU and
