@@ -106,6 +106,11 @@ static int hess_nz(const Model_& M) {
     return nz;
 }
 
+// a block's code in FP64 instructions, about (nl: its free parameters)
+static double block_cost(const Model_& M, int b, int nl) {
+    return 40.0 + 30.0 * nl + 15.0 * nl * (nl + 1) + M.P.blocks[b].nsl * (30.0 + 35.0 * nl + 6.0 * nl * (nl + 1));
+}
+
 // shape of the generated kernel: wave groups, their blocks, LDS layout
 HessShape hess_shape(const Model_& M, bool amps_only) {
     const Plan& P = M.P;
@@ -139,10 +144,7 @@ HessShape hess_shape(const Model_& M, bool amps_only) {
         // cuts: the largest group's cost (FP64 instructions) as small as possible; between
         // different parameter sets where there are enough of them
         std::vector<double> cost(n + 1, 0.0);
-        for (int k = 0; k < n; ++k) {
-            const double nl = (double)pars(bl[k]).size();
-            cost[k + 1] = cost[k] + 40.0 + 30.0 * nl + 15.0 * nl * (nl + 1) + P.blocks[bl[k]].nsl * (30.0 + 35.0 * nl + 6.0 * nl * (nl + 1));
-        }
+        for (int k = 0; k < n; ++k) cost[k + 1] = cost[k] + block_cost(M, bl[k], (int)pars(bl[k]).size());
         std::vector<std::vector<double>> best;
         std::vector<std::vector<int>> cut;
         auto solve = [&](bool at_sets) {
@@ -264,6 +266,9 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
         "    long long ldc, double* __restrict__ gpart, double* __restrict__ upart, double* __restrict__ zpart, int nwg,\n"
         "    const double* __restrict__ cfr, long long cld, int withK";
     const std::string CALL = "tab, slv, inv, invf, ld, wts, w1, w2, pw1, pw2, H, J, ldJ, U, W, D, ldc, gpart, upart, zpart, nwg, cfr, cld, withK";
+    bool branch_u = NA <= 12;
+    for (size_t b = 0; b < P.blocks.size(); ++b)
+        if (P.blocks[b].nsl > 0 && block_cost(M, (int)b, (int)M.bvars[b].size()) > 1000.0) branch_u = false;
     std::vector<int> order_cols;
     std::ostringstream bodies;
     // the generated functions: the groups, and in the split form the sets, the parameter
@@ -481,7 +486,7 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
             };
             auto ustore = [&](const std::string& v, int x, const char* ind) {
                 put(v, col_u0 + x, ind);
-                if (!fused) o << ind << (kind == GROUP && NA <= 12 ? "if (cls != 0) " : "") << "at(Uk + " << x << "LL * lu, wo) = " << v << ";\n";
+                if (!fused) o << ind << (kind == GROUP && branch_u ? "if (cls != 0) " : "") << "at(Uk + " << x << "LL * lu, wo) = " << v << ";\n";
             };
             // a parameter's finished derivative columns
             auto theta_cols = [&](int j) {
@@ -807,11 +812,14 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
         if (!fused) {
             // rows: uniform column addresses plus a 32-bit lane offset.  The column strides pass
             // through empty asm statements (phase_vars), or hundreds of column addresses are
-            // formed before the loop and kept in spilled registers.  Phase space has no u.  In
-            // the sets its stores go to one column that nothing reads: a branch around each
-            // store would cut the block's code into pieces that the compiler schedules and
-            // allocates badly (2.5 KB of scratch per lane).  Groups of a smaller model take the
-            // branch (305k events of the 10-amplitude model, mixed: 132 us, without 141 us).
+            // formed before the loop and kept in spilled registers.  Phase space has no u.  Its
+            // stores go to one column that nothing reads: a branch around each store cuts a
+            // block's code into pieces that the compiler schedules and allocates badly (2.5 KB
+            // of scratch per lane in the sets; 600k events, mixed: 12 amplitudes in blocks of
+            // 1600 instructions 477 us, without branches 265; 8 in blocks of up to 1400, 299
+            // and 206).  Only where every block is small is the branch the better one: 10
+            // amplitudes in blocks of 330 instructions 208 and 231 us, 8 in blocks of up to 460
+            // 136 and 154, 6 in blocks of up to 730 116 and 121; 13 in blocks of 330 the same.
             bodies << "  long long lj = ldJ, lc = ldc, lu = ldc;\n  (void)lj; (void)lc; (void)lu;\n";
             for (int p = 0; p < NP; ++p) bodies << "  " << JT << "* __restrict__ J" << p << " = J + H.row0[k] + " << p << " * cnt;\n";
             if (!amps_only) bodies << "  double *__restrict__ Uk = U + H.w0[k], *__restrict__ Wk = W + H.w0[k], *__restrict__ Dk = D + H.w0[k];\n";
