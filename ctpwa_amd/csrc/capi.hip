@@ -1082,8 +1082,8 @@ static long long hess_jbytes(bool amps_only) {
 }
 static long long up(long long x, long long m) { return (x + m - 1) / m * m; }
 // Sizes of a GramWS for the classes' event counts: events of one class per pass (chunk, a
-// multiple of 256), events of all classes per pass (cap), workgroups (four waves' registers
-// and the LDS of a CU shared out among the CU's workgroups), and the buffers in doubles
+// multiple of 256), events of all classes per pass (cap), workgroups (occ: of the compiled
+// kernel on a CU, 0 for an estimate), and the buffers in doubles
 struct GramSizes {
     long long chunk, cap, ldJ, ldc, J, U, W, D, z, part;     // ldJ, ldc: rows of J and of U, W, D
     int target, nz;
@@ -1115,7 +1115,7 @@ static long long gram_plan(int ncol, bool f32, int ncu, std::vector<GramPair>* p
     if (pairs) *pairs = pp;
     return off * 256;
 }
-static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long n3[3], int ncu) {
+static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long n3[3], int ncu, int occ) {
     GramSizes z{};
     const long long row = (long long)M.P.npol * 2 * S.C * 8;
     z.chunk = std::max<long long>(256, hess_jbytes(S.NU == 0) / row / 256 * 256);
@@ -1123,7 +1123,13 @@ static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long
     z.cap = std::max<long long>(1, std::min(all, z.chunk));
     // (split rows: one-wave workgroups, as many times over as there are sets; 2 or 8 per CU and
     // set are 2 % slower)
-    const int per_cu = S.split ? 4 : std::max(1, (int)std::min<long long>(8 / S.G, 160 * 1024 / std::max<long long>(1, S.lds * 8)));
+    // (rows: what the compiled kernel's registers and LDS allow, or for an estimate the LDS and 32
+    // waves.  With no more than two waves per SIMD, 3M events, mixed: 7 amplitudes, six workgroups
+    // of two waves, 627 us, now 570; 13 amplitudes, three of four, 1092 and 1018.  Fused: two
+    // waves per SIMD; 49 to 64 columns take 512 registers and run one wave at a time, in two
+    // rounds of half the events, which is no slower than one round)
+    const int fit = (int)std::min<long long>((S.fused ? 8 : 32) / S.G, 160 * 1024 / std::max<long long>(1, S.lds * 8));
+    const int per_cu = S.split ? 4 : std::max(1, occ > 0 && !S.fused ? occ : fit);
     // never more than fit on the chip at once (four workgroups over, for classes smaller than
     // a share, ran as a second round: the mixed form's Gram of 3.05M events 611 us, not 310);
     // at least one for each of up to four pieces
@@ -1158,7 +1164,7 @@ static long long hess_workspace_bytes(const Model_& M0, const long long n3[3], l
         Model_ M = M0;
         M.mixed = mixed;
         const HessShape S = hess_shape(M, false);
-        const GramSizes z = gram_sizes(M, S, n3, 256);
+        const GramSizes z = gram_sizes(M, S, n3, 256, 0);
         const long long nG = (long long)(2 * S.C) * (2 * S.C + 1) / 2, nUu = (long long)S.NU * (S.NU + 1) / 2;
         long long w = 3 * (nG + nUu + z.nz) + (S.f32 ? z.J / 2 : z.J) + z.U + z.W + z.D + z.z + z.part;
         w += (long long)M.P.ntheta * M.P.ntheta * 4 + (long long)M.P.namp * M.P.ntheta;      // index tables
@@ -1172,7 +1178,7 @@ static long long hess_workspace_bytes(const Model_& M0, const long long n3[3], l
 static long long agram_workspace_bytes(const Model_& M, long long n) {
     const long long n3[3] = {n, 0, 0};
     const HessShape S = hess_shape(M, true);
-    const GramSizes z = gram_sizes(M, S, n3, 256);
+    const GramSizes z = gram_sizes(M, S, n3, 256, 0);
     return (z.J + z.U + z.W + z.D + z.z + z.part + (long long)M.P.namp * (2 * M.P.namp + 1)) * 8;
 }
 
@@ -1198,7 +1204,6 @@ static void gram_setup(ctpwa_handle* h, GramTabs& g, int ncol, bool f32, int nwg
 static void gramws_setup(ctpwa_handle* h, GramWS& w, bool amps_only, const long long n3[3]) {
     const Model_& M = h->M;
     w.S = hess_shape(M, amps_only);
-    const GramSizes z = gram_sizes(M, w.S, n3, device_cus(h->device));
     std::vector<int> perm;
     w.mod = compile_eval(h->device, generate_hess_kernel(M, &perm, amps_only));
     HIPCHECK(hipModuleGetFunction(&w.fn, w.mod, amps_only ? "ctpwa_amp_gram" : w.S.fused ? "ctpwa_hess_fused" : "ctpwa_hess_rows"));
@@ -1206,6 +1211,9 @@ static void gramws_setup(ctpwa_handle* h, GramWS& w, bool amps_only, const long 
         HIPCHECK(hipModuleGetFunction(&w.fn_sum, w.mod, "ctpwa_hess_sum"));
         HIPCHECK(hipModuleGetFunction(&w.fn_theta, w.mod, "ctpwa_hess_theta"));
     }
+    int occ = 0;
+    HIPCHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&occ, w.fn, w.S.split ? 64 : 64 * w.S.G, 0));
+    const GramSizes z = gram_sizes(M, w.S, n3, device_cus(h->device), occ);
     if ((int)perm.size() != z.nz) throw std::runtime_error("Hessian: summed-column count mismatch");
     w.perm = h->upload(perm);
     w.nz = z.nz;
