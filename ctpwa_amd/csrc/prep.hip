@@ -585,34 +585,31 @@ __device__ __forceinline__ double2 block_psi(const AuxArgs& a, int b, long long 
     return make_double2(pr, pi);
 }
 
-// NP > 0: the model's polarisation count, known at compile time (registers, unrolled);
-// 0: any count
+// polarisation arrays of a compile-time length stay in registers, their loops unrolled
 template <int NP> struct PolArr { double r[NP], i[NP]; };
-template <> struct PolArr<0> { double r[MAXPOL], i[MAXPOL]; };
 
-// w += P_b(e, p0 + p) of NP polarisations (those below npol), or of all npol (NP = 0, p0 = 0)
+// w += P_b(e, p0 + p) of NP polarisations (those below npol)
 template <int NP>
 __device__ __forceinline__ void add_block(const AuxArgs& a, int b, long long e, int p0, int npol, PolArr<NP>& w) {
-    const int np = NP ? NP : npol;
     const int nsl = uni(&a.blocks[b].nsl), site = uni(&a.blocks[b].site);
     if (nsl <= 0) return;
     const double2 psi = block_psi(a, b, e);
     PolArr<NP> y;
-#pragma unroll NP ? NP : 1
-    for (int p = 0; p < np; ++p) { y.r[p] = 0.0; y.i[p] = 0.0; }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) { y.r[p] = 0.0; y.i[p] = 0.0; }
     for (int am = site; am < site + nsl; ++am) {
         const double cr = uni(a.table + a.off_c + 2 * am), ci = uni(a.table + a.off_c + 2 * am + 1);
         const int u = uni(&a.amps[am].u);
-#pragma unroll NP ? NP : 1
-        for (int p = 0; p < np; ++p) {
-            if (NP && p0 + p >= npol) continue;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            if (p0 + p >= npol) continue;
             const double2 s = post_sl(a.st, u, p0 + p, npol, e);
             y.r[p] += cr * s.x - ci * s.y;
             y.i[p] += cr * s.y + ci * s.x;
         }
     }
-#pragma unroll NP ? NP : 1
-    for (int p = 0; p < np; ++p) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
         w.r[p] += psi.x * y.r[p] - psi.y * y.i[p];
         w.i[p] += psi.x * y.i[p] + psi.y * y.r[p];
     }
@@ -648,68 +645,77 @@ __global__ void __launch_bounds__(128) k_amplitudes(AuxArgs a, long long e0, lon
 // P_b = Psi_b sum_{a in b} c_a sl_u(a),p and c_a = v_a K_a (src/ComputeResults.cu:57-190)
 // partial wave w = blocks wblk[wptr[w] .. wptr[w+1]) (a block and its identical-particle
 // permuted copies): out[w][i] = sum_pol |sum over the wave's blocks P_b|^2,
-// out[nwave][i] = the total intensity
-template <int NP>
+// out[nwave][i] = the total intensity.
+// MORE: more than NP polarisations, NP at a time, each sum carried on in out (in the order of
+// one pass over all).  Arrays of any length instead, indexed by a loop variable, lie in
+// scratch: six polarisations, 500k events, 10 amplitudes, 926 us, now 125.
+template <int NP, bool MORE>
 __global__ void __launch_bounds__(64) k_partial_int(AuxArgs a, const int* __restrict__ wptr, const int* __restrict__ wblk, int nwave,
                                                      long long e0, long long n, double* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const long long e = e0 + i;
-    const int npol = NP ? NP : a.npol;
-    PolArr<NP> S, W;
-#pragma unroll NP ? NP : 1
-    for (int p = 0; p < npol; ++p) { S.r[p] = 0.0; S.i[p] = 0.0; }
-    for (int w = 0; w < nwave; ++w) {
-#pragma unroll NP ? NP : 1
-        for (int p = 0; p < npol; ++p) { W.r[p] = 0.0; W.i[p] = 0.0; }
-        for (int k = uni(wptr + w); k < uni(wptr + w + 1); ++k) add_block<NP>(a, uni(wblk + k), e, 0, npol, W);
-        double v = 0.0;
-#pragma unroll NP ? NP : 1
-        for (int p = 0; p < npol; ++p) {
-            v += W.r[p] * W.r[p] + W.i[p] * W.i[p];
-            S.r[p] += W.r[p];
-            S.i[p] += W.i[p];
-        }
-        out[(long long)w * n + i] = v;
-    }
+    const int npol = MORE ? a.npol : NP;
     double I = 0.0;
-#pragma unroll NP ? NP : 1
-    for (int p = 0; p < npol; ++p) I += S.r[p] * S.r[p] + S.i[p] * S.i[p];
+    for (int p0 = 0; p0 < npol; p0 += NP) {
+        PolArr<NP> S, W;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) { S.r[p] = 0.0; S.i[p] = 0.0; }
+        for (int w = 0; w < nwave; ++w) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p) { W.r[p] = 0.0; W.i[p] = 0.0; }
+            for (int k = uni(wptr + w); k < uni(wptr + w + 1); ++k) add_block<NP>(a, uni(wblk + k), e, p0, npol, W);
+            double v = MORE && p0 ? out[(long long)w * n + i] : 0.0;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                v += W.r[p] * W.r[p] + W.i[p] * W.i[p];
+                S.r[p] += W.r[p];
+                S.i[p] += W.i[p];
+            }
+            out[(long long)w * n + i] = v;
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) I += S.r[p] * S.r[p] + S.i[p] * S.i[p];
+    }
     out[(long long)nwave * n + i] = I;
 }
 
 // coherent partial-wave amplitudes: out[w][i][p] = sum over the wave's blocks of P_b
 // (couplings applied), interleaved complex, events [e0, e0 + n)
-template <int NP>
+template <int NP, bool MORE>
 __global__ void __launch_bounds__(64) k_partial_amp(AuxArgs a, const int* __restrict__ wptr, const int* __restrict__ wblk, int nwave,
                                                      long long e0, long long n, double2* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const long long e = e0 + i;
-    for (int p0 = 0; p0 < a.npol; p0 += NP)
-        for (int w = 0; w < nwave; ++w) {
+    const int npol = MORE ? a.npol : NP;
+    for (int w = 0; w < nwave; ++w)
+        // (one wave's groups one after the other: they fill the same lines of out)
+        for (int p0 = 0; p0 < npol; p0 += NP) {
             PolArr<NP> W;
 #pragma unroll
             for (int p = 0; p < NP; ++p) { W.r[p] = 0.0; W.i[p] = 0.0; }
-            for (int k = uni(wptr + w); k < uni(wptr + w + 1); ++k) add_block<NP>(a, uni(wblk + k), e, p0, a.npol, W);
+            for (int k = uni(wptr + w); k < uni(wptr + w + 1); ++k) add_block<NP>(a, uni(wblk + k), e, p0, npol, W);
 #pragma unroll
             for (int p = 0; p < NP; ++p)
-                if (p0 + p < a.npol) out[((long long)w * n + i) * a.npol + p0 + p] = make_double2(W.r[p], W.i[p]);
+                if (p0 + p < npol) out[((long long)w * n + i) * npol + p0 + p] = make_double2(W.r[p], W.i[p]);
         }
 }
 
-template <int NP>
+template <int NP, bool MORE>
 __global__ void __launch_bounds__(64) k_intensity(AuxArgs a, int nblock, long long e0, long long n, double* __restrict__ out) {
     long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int npol = NP ? NP : a.npol;
-    PolArr<NP> S;
-#pragma unroll NP ? NP : 1
-    for (int p = 0; p < npol; ++p) { S.r[p] = 0.0; S.i[p] = 0.0; }
-    for (int b = 0; b < nblock; ++b) add_block<NP>(a, b, e0 + i, 0, npol, S);
+    const int npol = MORE ? a.npol : NP;
     double I = 0.0;
-#pragma unroll NP ? NP : 1
-    for (int p = 0; p < npol; ++p) I += S.r[p] * S.r[p] + S.i[p] * S.i[p];
+    for (int p0 = 0; p0 < npol; p0 += NP) {
+        PolArr<NP> S;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) { S.r[p] = 0.0; S.i[p] = 0.0; }
+        for (int b = 0; b < nblock; ++b) add_block<NP>(a, b, e0 + i, p0, npol, S);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) I += S.r[p] * S.r[p] + S.i[p] * S.i[p];
+    }
     out[i] = I;
 }
 
@@ -765,17 +771,16 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_finaliz
     return hipGetLastError();
 }
 
-// the polarisation count at compile time up to four; more: any count at once (MORE = 0), or in
-// groups of MORE
-#define POST_LAUNCH(K, MORE, npol, n, ...)                                                               \
+// the polarisation count at compile time up to four; more: four at a time
+#define POST_LAUNCH(K, npol, n, ...)                                                                     \
     do {                                                                                                 \
         const dim3 g_((unsigned)((n + 63) / 64)), b_(64);                                                \
         switch (npol) {                                                                                  \
-        case 1: hipLaunchKernelGGL(ctpwa::K<1>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
-        case 2: hipLaunchKernelGGL(ctpwa::K<2>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
-        case 3: hipLaunchKernelGGL(ctpwa::K<3>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
-        case 4: hipLaunchKernelGGL(ctpwa::K<4>, g_, b_, 0, stream, __VA_ARGS__); break;                  \
-        default: hipLaunchKernelGGL(ctpwa::K<MORE>, g_, b_, 0, stream, __VA_ARGS__);                     \
+        case 1: hipLaunchKernelGGL((ctpwa::K<1, false>), g_, b_, 0, stream, __VA_ARGS__); break;         \
+        case 2: hipLaunchKernelGGL((ctpwa::K<2, false>), g_, b_, 0, stream, __VA_ARGS__); break;         \
+        case 3: hipLaunchKernelGGL((ctpwa::K<3, false>), g_, b_, 0, stream, __VA_ARGS__); break;         \
+        case 4: hipLaunchKernelGGL((ctpwa::K<4, false>), g_, b_, 0, stream, __VA_ARGS__); break;         \
+        default: hipLaunchKernelGGL((ctpwa::K<4, true>), g_, b_, 0, stream, __VA_ARGS__);                \
         }                                                                                                \
     } while (0)
 
@@ -784,7 +789,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_partial
                                                                                      long long e0, long long n, double* out,
                                                                                      hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    POST_LAUNCH(k_partial_int, 0, a->npol, n, *a, wptr, wblk, nwave, e0, n, out);
+    POST_LAUNCH(k_partial_int, a->npol, n, *a, wptr, wblk, nwave, e0, n, out);
     return hipGetLastError();
 }
 
@@ -793,7 +798,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_partial
                                                                                      long long e0, long long n, double* out,
                                                                                      hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    POST_LAUNCH(k_partial_amp, 4, a->npol, n, *a, wptr, wblk, nwave, e0, n, (double2*)out);
+    POST_LAUNCH(k_partial_amp, a->npol, n, *a, wptr, wblk, nwave, e0, n, (double2*)out);
     return hipGetLastError();
 }
 
@@ -801,7 +806,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t ctpwa_launch_aux(con
                                                                              long long n, double* out, int intensity,
                                                                              hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    if (intensity) POST_LAUNCH(k_intensity, 0, a->npol, n, *a, nblock, e0, n, out);
+    if (intensity) POST_LAUNCH(k_intensity, a->npol, n, *a, nblock, e0, n, out);
     else hipLaunchKernelGGL(ctpwa::k_amplitudes, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, stream, *a, e0, n, out);
     return hipGetLastError();
 }
