@@ -1118,7 +1118,8 @@ static long long gram_plan(int ncol, bool f32, int ncu, std::vector<GramPair>* p
 static GramSizes gram_sizes(const Model_& M, const HessShape& S, const long long n3[3], int ncu, int occ) {
     GramSizes z{};
     const long long row = (long long)M.P.npol * 2 * S.C * 8;
-    z.chunk = std::max<long long>(256, hess_jbytes(S.NU == 0) / row / 256 * 256);
+    // (a row's byte offset in its column is a 32-bit number in the generated kernel)
+    z.chunk = std::max<long long>(256, std::min<long long>(1 << 28, hess_jbytes(S.NU == 0) / row / 256 * 256));
     const long long all = n3[0] + n3[1] + n3[2];
     z.cap = std::max<long long>(1, std::min(all, z.chunk));
     // (split rows: one-wave workgroups, as many times over as there are sets; 2 or 8 per CU and
