@@ -1961,14 +1961,16 @@ extern "C" long long ctpwa_generate_source(const char* plan_text, int precision,
     }
 }
 
-// source of the generated Hessian rows kernel for a plan, without a device
+// source of the generated Hessian kernel for a plan, without a device
 extern "C" long long ctpwa_generate_hessian_source(const char* plan_text, int precision, char* buf, long long cap) {
     try {
         if (precision != 0 && precision != 1) throw std::runtime_error("precision must be 0 (FP64) or 1 (mixed)");
         Model_ M = derive(parse_plan(plan_text));
         M.mixed = precision;
         std::string src = generate_hess_kernel(M, nullptr, false);
-        // models with Custom lineshapes: the second-order factor module follows
+        // the amplitude Gram's module follows, and for models with Custom lineshapes the
+        // second-order factors'
+        src += "\n// ---- module: ctpwa_amp_gram ----\n" + generate_hess_kernel(M, nullptr, true);
         if (!M.customs.empty()) src += "\n// ---- module: ctpwa_custom2 ----\n" + generate_custom2_kernel(M);
         if (buf && cap > 0) {
             long long n = std::min<long long>(cap - 1, (long long)src.size());
@@ -1982,8 +1984,8 @@ extern "C" long long ctpwa_generate_hessian_source(const char* plan_text, int pr
     }
 }
 
-// compile the fused kernel for a plan with hipRTC (no device needed); returns the
-// code-object size in bytes, or -1 with the compiler log in ctpwa_last_error()
+// compile a plan's generated kernels with hipRTC (no device needed); returns the
+// code objects' size in bytes, or -1 with the compiler log in ctpwa_last_error()
 extern "C" long long ctpwa_compile_check(const char* plan_text, int precision) {
     try {
         if (precision != 0 && precision != 1) throw std::runtime_error("precision must be 0 (FP64) or 1 (mixed)");
@@ -2007,6 +2009,7 @@ extern "C" long long ctpwa_compile_check(const char* plan_text, int precision) {
         };
         long long cs = compile(generate_eval_kernel(M));
         cs += compile(generate_hess_kernel(M, nullptr, false));
+        cs += compile(generate_hess_kernel(M, nullptr, true));
         // models with Custom lineshapes: also the Hessian's second-order factor module
         if (!M.customs.empty()) cs += compile(generate_custom2_kernel(M));
         return cs;

@@ -176,16 +176,16 @@ const char* ctpwa_kernel_source(const ctpwa_handle* h);
  * (NUL-terminated) into buf and returns the full size including the NUL, -1 on error */
 long long ctpwa_generate_source(const char* plan_text, int precision, char* buf, long long cap);
 
-/* source of the generated Hessian rows kernel for a plan (the per-event part of
+/* source of the generated Hessian kernel for a plan (the per-event part of
  * analysis::getHessian, src/Analysis.cu:2689-3378), without a device; as
- * ctpwa_generate_source.  For a model with Custom lineshapes the source of the
- * second-order factor module (ctpwa_custom2) follows a line
- * "// ---- module: ctpwa_custom2 ----" */
+ * ctpwa_generate_source.  The source of the amplitude Gram's module follows a line
+ * "// ---- module: ctpwa_amp_gram ----", and for a model with Custom lineshapes that of the
+ * second-order factor module (ctpwa_custom2) a line "// ---- module: ctpwa_custom2 ----" */
 long long ctpwa_generate_hessian_source(const char* plan_text, int precision, char* buf, long long cap);
 
-/* compile the fused kernel and the Hessian rows kernel for a plan with hipRTC (no device
- * needed), and for a plan with Custom lineshapes also the Hessian's second-order factor
- * kernel; returns the total code-object size, or -1 with the compiler log in
+/* compile the fused kernel, the Hessian's and the amplitude Gram's for a plan with hipRTC (no
+ * device needed), and for a plan with Custom lineshapes also the Hessian's second-order
+ * factor kernel; returns the total code-object size, or -1 with the compiler log in
  * ctpwa_last_error() */
 long long ctpwa_compile_check(const char* plan_text, int precision);
 
