@@ -1060,16 +1060,6 @@ extern "C" int ctpwa_nll_grad_noalloc(ctpwa_handle* h, const double* params_dev,
 }
 
 
-// second-part sums (and the sum of alpha I) of a model's Hessian
-static int hess_nz(const Model_& M) {
-    int nz = 1;
-    for (size_t b = 0; b < M.P.blocks.size(); ++b) {
-        if (M.P.blocks[b].nsl == 0) continue;
-        const int nl = (int)M.bvars[b].size();
-        nz += M.P.blocks[b].nsl * 2 * nl + nl * (nl + 1) / 2;
-    }
-    return nz;
-}
 // bytes of rows per pass: 2 GiB of Jacobian rows, 256 MiB of the amplitude Gram's, which a
 // handle keeps besides (environment CTPWA_HESS_JBYTES overrides it for measurements)
 static long long hess_jbytes(bool amps_only) {

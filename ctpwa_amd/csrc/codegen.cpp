@@ -1054,8 +1054,8 @@ std::string generate_eval_kernel(const Model_& M) {
     // make its wait cover them as well.
     // Wave groups load ahead the invariants only: the SL values are first used after the
     // propagators and the coupling sums (some 200 FP64 instructions), and with both ahead
-    // the eight groups of the 149-amplitude model spill (282 registers; 73 without, outside
-    // the loops).
+    // the eight groups of the 149-amplitude model spill 282 registers.  Without, 72: four of
+    // the eight loops reload up to sixteen values per iteration.
     const bool pf_sl = NG == 1;
     auto decl_set = [&](const Group& G, const char* pre, const char* ev) {
         if (pf_sl) for (int u : G.us)
@@ -1284,7 +1284,7 @@ std::string generate_eval_kernel(const Model_& M) {
         const int NX = 2 * NP;
         for (int g = 0; g < NG; ++g) {
             const Group& G = groups[g];
-            o << "template <bool UL>\n__device__ __forceinline__ void eval_g" << g << "(\n" << PARAMS;
+            o << "__device__ __forceinline__ void eval_g" << g << "(\n" << PARAMS;
             emit_prologue();
             if (g == 0) o << VALUE_ACCS;
             emit_accs(G);
@@ -1348,7 +1348,7 @@ std::string generate_eval_kernel(const Model_& M) {
           << "  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));\n  switch (wave) {\n";
         for (int g = 0; g < NG; ++g)
             o << "  " << (g + 1 < NG ? "case " + std::to_string(g) : std::string("default")) << ": eval_g" << g
-              << "<UL>(tab, slv, inv, invf, wts, part, wg_cls, wg_rng, ld, nwg, w1, w2, pw1, pw2, wg, red, lbuf, cfb); break;\n";
+              << "(tab, slv, inv, invf, wts, part, wg_cls, wg_rng, ld, nwg, w1, w2, pw1, pw2, wg, red, lbuf, cfb); break;\n";
         o << "  }\n}\n";
     }
     std::string lb = "__launch_bounds__(" + std::to_string(WGS) + (M.min_waves > 0 ? ", " + std::to_string(M.min_waves) : std::string()) + ")";

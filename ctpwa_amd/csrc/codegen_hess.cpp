@@ -95,8 +95,7 @@ __device__ __forceinline__ double col_part(const double* xs, int lane) {
 }
 )";
 
-// second-part sums of the assembly (Z and the sum of alpha I)
-static int hess_nz(const Model_& M) {
+int hess_nz(const Model_& M) {
     int nz = 1;
     for (size_t b = 0; b < M.P.blocks.size(); ++b) {
         if (M.P.blocks[b].nsl == 0) continue;
@@ -508,7 +507,6 @@ std::string generate_hess_kernel(const Model_& M, std::vector<int>* perm, bool a
             for (size_t k = 0; k < blocks.size(); ++k)
                 for (int j : M.bvars[blocks[k]]) last[j] = (int)k;
             std::vector<char> open_(NT, 0);
-            std::vector<char> topen(M.us.size(), 0);
             for (size_t kb = 0; kb < blocks.size(); ++kb) {
                 const int b = blocks[kb];
                 const PBlock& B = P.blocks[b];

@@ -228,9 +228,10 @@ k_gram_panels(const T* __restrict__ X0, int ncol, long long ldx, HessPieces H, i
 // off-diagonal panel pair's (A read and weighted once per step), (i, i + q mod T) for
 // q <= T / 2 on the diagonal, so every wave of a workgroup has the same work and the shares
 // are dealt out by it.  Bound by the matrix cores (64 cycles per FP64 product); every column
-// is read 3.3 times for 346 columns.  No register may spill: a reload between the loads waits
-// for all of them (7.3 instead of 3.5 ms for 1.2M rows of 346 and
-// 100k rows of 322 columns).  Panels of 64 columns read every column 7.8 times
+// is read 3.3 times for 346 columns.  Registers should not spill: a reload between the loads
+// waits for all of them (7.3 instead of 3.5 ms for 1.2M rows of 346 and 100k rows of 322
+// columns, which meet none; of the FP64 forms an off-diagonal pair of seven tiles reloads two
+// values per slab, of the FP32 forms one of eight tiles four).  Panels of 64 columns read every column 7.8 times
 // and computed full tile squares on the diagonal (7.5 ms).
 // LDS column strides: 16 columns x 2 rows (FP64) or x 4 rows (FP32) of a read lie in different
 // banks, and 16-byte stores stay aligned.

@@ -671,5 +671,7 @@ struct HessShape {
     long long oX = 0, oT = 0, oZ = 0, lds = 0;
 };
 HessShape hess_shape(const Model_& M, bool amps_only);
+// second-part sums of a model's Hessian, and the sum of alpha I
+int hess_nz(const Model_& M);
 
 }  // namespace ctpwa

@@ -491,8 +491,11 @@ __device__ __forceinline__ void assemble_main(const FinArgs& f) {
 // counter, runs the assembly on the totals and resets the counter for the next evaluation.
 // Bound by latency: cold reads of the partials and tables, and the handover.  Sixteen waves to
 // a workgroup (one workgroup and one count per sum, each with the assembly's inputs, took
-// 37 us at 149 amplitudes, 11 us at 10; now 12 and 9); the totals go through coherent stores and loads
-// and a wait instead of agent-scope fences, which write back and invalidate the L2 cache.
+// 37 us at 149 amplitudes, 11 us at 10; now 12 and 9); the totals go through relaxed
+// agent-scope stores and loads and a wait instead of agent-scope fences, which write back and
+// invalidate the L2 cache.  That rests on this target and not on the language's memory model:
+// agent-scope stores write through to where every compute unit's agent-scope loads look, and
+// after s_waitcnt vmcnt(0) they have arrived, so they precede the wave's barrier and the count.
 __device__ __forceinline__ void finalize_body(const FinArgs& f) {
     __shared__ int last;
     const int pair = blockIdx.x * (ASM_THREADS / 64) + (threadIdx.x >> 6);

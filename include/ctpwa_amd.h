@@ -154,7 +154,8 @@ long long ctpwa_footprint_bytes(const char* plan_text, long long n_phsp, long lo
                                 int precision);
 
 /* device bytes a handle allocates on its first ctpwa_hessian call and keeps until
- * ctpwa_destroy: partial sums, and with more than 64 Jacobian columns the rows of a pass
+ * ctpwa_destroy: partial sums, and the Jacobian and u rows of a pass in the mixed form, with
+ * more than 64 Jacobian columns, or where the polarisations' columns do not fit into LDS
  * (the larger of the two storage forms' needs) */
 long long ctpwa_hessian_workspace_bytes(const char* plan_text, long long n_phsp, long long n_data, long long n_bkg);
 
